@@ -156,7 +156,7 @@ struct cgfd_session {
   double cmet[9] = {0};
   int free_top = 0;
   FaceHost face[6];
-  int slot[4] = {0, 1, 2, 3};  // physical level slot of W^n and of the stage values U1, U2, U3
+  int slot[4] = {0, 1, 2, 3};  // physical level slots of W^n, W^{n-1} and the last step's U2, U3 (see stage_plan)
   float sc[9], isc[9];
   std::vector<SrcHost> src;
   std::vector<RecvHost> rec;
@@ -601,8 +601,30 @@ template <typename TC> int build_receivers(cgfd_session *s) {
 }
 
 // ---- stage argument assembly ----
-// Level slots of a stage: input, W^n, output, U1 (written with W^{n+1} by
-// S3) and U2 (read by S3); rhs_mode sends the output to the RHS level.
+// Stage q of a step: RK mode and level slots.  slot[] holds the slots of W^n,
+// W^{n-1}, and the last step's U2 and U3; the last three are free to write.
+// With the sum Q (FP32/FP64): U1 -> slot 3, U2 -> slot 2 and Q -> slot 1, U3
+// over U1, W^{n+1} over Q.  From the stage values (16-bit storage): U1 -> slot
+// 1, U2 -> slot 2, U3 -> slot 3, W^{n+1} over U1.  Either way W^{n+1} ends in
+// slot 1, which the step's end swaps with slot 0.
+struct StagePlan {
+  int in, out, mode;
+};
+template <typename TS> StagePlan stage_plan(const int *slot, int q) {
+  if constexpr (St<TS>::scaled) {
+    const StagePlan p[4] = {{slot[0], slot[1], MODE_S0}, {slot[1], slot[2], MODE_S12},
+                            {slot[2], slot[3], MODE_S12}, {slot[3], slot[1], MODE_S3}};
+    return p[q];
+  } else {
+    const StagePlan p[4] = {{slot[0], slot[3], MODE_S0}, {slot[3], slot[2], MODE_S1Q},
+                            {slot[2], slot[3], MODE_S12}, {slot[3], slot[1], MODE_S3Q}};
+    return p[q];
+  }
+}
+
+// Level slots of a stage: input, W^n, output, the last stage's level (slot 1
+// of the session) and U2 (read by S3); rhs_mode sends the output to the RHS
+// level.
 template <typename TS, typename TC>
 StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slot_out, int slot_end, int slot_u2,
                              bool rhs_mode) {
@@ -645,8 +667,14 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
   a.w_end = w + (long)slot_end * s->level_elems;
   a.w_u2 = w + (long)slot_u2 * s->level_elems;
   a.shot_stride = rhs_mode ? 0 : s->shot_elems;
-  // S3 weights of the stage values: w_i = b_{i-1} / a_{i-1}
+  // weights of the stage values: w_i = b_{i-1} / a_{i-1}; w3 is rounded down
+  // to a value whose complement is exact where the sum Q uses both
   for (int q = 0; q < 3; q++) a.rk_w[q] = (TC)(kRkB[q] / kRkA[q]);
+  if constexpr (!St<TS>::scaled) {
+    const double p = sizeof(TC) == 8 ? 9007199254740992.0 : 16777216.0;  // 2^53, 2^24
+    a.rk_w[2] = (TC)(std::floor(p / 3.0) / p);
+    a.rk_w[3] = TC(1) - a.rk_w[2];
+  }
   for (int c = 0; c < kNC; c++) { a.sc[c] = s->sc[c]; a.isc[c] = s->isc[c]; }
   a.shot_active = s->shot_active;
   return a;
@@ -786,12 +814,11 @@ int launch_stage(cgfd_session *s, const Shell &sh, StageArgs<TS, TC> &a, int dx,
 }
 
 // Tile autotuner: per (shape, z chunk), time the interior sweeps of one full
-// step's stage sequence (S0, S12, S12, S3 with the operator directions of
+// step's stage sequence (stage_plan, with the operator directions of
 // pair 0) and keep the fastest; the stages differ in traffic (30 to 57 words
 // per cell), so tuning on one mode alone can pick a tile that loses on the
-// others.  The RK coefficients are zero, and every level the sweeps write
-// (U1, U2, U3) is rewritten by the next step before it is read, so
-// tuning between steps leaves the state intact.  Each work split (core,
+// others.  Every level the sweeps write (slots 1..3) is rewritten by the next
+// step before it is read, so tuning between steps leaves the state intact.  Each work split (core,
 // whole planes, shell) is timed with its best tile and the fastest pair is
 // kept.  Results are cached per (grid, storage, shots, flags, metric form,
 // PML layout, pinned split) for the life of the process.
@@ -839,13 +866,11 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
     remember({s->tile_shape, s->tile_zchunk, s->split});
     return CGFD_OK;
   }
-  const int PRE = s->slot[0], U1 = s->slot[1], U2 = s->slot[2], U3 = s->slot[3];
-  const int sin[4] = {PRE, U1, U2, U3}, sout[4] = {U1, U2, U3, U1};
-  const int smode[4] = {MODE_S0, MODE_S12, MODE_S12, MODE_S3};
   StageArgs<TS, TC> sa[4];
   for (int q = 0; q < 4; q++) {
-    sa[q] = stage_args<TS, TC>(s, sin[q], PRE, sout[q], U1, U2, false);
-    sa[q].mode = smode[q];
+    const StagePlan p = stage_plan<TS>(s->slot, q);
+    sa[q] = stage_args<TS, TC>(s, p.in, s->slot[0], p.out, s->slot[1], s->slot[2], false);
+    sa[q].mode = p.mode;
     sa[q].ca = TC(0);
     sa[q].cb = TC(0);
     // time every shot slot, active or not: a batched session is tuned for
@@ -968,19 +993,13 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
       if (e != hipSuccess) return fail(CGFD_E_HIP, "receiver kernel: %s", hipGetErrorString(e));
     }
     const int ipair = it % 8;
-    // stage values U1..U3; S3 writes W^{n+1} over U1, which then becomes W
-    const int PRE = s->slot[0], U1 = s->slot[1], U2 = s->slot[2], U3 = s->slot[3];
     for (int istage = 0; istage < 4; istage++) {
       const int dx = (kFlags[ipair][0] + istage) % 2;
       const int dy = (kFlags[ipair][1] + istage) % 2;
       const int dz = (kFlags[ipair][2] + istage) % 2;
-      int in, out, mode;
-      if (istage == 0) { in = PRE; out = U1; mode = MODE_S0; }
-      else if (istage == 1) { in = U1; out = U2; mode = MODE_S12; }
-      else if (istage == 2) { in = U2; out = U3; mode = MODE_S12; }
-      else { in = U3; out = U1; mode = MODE_S3; }
-      StageArgs<TS, TC> a = stage_args<TS, TC>(s, in, PRE, out, U1, U2, false);
-      a.mode = mode;
+      const StagePlan p = stage_plan<TS>(s->slot, istage);
+      StageArgs<TS, TC> a = stage_args<TS, TC>(s, p.in, s->slot[0], p.out, s->slot[1], s->slot[2], false);
+      a.mode = p.mode;
       // coef = rk_a[istage]*dt, both float in the reference (drv_rk_curv_col.cu:341-342)
       a.ca = (istage < 3) ? (TC)kRkA[istage] * dt : TC(0);
       a.cb = (TC)kRkB[istage] * dt;
@@ -1000,7 +1019,7 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
         sa.s_tab = s->s_tab; sa.s_kind = s->s_kind; sa.F = (const TC *)s->s_F; sa.M = (const TC *)s->s_M;
         sa.ntab = s->s_ntab; sa.met = (const TC *)s->met; sa.med = (const TC *)s->med;
         sa.w_out = a.w_out; sa.w_end = a.w_end; sa.shot_stride = s->shot_elems;
-        sa.mode = mode; sa.istage = istage; sa.ca = a.ca; sa.cb = a.cb;
+        sa.mode = p.mode; sa.istage = istage; sa.ca = a.ca; sa.cb = a.cb; sa.w2 = a.rk_w[1];
         sa.clock = s->clock; sa.shot_start = s->shot_start; sa.shot_active = s->shot_active;
         sa.only_shot = -1; sa.fixed_it = 0;
         for (int c = 0; c < kNC; c++) sa.isc[c] = s->isc[c];
@@ -1009,8 +1028,8 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
       }
     }
     if (s->peak && s->free_top) {
-      // W^{n+1} sits in U1's slot before the swap (drv_rk_curv_col.cu:519-527)
-      const TS *wn = (const TS *)wav_level(s, 0, U1), *wo = (const TS *)wav_level(s, 0, PRE);
+      // W^{n+1} sits in slot 1 before the swap (drv_rk_curv_col.cu:519-527)
+      const TS *wn = (const TS *)wav_level(s, 0, s->slot[1]), *wo = (const TS *)wav_level(s, 0, s->slot[0]);
       hipError_t e = launch_peak<TS, TC>(wn, wo, s->shot_elems, s->L, (TC *)s->peak, dt, s->sc, s->shot_active,
                                          s->d.nshots, s->st);
       if (e != hipSuccess) return fail(CGFD_E_HIP, "peak motion kernel: %s", hipGetErrorString(e));

@@ -15,14 +15,24 @@ constexpr int kNC = 9;    // wavefield components
 enum Cmp { VX = 0, VY, VZ, TXX, TYY, TZZ, TYZ, TXZ, TXY };
 enum Met { JAC = 0, XIX, XIY, XIZ, ETX, ETY, ETZ, ZTX, ZTY, ZTZ, NMET };
 // RK modes of a stage kernel.  The classical RK4 step is evaluated from the
-// stored stage values U1..U3 (U_{i+1} = W^n + a_i dt K_i):
-//   S0:  U1 = W + a0 dt K0                      (input W^n)
-//   S12: U2 = W + a1 dt K1, U3 = W + a2 dt K2   (input U1 / U2, W^n read at the point)
-//   S3:  W^{n+1} = W + w1 (U1 - W) + w2 (U2 - W) + w3 (U3 - W) + b3 dt K3
-//        with w_i = b_{i-1} / a_{i-1} = 1/3, 2/3, 1/3 (input U3; written over U1)
-// which equals W + dt (b0 K0 + b1 K1 + b2 K2 + b3 K3).  MODE_RHS writes the
-// right-hand side alone (the per-stage operator).
-enum Mode { MODE_RHS = 0, MODE_S0 = 1, MODE_S12 = 2, MODE_S3 = 3 };
+// stage values U1..U3 (U_{i+1} = W^n + a_i dt K_i):
+//   S0:   U1 = W + a0 dt K0                      (input W^n)
+//   S12:  U2 = W + a1 dt K1, U3 = W + a2 dt K2   (input U1 / U2, W^n read at the point)
+//   S1Q:  S12's U2, and Q = (1 - w3) W + w1 (U1 - W) + w2 (U2 - W)
+//   S3Q:  W^{n+1} = Q + w3 U3 + b3 dt K3         (input U3; written over Q)
+//   S3:   W^{n+1} = W + w1 (U1 - W) + w2 (U2 - W) + w3 (U3 - W) + b3 dt K3
+//         (input U3; written over U1)
+// with w_i = b_{i-1} / a_{i-1} = 1/3, 2/3, 1/3, which equals
+// W + dt (b0 K0 + b1 K1 + b2 K2 + b3 K3).  FP32 and FP64 storage run S0, S1Q,
+// S12, S3Q: Q carries W, U1 and U2 into the last stage in one level, 108
+// instead of 117 level words per point and step, and S3Q reads 9 words at the
+// point where S3 reads 27 (per step, before and after: 400x400x200 Cartesian
+// FP32 5.46 -> 4.96 ms, 64 shots of 100x100x60 12.3 -> 10.7 ms, 128x128x96
+// curvilinear FP64 1.51 -> 1.26 ms; error against FP64 arithmetic 1.8-2.5e-7
+// -> 2.1-2.9e-7 after 19-32 FP32 steps).  16-bit storage runs S0, S12, S12, S3, so that the
+// sum is formed in FP32 from the stored levels and never stored in 16 bits.
+// MODE_RHS writes the right-hand side alone (the per-stage operator).
+enum Mode { MODE_RHS = 0, MODE_S0 = 1, MODE_S12 = 2, MODE_S3 = 3, MODE_S1Q = 4, MODE_S3Q = 5 };
 
 // ---- storage traits ---------------------------------------------------------
 template <typename TS> struct St;
@@ -109,13 +119,24 @@ template <typename T> __device__ __forceinline__ T &at_b(T *base, unsigned byte_
   return *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte_off);
 }
 
-// ---- the S3 combination (see Mode), one evaluation order for every kernel ----
-// partial = w1 (U1 - W) + w2 (U2 - W); W^{n+1} = W + ((partial + w3 (U3 - W)) + b3 dt K3)
+// ---- the RK combinations (see Mode), one evaluation order for every kernel ----
+// S3: partial = w1 (U1 - W) + w2 (U2 - W); W^{n+1} = W + ((partial + w3 (U3 - W)) + b3 dt K3)
 template <typename TC> __device__ __forceinline__ TC rk_partial(const TC *w, TC y0, TC u1, TC u2) {
   return w[0] * (u1 - y0) + w[1] * (u2 - y0);
 }
 template <typename TC> __device__ __forceinline__ TC rk_final(TC y0, TC partial, TC w3, TC u3, TC cbh) {
   return y0 + ((partial + w3 * (u3 - y0)) + cbh);
+}
+// S1Q: Q from W, U1 and U2's increment d2 = a1 dt K1 (the increment itself:
+// U2's rounding then stays out of Q).  w[2] = w3 is the value just below 1/3
+// for which w[3] = 1 - w3 is exact: a constant field stays constant, and the
+// 6e-8 (FP32) by which w3 misses 1/3 multiplies only U3 - W.
+template <typename TC> __device__ __forceinline__ TC rk_sum(const TC *w, TC y0, TC u1, TC d2) {
+  return w[3] * y0 + (w[0] * (u1 - y0) + w[1] * d2);
+}
+// S3Q
+template <typename TC> __device__ __forceinline__ TC rk_end(const TC *w, TC q, TC u3, TC cbh) {
+  return q + (w[2] * u3 + cbh);
 }
 
 // ---- operator constants (src/forward/fd_t.cu:76-148) ----------------------
@@ -157,7 +178,7 @@ template <typename TS, typename TM> struct FaceArgs {
   long shot_stride;             // elements between shots of this face's buffer
   const TM *A, *B, *D;          // nlay+1 profile values
   // shot-0 level bases, component stride fsize: stage input, W^n, output,
-  // U1 (S3 reads it and writes W^{n+1} over it) and U2 (read by S3)
+  // the last stage's level (see StageArgs) and U2 (read by S3)
   TS *a_in, *a_pre, *a_out, *a_end, *a_u2;
 };
 
@@ -173,13 +194,14 @@ template <typename TS, typename TM> struct StageArgs {
   int met_const;   // 1: one constant per metric component, off-diagonal ones zero (Cartesian grid)
   TM cmet[9];      // xi_x..zeta_z when met_const (off-diagonal entries exactly 0)
   FaceArgs<TS, TM> f[6];
-  // shot-0 level bases: stage input, W^n, output, U1 (S3: read, then
-  // overwritten by W^{n+1}) and U2 (S3)
+  // shot-0 level bases: stage input, W^n, output, the last stage's level (S1Q
+  // writes Q, S3Q reads Q and S3 reads U1 there; both write W^{n+1} over it)
+  // and U2 (S3)
   TS *w_in, *w_pre, *w_out, *w_end, *w_u2;
   long shot_stride;
   int mode;
   TM ca, cb;      // a_i dt and b_i dt of the stage
-  TM rk_w[3];     // w1, w2, w3 of the S3 combination
+  TM rk_w[4];     // w1, w2, w3 of the last stage's combination and 1 - w3
   float sc[kNC], isc[kNC];  // storage scale (value = stored*sc) and its inverse
   int nbox;
   int box[kMaxBox][6];      // i1,i2,j1,j2,k1,k2 inclusive, physical
@@ -204,10 +226,11 @@ template <typename TS, typename TM> struct SrcArgs {
   long ntab;
   const TM *met;            // for jac
   const TM *med;            // for 1/rho
-  TS *w_out, *w_end;   // stage output (S0..S2) / W^{n+1} (S3) of each shot
+  TS *w_out, *w_end;   // stage output (S0..S2) / Q (S1Q), W^{n+1} (S3, S3Q) of each shot
   long shot_stride;
   int mode, istage;
   TM ca, cb;
+  TM w2;               // U2's weight in Q (S1Q)
   const int *clock;         // current global step
   const int *shot_start;    // per-shot start step
   const int *shot_active;

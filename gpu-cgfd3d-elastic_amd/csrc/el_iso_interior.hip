@@ -180,9 +180,10 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
   // after its load (which makes the wave wait there for every load in
   // flight, the next plane's prefetch included).
   constexpr int mode = MODE;
-  // W^n at the point: S12 and S3; U1 and U2 at the point: S3 (folded into
-  // one partial sum per component as soon as they arrive)
-  constexpr bool need_pre = mode == MODE_S12 || mode == MODE_S3, need_u = mode == MODE_S3;
+  // W^n (S3Q: Q) at the point: every stage but the first; U1 and U2 at the
+  // point: S3 (folded into one partial sum per component as soon as they
+  // arrive)
+  constexpr bool need_pre = mode != MODE_S0 && mode != MODE_RHS, need_u = mode == MODE_S3;
   // The PML form fetches the RK levels for the current plane (not one plane
   // ahead): the 18 registers it saves are what its face update needs.
   constexpr bool LATE_RK = PML;
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
   auto load_rk = [&](unsigned qb, RT *pre, RT *u1, RT *u2) {
 #pragma unroll
     for (int c = 0; c < kNC; c++) {
-      pre[c] = need_pre ? ld_rk(&at_b(a.w_pre + so + c * cs, qb)) : RT(0);
+      pre[c] = need_pre ? ld_rk(&at_b((mode == MODE_S3Q ? a.w_end : a.w_pre) + so + c * cs, qb)) : RT(0);
       if constexpr (need_u) {
         u1[c] = ld_rk(&at_b(a.w_end + so + c * cs, qb));
         u2[c] = ld_rk(&at_b(a.w_u2 + so + c * cs, qb));
@@ -372,6 +373,12 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
         if constexpr (need_pre) pre_c = LATE_RK ? cv(c, pre_r[c]) : pre_v[c];
         if constexpr (mode == MODE_S12) {
           st_w(&at_b(wout, qb), (pre_c + a.ca * h[c]) * is);
+        } else if constexpr (mode == MODE_S1Q) {
+          const TC d2 = a.ca * h[c];
+          st_w(&at_b(wout, qb), (pre_c + d2) * is);
+          st_w(&at_b(wend, qb), rk_sum(a.rk_w, pre_c, q[c][zc0], d2) * is);
+        } else if constexpr (mode == MODE_S3Q) {
+          st_w(&at_b(wend, qb), rk_end(a.rk_w, pre_c, q[c][zc0], a.cb * h[c]) * is);
         } else if constexpr (mode == MODE_S0) {
           st_w(&at_b(wout, qb), (q[c][zc0] + a.ca * h[c]) * is);
         } else if constexpr (mode == MODE_S3) {
@@ -431,12 +438,18 @@ static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, 
   if (nwg == 0) return hipSuccess;
   dim3 grid((unsigned)nwg), block(TX * TY);
   const int sel = dx * 4 + dy * 2 + dz;
-  switch (a.mode) {
-    case MODE_S0: launch_march_m<TS, TC, TX, TY, MINB, CART, PML, MODE_S0>(a, b, g, grid, block, sel, st); break;
-    case MODE_S12: launch_march_m<TS, TC, TX, TY, MINB, CART, PML, MODE_S12>(a, b, g, grid, block, sel, st); break;
-    case MODE_S3: launch_march_m<TS, TC, TX, TY, MINB, CART, PML, MODE_S3>(a, b, g, grid, block, sel, st); break;
-    default: launch_march_m<TS, TC, TX, TY, MINB, CART, PML, MODE_RHS>(a, b, g, grid, block, sel, st); break;
+#define CGFD_M(M) \
+  if (a.mode == M) launch_march_m<TS, TC, TX, TY, MINB, CART, PML, M>(a, b, g, grid, block, sel, st)
+  if constexpr (St<TS>::scaled) {
+    CGFD_M(MODE_S3);
+  } else {
+    CGFD_M(MODE_S1Q);
+    CGFD_M(MODE_S3Q);
   }
+  CGFD_M(MODE_S0);
+  CGFD_M(MODE_S12);
+  CGFD_M(MODE_RHS);
+#undef CGFD_M
   return hipGetLastError();
 }
 

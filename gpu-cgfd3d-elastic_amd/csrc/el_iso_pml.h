@@ -49,7 +49,9 @@ __device__ __forceinline__ void pml_face(const StageArgs<TS, TC> &a, int fi, int
   for (int c = 0; c < kNC; c++) {
     const unsigned qb = (c * fs + ia) * (unsigned)sizeof(TS);
     P[c] = (TC)St<TS>::ld(&at_b(F.a_in + fso, qb)) * S(c);
-    if constexpr (MODE == MODE_S12 || MODE == MODE_S3) pre_a[c] = (TC)St<TS>::ld(&at_b(F.a_pre + fso, qb)) * S(c);
+    if constexpr (MODE == MODE_S12 || MODE == MODE_S1Q || MODE == MODE_S3)
+      pre_a[c] = (TC)St<TS>::ld(&at_b(F.a_pre + fso, qb)) * S(c);
+    if constexpr (MODE == MODE_S3Q) pre_a[c] = (TC)St<TS>::ld(&at_b(F.a_end + fso, qb)) * S(c);  // Q
     if constexpr (MODE == MODE_S3) {
       u1_a[c] = (TC)St<TS>::ld(&at_b(F.a_end + fso, qb)) * S(c);
       u2_a[c] = (TC)St<TS>::ld(&at_b(F.a_u2 + fso, qb)) * S(c);
@@ -91,6 +93,12 @@ __device__ __forceinline__ void pml_face(const StageArgs<TS, TC> &a, int fi, int
       St<TS>::st(&at_b(F.a_out + fso, qb), (P[c] + a.ca * Ph[c]) * is);
     } else if constexpr (MODE == MODE_S12) {
       St<TS>::st(&at_b(F.a_out + fso, qb), (pre_a[c] + a.ca * Ph[c]) * is);
+    } else if constexpr (MODE == MODE_S1Q) {
+      const TC d2 = a.ca * Ph[c];
+      St<TS>::st(&at_b(F.a_out + fso, qb), (pre_a[c] + d2) * is);
+      St<TS>::st(&at_b(F.a_end + fso, qb), rk_sum(a.rk_w, pre_a[c], P[c], d2) * is);
+    } else if constexpr (MODE == MODE_S3Q) {
+      St<TS>::st(&at_b(F.a_end + fso, qb), rk_end(a.rk_w, pre_a[c], P[c], a.cb * Ph[c]) * is);
     } else {
       const TC part = rk_partial(a.rk_w, pre_a[c], u1_a[c], u2_a[c]);
       St<TS>::st(&at_b(F.a_end + fso, qb), rk_final(pre_a[c], part, a.rk_w[2], P[c], a.cb * Ph[c]) * is);
@@ -137,9 +145,10 @@ __device__ __forceinline__ void pml_face_march(const StageArgs<TS, TC> &a, int f
   TC P[kNC], pre[kNC], part[kNC];
 #pragma unroll
   for (int c = 0; c < kNC; c++) P[c] = (TC)St<TS>::ld(&at_b(pin, qb(c))) * S(c);
-  if constexpr (MODE == MODE_S12 || MODE == MODE_S3) {
+  if constexpr (MODE != MODE_S0 && MODE != MODE_RHS) {  // W^n (S3Q: Q)
+    const TS *p = MODE == MODE_S3Q ? pend : ppre;
 #pragma unroll
-    for (int c = 0; c < kNC; c++) pre[c] = (TC)St<TS>::ld(&at_b(ppre, qb(c))) * S(c);
+    for (int c = 0; c < kNC; c++) pre[c] = (TC)St<TS>::ld(&at_b(p, qb(c))) * S(c);
   }
   if constexpr (MODE == MODE_S3) {
 #pragma unroll
@@ -170,6 +179,17 @@ __device__ __forceinline__ void pml_face_march(const StageArgs<TS, TC> &a, int f
   if constexpr (MODE == MODE_S12) {
 #pragma unroll
     for (int c = 0; c < kNC; c++) St<TS>::st(&at_b(pout, qb(c)), (pre[c] + a.ca * Ph[c]) * IS(c));
+  } else if constexpr (MODE == MODE_S1Q) {
+#pragma unroll
+    for (int c = 0; c < kNC; c++) {
+      const TC d2 = a.ca * Ph[c];
+      St<TS>::st(&at_b(pout, qb(c)), (pre[c] + d2) * IS(c));
+      St<TS>::st(&at_b(pend, qb(c)), rk_sum(a.rk_w, pre[c], P[c], d2) * IS(c));
+    }
+  } else if constexpr (MODE == MODE_S3Q) {
+#pragma unroll
+    for (int c = 0; c < kNC; c++)
+      St<TS>::st(&at_b(pend, qb(c)), rk_end(a.rk_w, pre[c], P[c], a.cb * Ph[c]) * IS(c));
   } else if constexpr (MODE == MODE_S0) {
 #pragma unroll
     for (int c = 0; c < kNC; c++) St<TS>::st(&at_b(pout, qb(c)), (P[c] + a.ca * Ph[c]) * IS(c));

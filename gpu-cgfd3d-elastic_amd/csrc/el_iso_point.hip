@@ -52,6 +52,14 @@ __device__ __forceinline__ void rk_store(const StageArgs<TS, TC> &a, long so, in
     } else if constexpr (MODE == MODE_S12) {
       const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc;
       St<TS>::st(&at_b(wout, qb), (pre + a.ca * h[c]) * is);
+    } else if constexpr (MODE == MODE_S1Q) {
+      const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc, u1 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
+      const TC d2 = a.ca * h[c];
+      St<TS>::st(&at_b(wout, qb), (pre + d2) * is);
+      St<TS>::st(&at_b(wend, qb), rk_sum(a.rk_w, pre, u1, d2) * is);
+    } else if constexpr (MODE == MODE_S3Q) {
+      const TC q = (TC)St<TS>::ld(&at_b(wend, qb)) * sc, u3 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
+      St<TS>::st(&at_b(wend, qb), rk_end(a.rk_w, q, u3, a.cb * h[c]) * is);
     } else {
       const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc;
       const TC u3 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
@@ -262,11 +270,13 @@ __global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
     const TC sc = St<TS>::scaled ? TC(1) / (TC)a.isc[c] : TC(1);
     const TC is = St<TS>::scaled ? (TC)a.isc[c] : TC(1);
     // stage values take a_i dt of the source (U_{i+1} = W + a_i dt (K_i + S_i)),
-    // W^{n+1} takes b3 dt of stage 3's; those of stages 0..2 reach it through U1..U3
+    // W^{n+1} takes b3 dt of stage 3's; those of stages 0..2 reach it through
+    // U1..U3 (U2's through Q where S1Q has formed it from the sweep's K1)
     if (a.mode == MODE_RHS) {
       St<TS>::st(a.w_out + q, ((TC)St<TS>::ld(a.w_out + q) * sc + v[c]) * is);
-    } else if (a.mode == MODE_S0 || a.mode == MODE_S12) {
+    } else if (a.mode == MODE_S0 || a.mode == MODE_S12 || a.mode == MODE_S1Q) {
       St<TS>::st(a.w_out + q, ((TC)St<TS>::ld(a.w_out + q) * sc + a.ca * v[c]) * is);
+      if (a.mode == MODE_S1Q) St<TS>::st(a.w_end + q, ((TC)St<TS>::ld(a.w_end + q) * sc + a.w2 * (a.ca * v[c])) * is);
     } else {
       St<TS>::st(a.w_end + q, ((TC)St<TS>::ld(a.w_end + q) * sc + a.cb * v[c]) * is);
     }
@@ -405,12 +415,15 @@ hipError_t launch_point(const StageArgs<TS, TC> &a, int dx, int dy, int dz, int 
   if (n == 0) return hipSuccess;
   const dim3 grid((unsigned)((n + 255) / 256), (unsigned)nshots);
   const int sel = dx * 4 + dy * 2 + dz;
-  switch (a.mode) {
-    case MODE_S0: launch_point_m<MODE_S0>(a, grid, sel, st); break;
-    case MODE_S12: launch_point_m<MODE_S12>(a, grid, sel, st); break;
-    case MODE_S3: launch_point_m<MODE_S3>(a, grid, sel, st); break;
-    default: launch_point_m<MODE_RHS>(a, grid, sel, st); break;
+  if constexpr (St<TS>::scaled) {
+    if (a.mode == MODE_S3) launch_point_m<MODE_S3>(a, grid, sel, st);
+  } else {
+    if (a.mode == MODE_S1Q) launch_point_m<MODE_S1Q>(a, grid, sel, st);
+    if (a.mode == MODE_S3Q) launch_point_m<MODE_S3Q>(a, grid, sel, st);
   }
+  if (a.mode == MODE_S0) launch_point_m<MODE_S0>(a, grid, sel, st);
+  if (a.mode == MODE_S12) launch_point_m<MODE_S12>(a, grid, sel, st);
+  if (a.mode == MODE_RHS) launch_point_m<MODE_RHS>(a, grid, sel, st);
   return hipGetLastError();
 }
 

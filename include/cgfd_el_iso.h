@@ -48,10 +48,11 @@ extern "C" {
 /* Four wavefield levels per shot.  A step stores the stage values
  * U_{i+1} = W^n + a_i dt K_i and forms W^{n+1} = W^n + w1 (U1 - W^n) +
  * w2 (U2 - W^n) + w3 (U3 - W^n) + b3 dt K3 (w = 1/3, 2/3, 1/3), the classical
- * RK4 step of drv_rk_curv_col.cu:193-542 with 117 instead of 144 level
- * words moved per point and step. */
+ * RK4 step of drv_rk_curv_col.cu:193-542 with 108 (FP32, FP64: the sum over
+ * W^n, U1 and U2 is kept as one level) or 117 (16-bit storage) instead of 144
+ * level words moved per point and step. */
 #define CGFD_LEVEL_PRE 0   /* W^n: the level receivers and snapshots read */
-#define CGFD_LEVEL_TMPA 1  /* after a step: W^{n-1}; during it U1 (stage value of stage 0) */
+#define CGFD_LEVEL_TMPA 1  /* after a step: W^{n-1} */
 #define CGFD_LEVEL_TMPB 2  /* U2 of the last step */
 #define CGFD_LEVEL_END 3   /* U3 of the last step */
 #define CGFD_LEVEL_RHS 4   /* right-hand side written by cgfd_el_iso_onestage */
