@@ -162,12 +162,20 @@ struct cgfd_session {
   std::vector<RecvHost> rec;
   // device source CSR (grow-only buffers: capacities in bytes)
   int s_npt = 0;
-  size_t s_cap[11] = {0};
+  size_t s_cap[14] = {0};
   int *s_pt_shot = nullptr, *s_pt_beg = nullptr, *s_ct_src = nullptr, *s_itb = nullptr, *s_ite = nullptr,
       *s_kind = nullptr;
   long *s_pt_off = nullptr, *s_tab = nullptr;
   void *s_ct_coef = nullptr, *s_F = nullptr, *s_M = nullptr;
   long s_ntab = 0;
+  // Source boxes (src_boxed): every shot's points lie in a box of at most
+  // kMaxSrcBox physical points, and the stages add the rates that the step's
+  // head tabulates over it.  Otherwise k_source follows each stage.
+  bool src_boxed = false;
+  long s_vol = 0;               // points reserved per box
+  int *s_pt_cell = nullptr;
+  SrcBox *s_box = nullptr;
+  void *s_v = nullptr;          // [nshots][4][9][s_vol]
   bool src_dirty = false;
   // device receivers
   int r_n = 0;
@@ -192,7 +200,7 @@ struct cgfd_session {
   void *host_seismo = nullptr;  // hipHostMalloc, nshots * host_stride samples
   long host_stride = 0;
   std::vector<int> start_h, active_h;  // host copies of shot_start / shot_active
-  int *clock = nullptr, *shot_start = nullptr, *shot_active = nullptr;
+  int *clock = nullptr, *shot_start = nullptr, *shot_active = nullptr;  // clock[2]: step it reads clock[it & 1]
   // interior tile choice (-1: not tuned yet)
   int tile_shape = -1, tile_zchunk = 48;
   bool tile_fixed = false;
@@ -452,6 +460,12 @@ int copy_window(cgfd_session *s, int a, int b) {
   return CGFD_OK;
 }
 
+// Largest source box that the stages add from a table: a 7x7x7 spread is 343
+// points, so a few sources close together still fit.  The table is rewritten
+// every step (36 values per point); beyond this the writes and the memory (64
+// shots: 38 MB at 4096 points) outgrow the launches they save.
+constexpr long kMaxSrcBox = 4096;
+
 // ---- rebuild device source CSR over all shots ----
 template <typename TM> int build_sources(cgfd_session *s) {
   s->s_npt = 0;
@@ -485,8 +499,44 @@ template <typename TM> int build_sources(cgfd_session *s) {
   }
   const int npt = (int)pts.size();
   s->s_ntab = ntab;
+  s->src_boxed = false;
   invalidate(s);
   if (npt == 0) { s->src_dirty = false; return CGFD_OK; }
+  // boxes over the shots' points; a point in the ghosts (accepted by the
+  // upload, never updated by a stage) rules them out
+  const Layout &L = s->L;
+  auto ijk = [&](long off, int *q) {
+    q[2] = (int)(off / L.pz) - kNG;
+    q[1] = (int)(off % L.pz / L.px) - kNG;
+    q[0] = (int)(off % L.px) - L.xa;
+  };
+  std::vector<SrcBox> box(s->d.nshots, SrcBox{0, 0, 0, 0, 0, 0});
+  bool boxed = true;
+  long vol = 0;
+  for (auto &kv : pts) {
+    int q[3];
+    ijk(kv.first.second, q);
+    if (q[0] < 0 || q[1] < 0 || q[2] < 0 || q[0] >= L.ni || q[1] >= L.nj || q[2] >= L.nk) { boxed = false; break; }
+    SrcBox &b = box[kv.first.first];
+    if (b.ni == 0) { b = SrcBox{q[0], q[1], q[2], 1, 1, 1}; }
+    int *lo[3] = {&b.i0, &b.j0, &b.k0}, *n[3] = {&b.ni, &b.nj, &b.nk};
+    for (int d = 0; d < 3; d++) {
+      const int hi = std::max(*lo[d] + *n[d] - 1, q[d]);
+      *lo[d] = std::min(*lo[d], q[d]);
+      *n[d] = hi - *lo[d] + 1;
+    }
+    const long v = (long)b.ni * b.nj * b.nk;
+    if (v > kMaxSrcBox) { boxed = false; break; }
+    vol = std::max(vol, v);
+  }
+  std::vector<int> pt_cell;
+  if (boxed)
+    for (auto &kv : pts) {
+      int q[3];
+      ijk(kv.first.second, q);
+      const SrcBox &b = box[kv.first.first];
+      pt_cell.push_back(((q[2] - b.k0) * b.nj + (q[1] - b.j0)) * b.ni + (q[0] - b.i0));
+    }
   std::vector<int> pt_shot, pt_beg, ct_src;
   std::vector<long> pt_off;
   std::vector<TM> ct_coef;
@@ -519,6 +569,16 @@ template <typename TM> int build_sources(cgfd_session *s) {
   for (int c = 0; c < 6; c++) Mall.insert(Mall.end(), M[c].begin(), M[c].end());
   if ((r = up(&s->s_F, Fall.data(), Fall.size() * sizeof(TM)))) return r;
   if ((r = up(&s->s_M, Mall.data(), Mall.size() * sizeof(TM)))) return r;
+  if (boxed) {
+    if ((r = up((void **)&s->s_pt_cell, pt_cell.data(), pt_cell.size() * 4))) return r;
+    if ((r = up((void **)&s->s_box, box.data(), box.size() * sizeof(SrcBox)))) return r;
+    // cells of a box that no point fills stay zero
+    const size_t nv = (size_t)s->d.nshots * 4 * kNC * vol;
+    if ((r = ensure(s, &s->s_v, &s->s_cap[slot++], nv * sizeof(TM)))) return r;
+    if ((r = fill_zero(s, s->s_v, nv, sizeof(TM)))) return r;
+    s->s_vol = vol;
+    s->src_boxed = true;
+  }
   s->s_npt = npt;
   s->src_dirty = false;
   return CGFD_OK;
@@ -667,14 +727,8 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
   a.w_end = w + (long)slot_end * s->level_elems;
   a.w_u2 = w + (long)slot_u2 * s->level_elems;
   a.shot_stride = rhs_mode ? 0 : s->shot_elems;
-  // weights of the stage values: w_i = b_{i-1} / a_{i-1}; w3 is rounded down
-  // to a value whose complement is exact where the sum Q uses both
+  // weights of the stage values: w_i = b_{i-1} / a_{i-1}
   for (int q = 0; q < 3; q++) a.rk_w[q] = (TC)(kRkB[q] / kRkA[q]);
-  if constexpr (!St<TS>::scaled) {
-    const double p = sizeof(TC) == 8 ? 9007199254740992.0 : 16777216.0;  // 2^53, 2^24
-    a.rk_w[2] = (TC)(std::floor(p / 3.0) / p);
-    a.rk_w[3] = TC(1) - a.rk_w[2];
-  }
   for (int c = 0; c < kNC; c++) { a.sc[c] = s->sc[c]; a.isc[c] = s->isc[c]; }
   a.shot_active = s->shot_active;
   return a;
@@ -721,7 +775,7 @@ struct Shell {
 // faster than with the core's chunk, and 5 % / 7 % faster than with twice it.
 int rim_zchunk(int core_zchunk) { return std::max(4, core_zchunk / 3); }
 
-Shell make_shell(cgfd_session *s) {
+Shell make_shell(cgfd_session *s, int shape = -1) {
   Shell sh{};
   const int ni = s->d.ni, nj = s->d.nj, nk = s->d.nk;
   auto lay = [&](int f) { return s->face[f].on ? s->face[f].nlay + 1 : 0; };
@@ -742,7 +796,7 @@ Shell make_shell(cgfd_session *s) {
     return sh;
   }
   sh.inner.zchunk = s->tile_zchunk;
-  sh.inner.shape = s->tile_shape < 0 ? 0 : s->tile_shape;
+  sh.inner.shape = shape >= 0 ? shape : s->tile_shape < 0 ? 0 : s->tile_shape;
   sh.rim.zchunk = rim_zchunk(sh.inner.zchunk);
   sh.rim.shape = sh.inner.shape;
   sh.rim.pml = 1;
@@ -751,8 +805,7 @@ Shell make_shell(cgfd_session *s) {
     if (s->split == CGFD_SPLIT_CORE) {
       // core: x from the first tile boundary at or past the x1 face box to
       // the last one before the x2 face box, y likewise on the tile height
-      int tx = 0, ty = 0;
-      interior_shape(sh.inner.shape, &tx, &ty);
+      const int tx = kTile[sh.inner.shape][0], ty = kTile[sh.inner.shape][1];
       const int ca0 = (ib0 + tx - 1) / tx * tx, ca1 = ca0 + (ib1 + 1 - ca0) / tx * tx - 1;
       const int cb0 = (jb0 + ty - 1) / ty * ty, cb1 = cb0 + (jb1 + 1 - cb0) / ty * ty - 1;
       if (ca1 >= ca0 && cb1 >= cb0) {
@@ -839,6 +892,16 @@ struct TileChoice {
 std::map<TileKey, TileChoice> g_tile_cache;
 std::mutex g_tile_mu;
 
+// workgroups of a sweep with the given z chunk
+long march_workgroups(const MarchSet &m, int zchunk) {
+  const int tx = kTile[m.shape][0], ty = kTile[m.shape][1];
+  long n = 0;
+  for (int q = 0; q < m.nbox; q++)
+    n += (long)((m.box[q][1] - m.box[q][0] + tx) / tx) * ((m.box[q][3] - m.box[q][2] + ty) / ty) *
+         ((m.box[q][5] - m.box[q][4] + zchunk) / zchunk);
+  return n;
+}
+
 template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   TileKey key{s->d.ni, s->d.nj, s->d.nk, s->d.storage, s->d.nshots, s->d.flags, s->met_const ? 1 : 0, s->free_top,
               {}, s->split_fixed ? s->split : -1};
@@ -919,9 +982,13 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
     // z chunks near 16..48 planes that split the swept planes evenly: every
     // chunk re-reads 4 planes below it, so a short last chunk costs almost a
     // full one (196 planes: 17, 20, 25, 28, 33, 49 instead of 16 .. 48,
-    // whose last chunk has 4 planes)
-    constexpr int kNZ = 8;
-    const int ztarget[kNZ] = {16, 20, 24, 28, 32, 48, 64, 96};
+    // whose last chunk has 4 planes).  Chunks of 4..12 planes are for sweeps
+    // that 16-plane chunks would leave with fewer than 2048 workgroups (8 per
+    // CU): there the idle CUs cost more than the planes read twice (64^3: 40
+    // workgroups of 17 planes, 38 us a sweep).  With 16-bit storage they would
+    // also move small grids from one split to another, whose roundings differ.
+    constexpr int kNZ = 12;
+    const int ztarget[kNZ] = {4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
     int zcands[kNZ];
     for (int zi = 0; zi < kNZ; zi++) {
       const int n = std::max(1, (nz + ztarget[zi] / 2) / ztarget[zi]);
@@ -929,12 +996,13 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
     }
     float best = 1e30f;
     int ts = 0, tz = 24;
-    for (int shape = 0; shape < interior_num_shapes(); shape++) {
+    for (int shape = 0; shape < kNumShapes; shape++) {
       s->tile_shape = shape;
       const Shell shs = make_shell(s);  // the core's bounds follow the tile shape
       for (int zi = 0; zi < kNZ; zi++) {
         const int zc = zcands[zi];
         if (zi > 0 && zc == zcands[zi - 1]) continue;
+        if (ztarget[zi] < 16 && (St<TS>::scaled || march_workgroups(shs.inner, 16) * s->d.nshots >= 2048)) continue;
         MarchSet ib = shs.inner, rb = shs.rim;
         ib.zchunk = zc;
         rb.zchunk = rim_zchunk(zc);
@@ -973,24 +1041,43 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   return CGFD_OK;
 }
 
+// Arguments of the source kernels; the stage's outputs and weights are set by
+// the caller.  table: rates tabulated over the boxes (needs src_boxed).
+template <typename TS, typename TC> SrcArgs<TS, TC> source_args(cgfd_session *s, bool table) {
+  SrcArgs<TS, TC> sa{};
+  sa.L = s->L; sa.npt = s->s_npt; sa.pt_shot = s->s_pt_shot; sa.pt_off = s->s_pt_off; sa.pt_beg = s->s_pt_beg;
+  sa.ct_src = s->s_ct_src; sa.ct_coef = (const TC *)s->s_ct_coef; sa.s_itb = s->s_itb; sa.s_ite = s->s_ite;
+  sa.s_tab = s->s_tab; sa.s_kind = s->s_kind; sa.F = (const TC *)s->s_F; sa.M = (const TC *)s->s_M;
+  sa.ntab = s->s_ntab; sa.met = (const TC *)s->met; sa.med = (const TC *)s->med;
+  sa.shot_start = s->shot_start; sa.shot_active = s->shot_active;
+  sa.only_shot = -1;
+  if (table) { sa.pt_cell = s->s_pt_cell; sa.src_v = (TC *)s->s_v; sa.src_vol = s->s_vol; }
+  for (int c = 0; c < kNC; c++) sa.isc[c] = s->isc[c];
+  return sa;
+}
+
 // Enqueue steps it0 .. it0+nsteps-1 of the RK4 loop on the session stream:
-// receivers, four stages (interior sweep, PML slabs / free-surface rows,
-// source) and the clock advance per step, then the W <-> U1 swap.
+// the head (receivers, source rates, clock), four stages (interior sweep, PML
+// slabs / free-surface rows, sources that have no box) per step, then the W <->
+// W^{n+1} swap.
 template <typename TS, typename TC>
 int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, bool timed) {
+  const bool boxed = s->s_npt > 0 && s->src_boxed;
   for (int n = 0; n < nsteps; n++) {
     const int it = it0 + n;
-    // receivers read W^n before the step (drv_rk_curv_col.cu:195-216)
-    if (s->r_n > 0) {
+    const int *clock = s->clock + (it & 1);
+    {
+      // receivers read W^n before the step (drv_rk_curv_col.cu:195-216)
       RecvArgs<TS, TC> ra{};
       ra.nrec = s->r_n; ra.r_shot = s->r_shot; ra.r_off = s->r_off; ra.r_frac = (const TC *)s->r_frac;
       ra.r_out = s->r_out; ra.r_nt = s->r_nt; ra.seismo = (TC *)s->seismo; ra.ring = s->ring;
       ra.w_pre = (const TS *)s->wav + (long)s->slot[0] * s->level_elems;
       ra.shot_stride = s->shot_elems; ra.cs = s->L.cs;
-      ra.clock = s->clock; ra.shot_start = s->shot_start; ra.shot_active = s->shot_active;
+      ra.shot_start = s->shot_start; ra.shot_active = s->shot_active;
       for (int c = 0; c < kNC; c++) ra.sc[c] = s->sc[c];
-      hipError_t e = launch_recv<TS, TC>(ra, s->st);
-      if (e != hipSuccess) return fail(CGFD_E_HIP, "receiver kernel: %s", hipGetErrorString(e));
+      const SrcArgs<TS, TC> sa = source_args<TS, TC>(s, boxed);
+      hipError_t e = launch_step_head<TS, TC>(ra, sa, clock, s->clock + ((it + 1) & 1), s->st);
+      if (e != hipSuccess) return fail(CGFD_E_HIP, "step head kernel: %s", hipGetErrorString(e));
     }
     const int ipair = it % 8;
     for (int istage = 0; istage < 4; istage++) {
@@ -1003,6 +1090,11 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
       // coef = rk_a[istage]*dt, both float in the reference (drv_rk_curv_col.cu:341-342)
       a.ca = (istage < 3) ? (TC)kRkA[istage] * dt : TC(0);
       a.cb = (TC)kRkB[istage] * dt;
+      if (boxed && kBoxedSrc<TS>) {
+        a.sbox = s->s_box;
+        a.src_v = (const TC *)s->s_v + (long)istage * kNC * s->s_vol;
+        a.src_vol = s->s_vol;
+      }
       const bool tim = timed && sh.inner.nbox;
       if (tim && s->ev.size() < s->ev_used + 2) {
         s->ev.resize(s->ev_used + 2);
@@ -1012,17 +1104,11 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
                                    tim ? s->ev[s->ev_used + 1] : nullptr);
       if (r) return r;
       if (tim) s->ev_used += 2;
-      if (s->s_npt > 0) {
-        SrcArgs<TS, TC> sa{};
-        sa.L = s->L; sa.npt = s->s_npt; sa.pt_shot = s->s_pt_shot; sa.pt_off = s->s_pt_off; sa.pt_beg = s->s_pt_beg;
-        sa.ct_src = s->s_ct_src; sa.ct_coef = (const TC *)s->s_ct_coef; sa.s_itb = s->s_itb; sa.s_ite = s->s_ite;
-        sa.s_tab = s->s_tab; sa.s_kind = s->s_kind; sa.F = (const TC *)s->s_F; sa.M = (const TC *)s->s_M;
-        sa.ntab = s->s_ntab; sa.met = (const TC *)s->met; sa.med = (const TC *)s->med;
+      if (s->s_npt > 0 && !(boxed && kBoxedSrc<TS>)) {
+        SrcArgs<TS, TC> sa = source_args<TS, TC>(s, boxed);
         sa.w_out = a.w_out; sa.w_end = a.w_end; sa.shot_stride = s->shot_elems;
         sa.mode = p.mode; sa.istage = istage; sa.ca = a.ca; sa.cb = a.cb; sa.w2 = a.rk_w[1];
-        sa.clock = s->clock; sa.shot_start = s->shot_start; sa.shot_active = s->shot_active;
-        sa.only_shot = -1; sa.fixed_it = 0;
-        for (int c = 0; c < kNC; c++) sa.isc[c] = s->isc[c];
+        sa.clock = clock;
         hipError_t e = launch_source<TS, TC>(sa, s->st);
         if (e != hipSuccess) return fail(CGFD_E_HIP, "source kernel: %s", hipGetErrorString(e));
       }
@@ -1034,8 +1120,6 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
                                          s->d.nshots, s->st);
       if (e != hipSuccess) return fail(CGFD_E_HIP, "peak motion kernel: %s", hipGetErrorString(e));
     }
-    hipError_t e = launch_clock_advance(s->clock, s->st);
-    if (e != hipSuccess) return fail(CGFD_E_HIP, "clock kernel: %s", hipGetErrorString(e));
     std::swap(s->slot[0], s->slot[1]);  // W^{n+1} becomes W (drv_rk_curv_col.cu:529-541)
   }
   return CGFD_OK;
@@ -1078,7 +1162,7 @@ template <typename TS, typename TC> int enqueue_t(cgfd_session *s, int it0, int 
   if (s->rec_dirty) { int r = build_receivers<TC>(s); if (r) return r; }
   const Shell sh = make_shell(s);
   const TC dt = (TC)dt_in;
-  hipError_t e = launch_fill<int>(s->clock, 1, it0, s->st);
+  hipError_t e = launch_fill<int>(s->clock + (it0 & 1), 1, it0, s->st);
   if (e != hipSuccess) return fail(CGFD_E_HIP, "clock set: %s", hipGetErrorString(e));
   s->ev_used = 0;
   const bool graphs = s->use_graph && !s->timing;
@@ -1171,22 +1255,16 @@ template <typename TS, typename TC> int onestage_t(cgfd_session *s, int shot, in
   a.shot_active = nullptr;
   a.mode = MODE_RHS;
   a.ca = TC(0); a.cb = TC(0);
-  const Shell sh = make_shell(s);
+  const Shell sh = make_shell(s, kRhsShape);
   int r = launch_stage<TS, TC>(s, sh, a, dx, dy, dz, 1, nullptr, nullptr);
   if (r) return r;
   if (s->s_npt > 0) {
     // the source kernel scans all shots' points; inject this shot's at step it
-    SrcArgs<TS, TC> sa{};
-    sa.L = s->L; sa.npt = s->s_npt; sa.pt_shot = s->s_pt_shot; sa.pt_off = s->s_pt_off; sa.pt_beg = s->s_pt_beg;
-    sa.ct_src = s->s_ct_src; sa.ct_coef = (const TC *)s->s_ct_coef; sa.s_itb = s->s_itb; sa.s_ite = s->s_ite;
-    sa.s_tab = s->s_tab; sa.s_kind = s->s_kind; sa.F = (const TC *)s->s_F; sa.M = (const TC *)s->s_M;
-    sa.ntab = s->s_ntab; sa.met = (const TC *)s->met; sa.med = (const TC *)s->med;
+    SrcArgs<TS, TC> sa = source_args<TS, TC>(s, false);
     sa.w_out = (TS *)s->rhs; sa.w_end = (TS *)s->rhs;
     sa.shot_stride = 0;
-    sa.mode = MODE_RHS; sa.istage = istage; sa.ca = TC(0); sa.cb = TC(0);
-    sa.clock = s->clock; sa.shot_start = s->shot_start; sa.shot_active = s->shot_active;
+    sa.mode = MODE_RHS; sa.istage = istage;
     sa.only_shot = shot; sa.fixed_it = it;
-    for (int c = 0; c < kNC; c++) sa.isc[c] = s->isc[c];
     hipError_t e = launch_source<TS, TC>(sa, s->st);
     if (e != hipSuccess) return fail(CGFD_E_HIP, "source kernel: %s", hipGetErrorString(e));
   }
@@ -1213,10 +1291,10 @@ long long cgfd_footprint_bytes(const cgfd_desc *d, int nrecv, int nt_total) {
   long long wav = ns * 4LL * kNC * L.cs * (long long)es;
   long long model = (long long)(NMET + 3) * L.cs * (long long)ms + 18LL * d->ni * d->nj * (long long)ms;
   // peak-motion maps (when enabled), the sub-volume gather buffer (at most
-  // one component) and the source tables (7^3 points, 9 tables of 4 stage
-  // values per step, per shot)
+  // one component) and the source tables (7^3 points with 36 rates each, 9
+  // tables of 4 stage values per step, per shot)
   long long extra = ns * 18LL * d->ni * d->nj * (long long)ms + L.cs * (long long)ms +
-                    ns * (343LL * 24 + 9LL * 4 * (nt_total > 0 ? nt_total : 0) * (long long)ms);
+                    ns * (343LL * (28 + 36 * (long long)ms) + 9LL * 4 * (nt_total > 0 ? nt_total : 0) * (long long)ms);
   // PML memory: 5 faces of 11 layers at most is bounded by 5 levels over the shell
   long long shell = 2LL * 11 * d->nj * d->nk + 2LL * 11 * d->ni * d->nk + 2LL * 11 * d->ni * d->nj;
   long long aux = ns * 5LL * kNC * shell * (long long)es;
@@ -1266,7 +1344,7 @@ int cgfd_create(const cgfd_desc *d, cgfd_session **out) {
   if ((r = dalloc(s, &s->met, (size_t)NMET * s->L.cs * s->ms))) return cleanup(r);
   if ((r = dalloc(s, &s->med, (size_t)3 * s->L.cs * s->ms))) return cleanup(r);
   if ((r = dalloc(s, &s->mat, (size_t)18 * d->ni * d->nj * s->ms))) return cleanup(r);
-  if ((r = dalloc(s, (void **)&s->clock, sizeof(int)))) return cleanup(r);
+  if ((r = dalloc(s, (void **)&s->clock, 2 * sizeof(int)))) return cleanup(r);
   if ((r = dalloc(s, (void **)&s->shot_start, sizeof(int) * d->nshots))) return cleanup(r);
   if ((r = dalloc(s, (void **)&s->shot_active, sizeof(int) * d->nshots))) return cleanup(r);
   if ((r = fill_zero(s, s->wav, (size_t)d->nshots * s->shot_elems, s->es))) return cleanup(r);
@@ -1275,7 +1353,7 @@ int cgfd_create(const cgfd_desc *d, cgfd_session **out) {
   if ((r = fill_zero(s, s->mat, (size_t)18 * d->ni * d->nj, s->ms))) return cleanup(r);
   if (launch_fill<int>(s->shot_start, d->nshots, 0, s->st) != hipSuccess ||
       launch_fill<int>(s->shot_active, d->nshots, 1, s->st) != hipSuccess ||
-      launch_fill<int>(s->clock, 1, 0, s->st) != hipSuccess)
+      launch_fill<int>(s->clock, 2, 0, s->st) != hipSuccess)
     return cleanup(fail(CGFD_E_HIP, "initial fills failed"));
   s->src.resize(d->nshots);
   s->rec.resize(d->nshots);
@@ -1760,7 +1838,7 @@ int cgfd_set_tile(cgfd_session *s, int shape, int zchunk) {
     s->tile_shape = -1;
     return CGFD_OK;
   }
-  if (shape >= interior_num_shapes() || zchunk < 1) return fail(CGFD_E_ARG, "tile %d/%d invalid", shape, zchunk);
+  if (shape >= kNumShapes || zchunk < 1) return fail(CGFD_E_ARG, "tile %d/%d invalid", shape, zchunk);
   s->tile_fixed = true;
   s->tile_shape = shape;
   s->tile_zchunk = zchunk;
@@ -1792,8 +1870,7 @@ int cgfd_get_split(cgfd_session *s, int *split) {
 }
 int cgfd_get_tile(cgfd_session *s, int *shape, int *tx, int *ty, int *zchunk) {
   if (!s) return fail(CGFD_E_ARG, "null session");
-  int sh = s->tile_shape < 0 ? 0 : s->tile_shape, a = 0, b = 0;
-  interior_shape(sh, &a, &b);
+  const int sh = s->tile_shape < 0 ? 0 : s->tile_shape, a = kTile[sh][0], b = kTile[sh][1];
   if (shape) *shape = s->tile_shape;
   if (tx) *tx = a;
   if (ty) *ty = b;

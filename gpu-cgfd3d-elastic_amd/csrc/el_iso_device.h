@@ -127,16 +127,26 @@ template <typename TC> __device__ __forceinline__ TC rk_partial(const TC *w, TC 
 template <typename TC> __device__ __forceinline__ TC rk_final(TC y0, TC partial, TC w3, TC u3, TC cbh) {
   return y0 + ((partial + w3 * (u3 - y0)) + cbh);
 }
+// S1Q and S3Q spell their roundings out: which product of a sum the compiler
+// fuses would otherwise differ between the sweep's variants, and at a wave front
+// the stages cancel, which made it 4e-6 of a seismogram instead of 1e-10.
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 // S1Q: Q from W, U1 and U2's increment d2 = a1 dt K1 (the increment itself:
-// U2's rounding then stays out of Q).  w[2] = w3 is the value just below 1/3
-// for which w[3] = 1 - w3 is exact: a constant field stays constant, and the
-// 6e-8 (FP32) by which w3 misses 1/3 multiplies only U3 - W.
-template <typename TC> __device__ __forceinline__ TC rk_sum(const TC *w, TC y0, TC u1, TC d2) {
-  return w[3] * y0 + (w[0] * (u1 - y0) + w[1] * d2);
+// U2's rounding then stays out of Q).  (1 - w3) W is taken as W - w3 W with the
+// w3 that S3Q adds back, so the 1e-8 by which an FP32 w3 misses 1/3 multiplies
+// U3 - W as it does in S3; a complement rounded on its own drifts twice as fast
+// (2.2e-6 against 1.1e-6, S3 1.2e-6, after 500 FP32 steps of an oscillator).
+template <typename TC> __device__ __forceinline__ void rk_sum(const TC *w, TC y0, TC u1, TC ca, TC h, TC &u2, TC &q) {
+#pragma clang fp contract(off)
+  const TC d2 = ca * h;
+  u2 = y0 + d2;
+  q = y0 + fma_t(-w[2], y0, fma_t(w[0], u1 - y0, w[1] * d2));
 }
 // S3Q
-template <typename TC> __device__ __forceinline__ TC rk_end(const TC *w, TC q, TC u3, TC cbh) {
-  return q + (w[2] * u3 + cbh);
+template <typename TC> __device__ __forceinline__ TC rk_end(const TC *w, TC q, TC u3, TC cb, TC h) {
+#pragma clang fp contract(off)
+  return q + fma_t(w[2], u3, cb * h);
 }
 
 // ---- operator constants (src/forward/fd_t.cu:76-148) ----------------------
@@ -185,6 +195,14 @@ template <typename TS, typename TM> struct FaceArgs {
 // boxes one per-point launch may cover (the boundary shell splits into at most 26)
 constexpr int kMaxBox = 26;
 
+// storage types whose stage kernels add sources from the step's table
+template <typename TS> constexpr bool kBoxedSrc = !St<TS>::scaled;
+
+// Bounding box (physical) of one shot's source points; ni = 0: none.
+struct SrcBox {
+  int i0, j0, k0, ni, nj, nk;
+};
+
 template <typename TS, typename TM> struct StageArgs {
   Layout L;
   const TM *met;   // NMET components, stride L.cs
@@ -201,12 +219,18 @@ template <typename TS, typename TM> struct StageArgs {
   long shot_stride;
   int mode;
   TM ca, cb;      // a_i dt and b_i dt of the stage
-  TM rk_w[4];     // w1, w2, w3 of the last stage's combination and 1 - w3
+  TM rk_w[3];     // w1, w2, w3 of the last stage's combination
   float sc[kNC], isc[kNC];  // storage scale (value = stored*sc) and its inverse
   int nbox;
   int box[kMaxBox][6];      // i1,i2,j1,j2,k1,k2 inclusive, physical
   long box_end[kMaxBox];    // cumulative point counts
   const int *shot_active;   // per-shot 0/1, or null
+  // Source rates of this step and stage over each shot's box, added to the
+  // right-hand side where it is formed (null: sources come from k_source, and
+  // always with 16-bit storage, whose outputs are rounded before the source).
+  const SrcBox *sbox;       // [nshots]
+  const TM *src_v;          // shot 0's rates of this stage, [9][src_vol]
+  long src_vol;             // points reserved per box; a shot's stages are 4*9*src_vol apart
 };
 
 // Source contributions grouped by grid point (CSR), all shots of a session.
@@ -237,6 +261,9 @@ template <typename TS, typename TM> struct SrcArgs {
   int only_shot;            // >= 0: inject this shot only, at step fixed_it
   int fixed_it;
   float isc[kNC];
+  const int *pt_cell;       // [npt] cell in the shot's box
+  TM *src_v;                // [nshots][4][9][src_vol] rates of a step tabulated by k_step_head, or null
+  long src_vol;
 };
 
 template <typename TS, typename TC> struct RecvArgs {

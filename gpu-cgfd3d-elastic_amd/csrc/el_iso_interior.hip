@@ -104,6 +104,16 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
         tile_faces |= 1u << fi;
     }
   }
+  // planes of this tile that meet the shot's source box (none: src_k0 > src_k1)
+  int src_k0 = 1, src_k1 = 0;
+  constexpr bool boxed = kBoxedSrc<TS> && MODE != MODE_RHS;
+  if (boxed && a.sbox) {
+    const SrcBox sb = a.sbox[shot];
+    if (sb.ni > 0 && sb.i0 < i0 + TX && sb.i0 + sb.ni > i0 && sb.j0 < j0 + TY && sb.j0 + sb.nj > j0) {
+      src_k0 = sb.k0;
+      src_k1 = sb.k0 + sb.nk - 1;
+    }
+  }
   // lanes past the last ghost column/row only feed LDS cells no owner reads;
   // clamping their address keeps every load unconditional and in bounds
   const int ic = i <= L.ni + 2 ? i : L.ni + 2, jc = j <= L.nj + 2 ? j : L.nj + 2;
@@ -364,6 +374,8 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
           else face(std::integral_constant<int, 2>{}, fi);
         }
       }
+      if constexpr (boxed)
+        if (k >= src_k0 && k <= src_k1) src_add<TS, TC>(a, shot, i, j, k, h);
 #pragma unroll
       for (int c = 0; c < kNC; c++) {
         TS *wout = a.w_out + so + c * cs;
@@ -374,11 +386,12 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
         if constexpr (mode == MODE_S12) {
           st_w(&at_b(wout, qb), (pre_c + a.ca * h[c]) * is);
         } else if constexpr (mode == MODE_S1Q) {
-          const TC d2 = a.ca * h[c];
-          st_w(&at_b(wout, qb), (pre_c + d2) * is);
-          st_w(&at_b(wend, qb), rk_sum(a.rk_w, pre_c, q[c][zc0], d2) * is);
+          TC u2, qs;
+          rk_sum(a.rk_w, pre_c, q[c][zc0], a.ca, h[c], u2, qs);
+          st_w(&at_b(wout, qb), u2 * is);
+          st_w(&at_b(wend, qb), qs * is);
         } else if constexpr (mode == MODE_S3Q) {
-          st_w(&at_b(wend, qb), rk_end(a.rk_w, pre_c, q[c][zc0], a.cb * h[c]) * is);
+          st_w(&at_b(wend, qb), rk_end(a.rk_w, pre_c, q[c][zc0], a.cb, h[c]) * is);
         } else if constexpr (mode == MODE_S0) {
           st_w(&at_b(wout, qb), (q[c][zc0] + a.ca * h[c]) * is);
         } else if constexpr (mode == MODE_S3) {
@@ -448,67 +461,39 @@ static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, 
   }
   CGFD_M(MODE_S0);
   CGFD_M(MODE_S12);
-  CGFD_M(MODE_RHS);
+  if constexpr (CGFD_SHAPE == kRhsShape) CGFD_M(MODE_RHS);
 #undef CGFD_M
   return hipGetLastError();
 }
 
-// tile shapes the autotuner chooses from (TX x TY threads, one per column)
-#if !defined(CGFD_TYPE) || CGFD_TYPE == 0
-int interior_num_shapes() { return 4; }
-
-void interior_shape(int id, int *tx, int *ty) {
-  static const int T[4][2] = {{64, 4}, {32, 8}, {64, 8}, {32, 16}};
-  id = id < 0 ? 0 : id > 3 ? 3 : id;
-  *tx = T[id][0];
-  *ty = T[id][1];
-}
-#endif
-
-template <typename TS, typename TC, bool PML>
-static hipError_t launch_march_shape(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz,
-                                     int nshots, hipStream_t st) {
+// One tile shape of one storage type per object file (CGFD_SHAPE, CGFD_TYPE):
+// they compile in parallel.
+template <typename TS, typename TC, int SHAPE>
+hipError_t launch_interior_shape(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz, int nshots,
+                                 hipStream_t st) {
+  constexpr int TX = kTile[SHAPE][0], TY = kTile[SHAPE][1], MINB = TX * TY > 256 ? 1 : 2;
   if (a.met_const) {
-    switch (b.shape) {
-      case 0: return launch_march_t<TS, TC, 64, 4, 2, true, PML>(a, b, dx, dy, dz, nshots, st);
-      case 1: return launch_march_t<TS, TC, 32, 8, 2, true, PML>(a, b, dx, dy, dz, nshots, st);
-      case 3: return launch_march_t<TS, TC, 32, 16, 1, true, PML>(a, b, dx, dy, dz, nshots, st);
-      default: return launch_march_t<TS, TC, 64, 8, 1, true, PML>(a, b, dx, dy, dz, nshots, st);
-    }
+    if (b.pml) return launch_march_t<TS, TC, TX, TY, MINB, true, true>(a, b, dx, dy, dz, nshots, st);
+    return launch_march_t<TS, TC, TX, TY, MINB, true, false>(a, b, dx, dy, dz, nshots, st);
   }
-  switch (b.shape) {
-    case 0: return launch_march_t<TS, TC, 64, 4, 2, false, PML>(a, b, dx, dy, dz, nshots, st);
-    case 1: return launch_march_t<TS, TC, 32, 8, 2, false, PML>(a, b, dx, dy, dz, nshots, st);
-    case 3: return launch_march_t<TS, TC, 32, 16, 1, false, PML>(a, b, dx, dy, dz, nshots, st);
-    default: return launch_march_t<TS, TC, 64, 8, 1, false, PML>(a, b, dx, dy, dz, nshots, st);
-  }
+  if (b.pml) return launch_march_t<TS, TC, TX, TY, MINB, false, true>(a, b, dx, dy, dz, nshots, st);
+  return launch_march_t<TS, TC, TX, TY, MINB, false, false>(a, b, dx, dy, dz, nshots, st);
 }
 
-template <typename TS, typename TC>
-hipError_t launch_interior(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz, int nshots,
-                           hipStream_t st) {
-  if (b.nbox < 1) return hipSuccess;
-  if (b.pml) return launch_march_shape<TS, TC, true>(a, b, dx, dy, dz, nshots, st);
-  return launch_march_shape<TS, TC, false>(a, b, dx, dy, dz, nshots, st);
-}
-
-#define CGFD_INST(TS, TC)                                                                                   \
-  template hipError_t launch_interior<TS, TC>(const StageArgs<TS, TC> &, const MarchSet &, int, int, int, int, \
-                                              hipStream_t);
-// CGFD_TYPE selects one storage type per object so the four compile in
-// parallel; without it every type is instantiated here.
-#if !defined(CGFD_TYPE) || CGFD_TYPE == 0
-CGFD_INST(float, float)
+#if CGFD_TYPE == 0
+using TypeS = float;
+using TypeC = float;
+#elif CGFD_TYPE == 1
+using TypeS = double;
+using TypeC = double;
+#elif CGFD_TYPE == 2
+using TypeS = __half;
+using TypeC = float;
+#else
+using TypeS = __hip_bfloat16;
+using TypeC = float;
 #endif
-#if !defined(CGFD_TYPE) || CGFD_TYPE == 1
-CGFD_INST(double, double)
-#endif
-#if !defined(CGFD_TYPE) || CGFD_TYPE == 2
-CGFD_INST(__half, float)
-#endif
-#if !defined(CGFD_TYPE) || CGFD_TYPE == 3
-CGFD_INST(__hip_bfloat16, float)
-#endif
-#undef CGFD_INST
+template hipError_t launch_interior_shape<TypeS, TypeC, CGFD_SHAPE>(const StageArgs<TypeS, TypeC> &, const MarchSet &,
+                                                                    int, int, int, int, hipStream_t);
 
 }  // namespace cgfd

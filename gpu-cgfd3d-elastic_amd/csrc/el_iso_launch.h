@@ -9,9 +9,10 @@ hipError_t launch_point(const StageArgs<TS, TC> &a, int dx, int dy, int dz, int 
 
 template <typename TS, typename TC> hipError_t launch_source(const SrcArgs<TS, TC> &a, hipStream_t st);
 
-template <typename TS, typename TC> hipError_t launch_recv(const RecvArgs<TS, TC> &a, hipStream_t st);
-
-hipError_t launch_clock_advance(int *clock, hipStream_t st);
+// receivers, source rates of the step (s.src_v set) and *clock_next = *clock + 1
+template <typename TS, typename TC>
+hipError_t launch_step_head(const RecvArgs<TS, TC> &r, const SrcArgs<TS, TC> &s, const int *clock, int *clock_next,
+                            hipStream_t st);
 
 // peak ground motion maps of every shot after one step (free surface only)
 template <typename TS, typename TC>
@@ -34,7 +35,7 @@ struct MarchSet {
   int nbox;
   int box[6][6];
   int zchunk;  // planes per workgroup along z
-  int shape;   // tile shape id, see interior_shape()
+  int shape;   // tile shape id, index into kTile
   int pml;     // the boxes reach into PML face boxes
 };
 
@@ -44,11 +45,26 @@ struct MarchGrid {
   int wg_beg[7];
 };
 
-int interior_num_shapes();
-void interior_shape(int id, int *tx, int *ty);
+// tile shapes the autotuner chooses from (TX x TY threads, one per column)
+constexpr int kNumShapes = 4;
+constexpr int kTile[kNumShapes][2] = {{64, 4}, {32, 8}, {64, 8}, {32, 16}};
+// the bare right-hand side (one operator call, never timed) runs this shape only
+constexpr int kRhsShape = 1;
+
+template <typename TS, typename TC, int SHAPE>
+hipError_t launch_interior_shape(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz, int nshots,
+                                 hipStream_t st);
 
 template <typename TS, typename TC>
 hipError_t launch_interior(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz, int nshots,
-                           hipStream_t st);
+                           hipStream_t st) {
+  if (b.nbox < 1) return hipSuccess;
+  switch (b.shape) {
+    case 0: return launch_interior_shape<TS, TC, 0>(a, b, dx, dy, dz, nshots, st);
+    case 1: return launch_interior_shape<TS, TC, 1>(a, b, dx, dy, dz, nshots, st);
+    case 2: return launch_interior_shape<TS, TC, 2>(a, b, dx, dy, dz, nshots, st);
+    default: return launch_interior_shape<TS, TC, 3>(a, b, dx, dy, dz, nshots, st);
+  }
+}
 
 }  // namespace cgfd

@@ -15,6 +15,19 @@
 
 namespace cgfd {
 
+// Source rates at a point of the shot's box (see StageArgs::sbox) join its
+// right-hand side.
+template <typename TS, typename TC>
+__device__ __forceinline__ void src_add(const StageArgs<TS, TC> &a, int shot, int i, int j, int k, TC *h) {
+#pragma clang fp contract(off)
+  const SrcBox b = a.sbox[shot];
+  const int di = i - b.i0, dj = j - b.j0, dk = k - b.k0;
+  if ((unsigned)di >= (unsigned)b.ni || (unsigned)dj >= (unsigned)b.nj || (unsigned)dk >= (unsigned)b.nk) return;
+  const TC *v = a.src_v + (long)shot * (4 * kNC) * a.src_vol + ((dk * b.nj + dj) * b.ni + di);
+#pragma unroll
+  for (int c = 0; c < kNC; c++) h[c] += v[c * a.src_vol];
+}
+
 // One face fi (its box must contain the point): Dd are the raw derivatives
 // along the face's axis and e1..e3 the matching metric row; MODE is the RK
 // mode (compile-time: each mode's loads are unconditional).
@@ -94,11 +107,12 @@ __device__ __forceinline__ void pml_face(const StageArgs<TS, TC> &a, int fi, int
     } else if constexpr (MODE == MODE_S12) {
       St<TS>::st(&at_b(F.a_out + fso, qb), (pre_a[c] + a.ca * Ph[c]) * is);
     } else if constexpr (MODE == MODE_S1Q) {
-      const TC d2 = a.ca * Ph[c];
-      St<TS>::st(&at_b(F.a_out + fso, qb), (pre_a[c] + d2) * is);
-      St<TS>::st(&at_b(F.a_end + fso, qb), rk_sum(a.rk_w, pre_a[c], P[c], d2) * is);
+      TC u2, q;
+      rk_sum(a.rk_w, pre_a[c], P[c], a.ca, Ph[c], u2, q);
+      St<TS>::st(&at_b(F.a_out + fso, qb), u2 * is);
+      St<TS>::st(&at_b(F.a_end + fso, qb), q * is);
     } else if constexpr (MODE == MODE_S3Q) {
-      St<TS>::st(&at_b(F.a_end + fso, qb), rk_end(a.rk_w, pre_a[c], P[c], a.cb * Ph[c]) * is);
+      St<TS>::st(&at_b(F.a_end + fso, qb), rk_end(a.rk_w, pre_a[c], P[c], a.cb, Ph[c]) * is);
     } else {
       const TC part = rk_partial(a.rk_w, pre_a[c], u1_a[c], u2_a[c]);
       St<TS>::st(&at_b(F.a_end + fso, qb), rk_final(pre_a[c], part, a.rk_w[2], P[c], a.cb * Ph[c]) * is);
@@ -182,14 +196,15 @@ __device__ __forceinline__ void pml_face_march(const StageArgs<TS, TC> &a, int f
   } else if constexpr (MODE == MODE_S1Q) {
 #pragma unroll
     for (int c = 0; c < kNC; c++) {
-      const TC d2 = a.ca * Ph[c];
-      St<TS>::st(&at_b(pout, qb(c)), (pre[c] + d2) * IS(c));
-      St<TS>::st(&at_b(pend, qb(c)), rk_sum(a.rk_w, pre[c], P[c], d2) * IS(c));
+      TC u2, q;
+      rk_sum(a.rk_w, pre[c], P[c], a.ca, Ph[c], u2, q);
+      St<TS>::st(&at_b(pout, qb(c)), u2 * IS(c));
+      St<TS>::st(&at_b(pend, qb(c)), q * IS(c));
     }
   } else if constexpr (MODE == MODE_S3Q) {
 #pragma unroll
     for (int c = 0; c < kNC; c++)
-      St<TS>::st(&at_b(pend, qb(c)), rk_end(a.rk_w, pre[c], P[c], a.cb * Ph[c]) * IS(c));
+      St<TS>::st(&at_b(pend, qb(c)), rk_end(a.rk_w, pre[c], P[c], a.cb, Ph[c]) * IS(c));
   } else if constexpr (MODE == MODE_S0) {
 #pragma unroll
     for (int c = 0; c < kNC; c++) St<TS>::st(&at_b(pout, qb(c)), (P[c] + a.ca * Ph[c]) * IS(c));

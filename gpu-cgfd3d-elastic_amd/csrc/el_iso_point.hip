@@ -54,12 +54,13 @@ __device__ __forceinline__ void rk_store(const StageArgs<TS, TC> &a, long so, in
       St<TS>::st(&at_b(wout, qb), (pre + a.ca * h[c]) * is);
     } else if constexpr (MODE == MODE_S1Q) {
       const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc, u1 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
-      const TC d2 = a.ca * h[c];
-      St<TS>::st(&at_b(wout, qb), (pre + d2) * is);
-      St<TS>::st(&at_b(wend, qb), rk_sum(a.rk_w, pre, u1, d2) * is);
+      TC u2, q;
+      rk_sum(a.rk_w, pre, u1, a.ca, h[c], u2, q);
+      St<TS>::st(&at_b(wout, qb), u2 * is);
+      St<TS>::st(&at_b(wend, qb), q * is);
     } else if constexpr (MODE == MODE_S3Q) {
       const TC q = (TC)St<TS>::ld(&at_b(wend, qb)) * sc, u3 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
-      St<TS>::st(&at_b(wend, qb), rk_end(a.rk_w, q, u3, a.cb * h[c]) * is);
+      St<TS>::st(&at_b(wend, qb), rk_end(a.rk_w, q, u3, a.cb, h[c]) * is);
     } else {
       const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc;
       const TC u3 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
@@ -207,6 +208,8 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
   // ---- CFS-PML faces, in the reference's face order ----
   pml_apply<MODE, TS, TC>(a, shot, i, j, k, Dx, Dy, Dz, xix, xiy, xiz, etx, ety, etz, ztx, zty, ztz, lam, mu, lam2mu,
                           slw, h);
+  if constexpr (kBoxedSrc<TS> && MODE != MODE_RHS)
+    if (a.sbox) src_add<TS, TC>(a, shot, i, j, k, h);
 
   rk_store<MODE, TS, TC>(a, so, o, h);
 }
@@ -221,21 +224,13 @@ __global__ __launch_bounds__(256) void k_point(StageArgs<TS, TC> a) {
   point_update<DX, DY, DZ, MODE, TS, TC>(a, shot, i, j, k);
 }
 
-// ---- source injection (sv_curv_col_el_iso_rhs_src_gpu, sv_curv_col_el_gpu.cu:227-301) ----
-// One thread per distinct grid point; contributions of the shot's sources are
-// summed in source order and applied to the RK outputs of this stage.
+// ---- sources (sv_curv_col_el_iso_rhs_src_gpu, sv_curv_col_el_gpu.cu:227-301) ----
+// Rates (dU/dt) that the shot's sources give grid point p at stage istage of
+// step it, contributions summed in source order; false where none acts.
 template <typename TS, typename TC>
-__global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= a.npt) return;
-  const int shot = a.pt_shot[p];
-  if (a.only_shot >= 0 && shot != a.only_shot) return;
-  if (a.only_shot < 0 && !a.shot_active[shot]) return;
-  const int it = a.only_shot >= 0 ? a.fixed_it : *a.clock - a.shot_start[shot];
+__device__ __forceinline__ bool src_rate(const SrcArgs<TS, TC> &a, int p, int it, int istage, TC *v) {
   const long o = a.pt_off[p];
-  const long cs = a.L.cs;
-  const TC jac = a.met[JAC * cs + o], slw = a.med[2 * cs + o];
-  TC v[kNC];
+  const TC jac = a.met[JAC * a.L.cs + o], slw = a.med[2 * a.L.cs + o];
 #pragma unroll
   for (int c = 0; c < kNC; c++) v[c] = TC(0);
   bool any = false;
@@ -243,7 +238,7 @@ __global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
     const int s = a.ct_src[q];
     if (it < a.s_itb[s] || it > a.s_ite[s]) continue;
     any = true;
-    const long ist = a.s_tab[s] + (long)(it - a.s_itb[s]) * 4 + a.istage;
+    const long ist = a.s_tab[s] + (long)(it - a.s_itb[s]) * 4 + istage;
     const TC coef = a.ct_coef[q];
     if (a.s_kind[s] & 1) {
       const TC V = coef * slw / jac;
@@ -261,7 +256,32 @@ __global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
       v[TXY] += -a.M[5 * a.ntab + ist] * rjac;
     }
   }
-  if (!any) return;
+  return any;
+}
+
+// One thread per distinct grid point; the rates, from the step's table where
+// there is one (10.5 -> 6 us: the contributions are a chain of dependent
+// loads), are applied to the RK outputs of this stage.  Serves 16-bit storage,
+// the bare right-hand side and sources that spread too far for a box (see
+// k_step_head).
+template <typename TS, typename TC>
+__global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= a.npt) return;
+  const int shot = a.pt_shot[p];
+  if (a.only_shot >= 0 && shot != a.only_shot) return;
+  if (a.only_shot < 0 && !a.shot_active[shot]) return;
+  const int it = a.only_shot >= 0 ? a.fixed_it : *a.clock - a.shot_start[shot];
+  const long o = a.pt_off[p];
+  const long cs = a.L.cs;
+  TC v[kNC];
+  if (a.src_v) {
+    const TC *r = a.src_v + ((long)shot * 4 + a.istage) * kNC * a.src_vol + a.pt_cell[p];
+#pragma unroll
+    for (int c = 0; c < kNC; c++) v[c] = r[c * a.src_vol];
+  } else if (!src_rate(a, p, it, a.istage, v)) {
+    return;
+  }
   const long so = (long)shot * a.shot_stride;
 #pragma unroll
   for (int c = 0; c < kNC; c++) {
@@ -287,13 +307,12 @@ __global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
 // Corner 5 carries both (x1,y1,z2) and (x2,y1,z2) weights and corner 4 is
 // unused, as in the reference; with on-node receivers the quirk vanishes.
 template <typename TS, typename TC>
-__global__ __launch_bounds__(256) void k_recv(RecvArgs<TS, TC> a) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void record(const RecvArgs<TS, TC> &a, int t, int clock) {
   if (t >= a.nrec * kNC) return;
   const int r = t / kNC, c = t % kNC;
   const int shot = a.r_shot[r];
   if (a.shot_active && !a.shot_active[shot]) return;
-  const int it = *a.clock - a.shot_start[shot];
+  const int it = clock - a.shot_start[shot];
   if (it < 0 || it >= a.r_nt[r]) return;
   const TS *w = a.w_pre + (long)shot * a.shot_stride + c * a.cs;
   const long *ix = a.r_off + (long)r * 8;
@@ -309,11 +328,35 @@ __global__ __launch_bounds__(256) void k_recv(RecvArgs<TS, TC> a) {
   a.seismo[a.r_out[r] + (long)c * pitch + (a.ring > 0 ? it % a.ring : it)] = s;
 }
 
-#if !defined(CGFD_TYPE) || CGFD_TYPE == 0
-__global__ void k_clock_advance(int *clock) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *clock += 1;
+// ---- the head of a step ----
+// One launch before the four stages: receivers sample W^n (blocks below
+// recv_blocks), the source rates of all four stages are tabulated over each
+// shot's box (the blocks after), and the step number for the next step is
+// written to the other of two clocks, so no block reads a clock that another
+// block of the launch writes.  The work is a few thousand threads of dependent
+// loads: one launch instead of six (receivers, one source injection per stage,
+// clock), each of which took 5-10 us of latency and 3-7 us between launches;
+// per step on 64^3 343 -> 200 us with the small z chunks of the sweep.
+template <typename TS, typename TC>
+__global__ __launch_bounds__(256) void k_step_head(RecvArgs<TS, TC> r, SrcArgs<TS, TC> s, const int *clock,
+                                                   int *clock_next, int recv_blocks) {
+  const int now = *clock;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *clock_next = now + 1;
+  if ((int)blockIdx.x < recv_blocks) {
+    record(r, blockIdx.x * blockDim.x + threadIdx.x, now);
+    return;
+  }
+  const int t = (blockIdx.x - recv_blocks) * blockDim.x + threadIdx.x;
+  if (!s.src_v || t >= 4 * s.npt) return;
+  const int p = t >> 2, istage = t & 3;
+  const int shot = s.pt_shot[p];
+  if (!s.shot_active[shot]) return;
+  TC v[kNC];
+  src_rate(s, p, now - s.shot_start[shot], istage, v);
+  TC *out = s.src_v + ((long)shot * 4 + istage) * kNC * s.src_vol + s.pt_cell[p];
+#pragma unroll
+  for (int c = 0; c < kNC; c++) out[c * s.src_vol] = v[c];
 }
-#endif
 
 template <typename T> __global__ __launch_bounds__(256) void k_fill(T *p, long n, T v) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -433,18 +476,14 @@ template <typename TS, typename TC> hipError_t launch_source(const SrcArgs<TS, T
   return hipGetLastError();
 }
 
-template <typename TS, typename TC> hipError_t launch_recv(const RecvArgs<TS, TC> &a, hipStream_t st) {
-  if (a.nrec == 0) return hipSuccess;
-  hipLaunchKernelGGL((k_recv<TS, TC>), dim3((a.nrec * kNC + 255) / 256), dim3(256), 0, st, a);
+template <typename TS, typename TC>
+hipError_t launch_step_head(const RecvArgs<TS, TC> &r, const SrcArgs<TS, TC> &s, const int *clock, int *clock_next,
+                            hipStream_t st) {
+  const int rb = (r.nrec * kNC + 255) / 256, sb = s.src_v ? (4 * s.npt + 255) / 256 : 0;
+  hipLaunchKernelGGL((k_step_head<TS, TC>), dim3(rb + sb > 0 ? rb + sb : 1), dim3(256), 0, st, r, s, clock, clock_next,
+                     rb);
   return hipGetLastError();
 }
-
-#if !defined(CGFD_TYPE) || CGFD_TYPE == 0
-hipError_t launch_clock_advance(int *clock, hipStream_t st) {
-  hipLaunchKernelGGL(k_clock_advance, dim3(1), dim3(64), 0, st, clock);
-  return hipGetLastError();
-}
-#endif
 
 template <typename T> hipError_t launch_fill(T *p, long n, T v, hipStream_t st) {
   if (n <= 0) return hipSuccess;
@@ -461,7 +500,8 @@ template <typename T> hipError_t launch_fill(T *p, long n, T v, hipStream_t st) 
   template hipError_t launch_gather<TS, TC>(const TS *, const Layout &, int, int, int, int, int, int, int, int,   \
                                             int, TC, TC *, hipStream_t);                                        \
   template hipError_t launch_source<TS, TC>(const SrcArgs<TS, TC> &, hipStream_t);                          \
-  template hipError_t launch_recv<TS, TC>(const RecvArgs<TS, TC> &, hipStream_t);
+  template hipError_t launch_step_head<TS, TC>(const RecvArgs<TS, TC> &, const SrcArgs<TS, TC> &, const int *, \
+                                               int *, hipStream_t);
 // CGFD_TYPE selects one storage type per object so the four compile in
 // parallel; without it every type is instantiated here.
 #if !defined(CGFD_TYPE) || CGFD_TYPE == 0
