@@ -205,6 +205,7 @@ struct cgfd_session {
   int tile_shape = -1, tile_zchunk = 48;
   bool tile_fixed = false;
   int split = -1;  // CGFD_SPLIT_*, chosen by the autotuner (-1: not yet: planes)
+  bool fuse = true;  // free-surface rows in the PML sweep's launch where its shape allows
   bool split_fixed = false;  // cgfd_set_split pinned it
   // timing
   bool timing = false;
@@ -736,8 +737,8 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
 
 // Work split of one stage.  CGFD_SPLIT_PLANES: the z-marching kernel sweeps
 // whole x-y planes from the bottom up to the last plane below the
-// free-surface rows, applying the CFS-PML terms inside the face boxes, and one
-// per-point launch takes the 4 free-surface rows.  CGFD_SPLIT_CORE: the same
+// free-surface rows, applying the CFS-PML terms inside the face boxes.
+// CGFD_SPLIT_CORE: the same
 // planes in two sweeps, the PML-free form over a core box inside every face
 // box whose x extent starts and ends on tile boundaries (so its rows load
 // whole 128-byte lines), and the PML form over the up to six rim boxes around
@@ -745,8 +746,13 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
 // / 164 VGPRs against 160 / 168 / 212 in S0 / S1-S2 / S3), so more waves
 // hide its latency.  CGFD_SPLIT_SHELL (or CGFD_FLAG_PML_POINT): the sweep
 // keeps to the box inside every face box and the per-point launch takes the
-// whole shell (face slabs and surface rows); the per-point launch also
-// covers everything for tiny grids or the plain method.  (Splitting that
+// whole shell (face slabs and surface rows: a launch of their own gained
+// nothing next to the slabs, 183 against 162 + 26 us on 211x187x121 bfloat16).
+// In the other splits the 4 free-surface rows go to k_surface, or ride with the
+// PML sweep's launch where that is faster (small grids: one launch gap and one
+// tail less); with 16-bit storage to the per-point kernel, whose summation order
+// their stored roundings follow.  The per-point launch covers everything for
+// tiny grids or the plain method.  (Splitting that
 // shell into per-axis single-face launches measured slower: the x slabs are
 // only nlay+1 points wide, and four launches add four tails.)
 struct BoxList {
@@ -765,7 +771,8 @@ struct BoxList {
 struct Shell {
   MarchSet inner;  // PML-free sweep (core or shell split) or the whole-plane sweep
   MarchSet rim;    // core split: PML-form sweep of the boxes around the core
-  BoxList point;
+  BoxList point;   // shell split: slabs and surface rows; plain method: everything
+  bool surface;    // the free-surface rows go to k_surface
 };
 
 // z chunk of the rim sweep: a third of the core's, at least 4 planes.  The
@@ -775,7 +782,7 @@ struct Shell {
 // faster than with the core's chunk, and 5 % / 7 % faster than with twice it.
 int rim_zchunk(int core_zchunk) { return std::max(4, core_zchunk / 3); }
 
-Shell make_shell(cgfd_session *s, int shape = -1) {
+Shell make_shell(cgfd_session *s, bool rhs = false) {
   Shell sh{};
   const int ni = s->d.ni, nj = s->d.nj, nk = s->d.nk;
   auto lay = [&](int f) { return s->face[f].on ? s->face[f].nlay + 1 : 0; };
@@ -796,10 +803,17 @@ Shell make_shell(cgfd_session *s, int shape = -1) {
     return sh;
   }
   sh.inner.zchunk = s->tile_zchunk;
-  sh.inner.shape = shape >= 0 ? shape : s->tile_shape < 0 ? 0 : s->tile_shape;
+  sh.inner.shape = rhs ? kRhsShape : s->tile_shape < 0 ? 0 : s->tile_shape;
   sh.rim.zchunk = rim_zchunk(sh.inner.zchunk);
   sh.rim.shape = sh.inner.shape;
   sh.rim.pml = 1;
+  // who takes the surface rows next to a whole-plane sweep
+  const bool tiles = s->es >= 4;
+  const bool fuse = s->free_top && tiles && s->fuse && !rhs && sh.inner.shape == kSurfShape;
+  auto surface_rows = [&]() {
+    sh.surface = s->free_top && tiles;
+    if (!tiles) sh.point.add(0, ni - 1, 0, nj - 1, ktopm + 1, nk - 1);
+  };
   const bool any_face = ib0 > 0 || ib1 < ni - 1 || jb0 > 0 || jb1 < nj - 1 || kb0 > 0 || kb1 < ktopm;
   if (any_face && !(s->d.flags & CGFD_FLAG_PML_POINT) && s->split != CGFD_SPLIT_SHELL) {
     if (s->split == CGFD_SPLIT_CORE) {
@@ -816,13 +830,15 @@ Shell make_shell(cgfd_session *s, int shape = -1) {
         addm(sh.rim, ca1 + 1, ni - 1, cb0, cb1, 0, ktopm);      // x2 side
         addm(sh.rim, ca0, ca1, cb0, cb1, 0, kb0 - 1);           // below the core
         addm(sh.rim, ca0, ca1, cb0, cb1, kb1 + 1, ktopm);       // above it (no free surface)
-        sh.point.add(0, ni - 1, 0, nj - 1, ktopm + 1, nk - 1);
+        sh.rim.surface = fuse && sh.rim.nbox > 0;
+        surface_rows();
         return sh;
       }
     }
     sh.inner.pml = 1;
     addm(sh.inner, 0, ni - 1, 0, nj - 1, 0, ktopm);
-    sh.point.add(0, ni - 1, 0, nj - 1, ktopm + 1, nk - 1);
+    sh.inner.surface = fuse;
+    surface_rows();
     return sh;
   }
   addm(sh.inner, ib0, ib1, jb0, jb1, kb0, kb1);
@@ -843,17 +859,20 @@ template <typename TS, typename TC> void set_boxes(StageArgs<TS, TC> &a, const B
   }
 }
 
-// one stage over the whole grid: z-marching sweep (timed when requested), then
-// the per-point boxes
+// one stage over the whole grid: z-marching sweeps (timed when requested, then
+// without the surface rows), the per-point boxes and the free-surface rows
 template <typename TS, typename TC>
 int launch_stage(cgfd_session *s, const Shell &sh, StageArgs<TS, TC> &a, int dx, int dy, int dz, int nshots,
                  hipEvent_t ev0, hipEvent_t ev1) {
-  if (sh.inner.nbox) {
+  MarchSet inner = sh.inner, rim = sh.rim;
+  if (ev0) inner.surface = rim.surface = 0;
+  const bool fused = inner.surface || rim.surface;
+  if (inner.nbox) {
     if (ev0) HIPCHK(hipEventRecord(ev0, s->st));
-    hipError_t e = launch_interior<TS, TC>(a, sh.inner, dx, dy, dz, nshots, s->st);
+    hipError_t e = launch_interior<TS, TC>(a, inner, dx, dy, dz, nshots, s->st);
     if (e != hipSuccess) return fail(CGFD_E_HIP, "interior kernel: %s", hipGetErrorString(e));
-    if (sh.rim.nbox) {
-      e = launch_interior<TS, TC>(a, sh.rim, dx, dy, dz, nshots, s->st);
+    if (rim.nbox) {
+      e = launch_interior<TS, TC>(a, rim, dx, dy, dz, nshots, s->st);
       if (e != hipSuccess) return fail(CGFD_E_HIP, "rim kernel: %s", hipGetErrorString(e));
     }
     if (ev1) HIPCHK(hipEventRecord(ev1, s->st));
@@ -863,18 +882,21 @@ int launch_stage(cgfd_session *s, const Shell &sh, StageArgs<TS, TC> &a, int dx,
     hipError_t e = launch_point<TS, TC>(a, dx, dy, dz, nshots, s->st);
     if (e != hipSuccess) return fail(CGFD_E_HIP, "point kernel: %s", hipGetErrorString(e));
   }
+  if (sh.surface && !fused) {
+    hipError_t e = launch_surface<TS, TC>(a, dx, dy, dz, nshots, s->st);
+    if (e != hipSuccess) return fail(CGFD_E_HIP, "surface kernel: %s", hipGetErrorString(e));
+  }
   return CGFD_OK;
 }
 
-// Tile autotuner: per (shape, z chunk), time the interior sweeps of one full
-// step's stage sequence (stage_plan, with the operator directions of
-// pair 0) and keep the fastest; the stages differ in traffic (30 to 57 words
+// Tile autotuner: per (work split, shape, z chunk, surface rows fused or not),
+// time one full step's stage sequence (stage_plan, with the operator directions
+// of pair 0) and keep the fastest; the stages differ in traffic (30 to 57 words
 // per cell), so tuning on one mode alone can pick a tile that loses on the
 // others.  Every level the sweeps write (slots 1..3) is rewritten by the next
-// step before it is read, so tuning between steps leaves the state intact.  Each work split (core,
-// whole planes, shell) is timed with its best tile and the fastest pair is
-// kept.  Results are cached per (grid, storage, shots, flags, metric form,
-// PML layout, pinned split) for the life of the process.
+// step before it is read, so tuning between steps leaves the state intact.
+// Results are cached per (grid, storage, shots, flags, metric form, PML layout,
+// pinned split) for the life of the process.
 struct TileKey {
   int ni, nj, nk, storage, nshots, flags, met_const, free_top;
   std::array<int, 6> nlay;  // PML layers per face (0: none)
@@ -886,6 +908,7 @@ struct TileKey {
 };
 struct TileChoice {
   int shape, zchunk, split;
+  bool fuse;
 };
 // shared by every session of the process; sessions may tune on several
 // threads at once (the shot server's worker and callers of their own)
@@ -913,6 +936,7 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
       s->tile_shape = hit->second.shape;
       s->tile_zchunk = hit->second.zchunk;
       s->split = hit->second.split;
+      s->fuse = hit->second.fuse;
       return CGFD_OK;
     }
   }
@@ -926,7 +950,7 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   const Shell planes = make_shell(s);
   if (!planes.inner.nbox) {  // no sweep at all (plain method, tiny grid)
     if (pinned >= 0) s->split = pinned;
-    remember({s->tile_shape, s->tile_zchunk, s->split});
+    remember({s->tile_shape, s->tile_zchunk, s->split, s->fuse});
     return CGFD_OK;
   }
   StageArgs<TS, TC> sa[4];
@@ -945,15 +969,17 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
-  // minimum over reps 1..2 of one full step's four stages of `launch`
-  auto timed = [&](auto launch, float &tmin) -> int {
+  // minimum over reps 1..2 of one full step's four stages under the session's
+  // present choice
+  auto timed = [&](float &tmin) -> int {
+    const Shell sh = make_shell(s);
     tmin = 1e30f;
     for (int rep = 0; rep < 3; rep++) {
       HIPCHK(hipEventRecord(e0, s->st));
       for (int q = 0; q < 4; q++) {
         const int d = (kFlags[0][0] + q) % 2;
-        hipError_t e = launch(q, d);
-        if (e != hipSuccess) return fail(CGFD_E_HIP, "autotune launch: %s", hipGetErrorString(e));
+        int r = launch_stage<TS, TC>(s, sh, sa[q], d, d, d, s->d.nshots, nullptr, nullptr);
+        if (r) return r;
       }
       HIPCHK(hipEventRecord(e1, s->st));
       HIPCHK(hipEventSynchronize(e1));
@@ -965,78 +991,57 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   };
   // Work splits: whole-plane sweep (PML terms inside) and, when the grid has
   // PML faces, the PML-free core with the PML-form rim, and the sweep inside
-  // the face boxes with the per-point kernel on the slabs.  Each is timed
-  // with its best tile plus its per-point launch (a pinned split alone).
+  // the face boxes with the per-point kernel on the slabs (a pinned split
+  // alone).
   const bool faces = planes.inner.pml && !(s->d.flags & CGFD_FLAG_PML_POINT);
   std::vector<int> splits;
   if (pinned >= 0) splits.push_back(faces ? pinned : CGFD_SPLIT_PLANES);
   else if (faces) splits = {CGFD_SPLIT_CORE, CGFD_SPLIT_PLANES, CGFD_SPLIT_SHELL};
   else splits = {CGFD_SPLIT_PLANES};
-  float best_total = 1e30f;
+  float best = 1e30f;
   int bs = 0, bz = 24, bsplit = splits[0];
+  bool bfuse = false;
   for (int split : splits) {
     s->split = split;
-    s->tile_shape = 0;
-    const Shell sh = make_shell(s);
-    const int nz = sh.inner.box[0][5] - sh.inner.box[0][4] + 1;
-    // z chunks near 16..48 planes that split the swept planes evenly: every
-    // chunk re-reads 4 planes below it, so a short last chunk costs almost a
-    // full one (196 planes: 17, 20, 25, 28, 33, 49 instead of 16 .. 48,
-    // whose last chunk has 4 planes).  Chunks of 4..12 planes are for sweeps
-    // that 16-plane chunks would leave with fewer than 2048 workgroups (8 per
-    // CU): there the idle CUs cost more than the planes read twice (64^3: 40
-    // workgroups of 17 planes, 38 us a sweep).  With 16-bit storage they would
-    // also move small grids from one split to another, whose roundings differ.
-    constexpr int kNZ = 12;
-    const int ztarget[kNZ] = {4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
-    int zcands[kNZ];
-    for (int zi = 0; zi < kNZ; zi++) {
-      const int n = std::max(1, (nz + ztarget[zi] / 2) / ztarget[zi]);
-      zcands[zi] = (nz + n - 1) / n;
-    }
-    float best = 1e30f;
-    int ts = 0, tz = 24;
     for (int shape = 0; shape < kNumShapes; shape++) {
       s->tile_shape = shape;
-      const Shell shs = make_shell(s);  // the core's bounds follow the tile shape
-      for (int zi = 0; zi < kNZ; zi++) {
-        const int zc = zcands[zi];
-        if (zi > 0 && zc == zcands[zi - 1]) continue;
-        if (ztarget[zi] < 16 && (St<TS>::scaled || march_workgroups(shs.inner, 16) * s->d.nshots >= 2048)) continue;
-        MarchSet ib = shs.inner, rb = shs.rim;
-        ib.zchunk = zc;
-        rb.zchunk = rim_zchunk(zc);
-        float t;
-        int r = timed(
-            [&](int q, int d) {
-              hipError_t e = launch_interior<TS, TC>(sa[q], ib, d, d, d, s->d.nshots, s->st);
-              if (e == hipSuccess && rb.nbox) e = launch_interior<TS, TC>(sa[q], rb, d, d, d, s->d.nshots, s->st);
-              return e;
-            },
-            t);
-        if (r) return r;
-        if (t < best) { best = t; ts = shape; tz = zc; }
+      s->fuse = true;
+      const Shell sh = make_shell(s);  // the core's bounds follow the tile shape
+      const int nz = sh.inner.box[0][5] - sh.inner.box[0][4] + 1;
+      // z chunks near 16..48 planes that split the swept planes evenly: every
+      // chunk re-reads 4 planes below it, so a short last chunk costs almost a
+      // full one (196 planes: 17, 20, 25, 28, 33, 49 instead of 16 .. 48,
+      // whose last chunk has 4 planes).  Chunks of 4..12 planes are for sweeps
+      // that 16-plane chunks would leave with fewer than 2048 workgroups (8 per
+      // CU): there the idle CUs cost more than the planes read twice (64^3: 40
+      // workgroups of 17 planes, 38 us a sweep).  With 16-bit storage they would
+      // also move small grids from one split to another, whose roundings differ.
+      constexpr int kNZ = 12;
+      const int ztarget[kNZ] = {4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
+      int last = 0;
+      for (int target : ztarget) {
+        if (target < 16 && (St<TS>::scaled || march_workgroups(sh.inner, 16) * s->d.nshots >= 2048)) continue;
+        const int n = std::max(1, (nz + target / 2) / target), zc = (nz + n - 1) / n;
+        if (zc == last) continue;
+        last = zc;
+        s->tile_zchunk = zc;
+        for (int fuse = 0; fuse <= (sh.inner.surface || sh.rim.surface ? 1 : 0); fuse++) {
+          s->fuse = fuse != 0;
+          float t;
+          int r = timed(t);
+          if (r) return r;
+          if (t < best) { best = t; bs = shape; bz = zc; bsplit = split; bfuse = s->fuse; }
+        }
       }
     }
-    float tp = 0;
-    if (sh.point.n) {
-      int r = timed(
-          [&](int q, int d) {
-            StageArgs<TS, TC> pa = sa[q];
-            set_boxes(pa, sh.point);
-            return launch_point<TS, TC>(pa, d, d, d, s->d.nshots, s->st);
-          },
-          tp);
-      if (r) return r;
-    }
-    if (best + tp < best_total) { best_total = best + tp; bs = ts; bz = tz; bsplit = split; }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   s->tile_shape = bs;
   s->tile_zchunk = bz;
   s->split = bsplit;
-  remember({bs, bz, bsplit});
+  s->fuse = bfuse;
+  remember({bs, bz, bsplit, bfuse});
   invalidate(s);
   return CGFD_OK;
 }
@@ -1255,7 +1260,7 @@ template <typename TS, typename TC> int onestage_t(cgfd_session *s, int shot, in
   a.shot_active = nullptr;
   a.mode = MODE_RHS;
   a.ca = TC(0); a.cb = TC(0);
-  const Shell sh = make_shell(s, kRhsShape);
+  const Shell sh = make_shell(s, true);
   int r = launch_stage<TS, TC>(s, sh, a, dx, dy, dz, 1, nullptr, nullptr);
   if (r) return r;
   if (s->s_npt > 0) {

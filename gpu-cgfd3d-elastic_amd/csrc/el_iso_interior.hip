@@ -30,15 +30,14 @@
 // or two rows of one plane); only the tiles at the two x ends diverge.  The
 // interior variant (PML = false) sweeps a box outside every face box.
 // Points within 4 rows of a free surface go to the per-point kernel.
-#include "el_iso_device.h"
-#include "el_iso_launch.h"
-#include "el_iso_pml.h"
+#include "el_iso_point.h"
 
 #include <type_traits>
 
 namespace cgfd {
 
-template <int DX, int DY, int DZ, typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, int MODE>
+template <int DX, int DY, int DZ, typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, int MODE,
+          bool SURF>
 __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, MarchSet b, MarchGrid g) {
   constexpr int NT = TX * TY;
   constexpr int HXL = (DX == 0) ? 3 : 1;
@@ -58,18 +57,31 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
   constexpr int NPX = (kNC + XPC - 1) / XPC;            // x-halo passes
   constexpr int NPER = NPY + NPX;                       // halo loads per thread
   __shared__ TC lds[2][kNC][LH][LW];
+  static_assert(!SURF || (TX == kSurfX && TY == kSurfY && kSurfLds <= 2 * kNC * LH * LW), "surface tiles");
 
   // XCD-aware remap: consecutive hardware workgroup ids land on different
   // XCDs (round robin).  Each XCD takes a contiguous eighth of every shot's
   // tiles, shot after shot: halos of neighbouring tiles meet in its L2, and
   // any subset of active shots keeps all eight XCDs busy.  The grid holds
   // 8 x part x nshots workgroups; the few past a shot's last tile exit.
+  // SURF: the tiles of the free-surface rows follow, an eighth to each XCD too.
   const int per_shot = g.wg_beg[b.nbox];
   const int part = (per_shot + 7) / 8;
+  const int nsurf = SURF ? g.sntx * g.snty * 4 : 0, spart = (nsurf + 7) / 8;
   const int hw = blockIdx.x;
   const int xcd = hw % 8, m = hw / 8;
-  const int shot = m / part;
-  const int rw = xcd * part + (m - shot * part);
+  const int shot = m / (part + spart);
+  const int rm = m - shot * (part + spart);
+  if constexpr (SURF) {
+    if (rm >= part) {
+      const int q = xcd * spart + rm - part;
+      if (q >= nsurf || (a.shot_active && !a.shot_active[shot])) return;
+      surface_tile<DX, DY, DZ, MODE>(a, shot, q % g.sntx, q / g.sntx % g.snty, a.L.nk - 4 + q / (g.sntx * g.snty),
+                                     &lds[0][0][0][0]);
+      return;
+    }
+  }
+  const int rw = xcd * part + rm;
   if (rw >= per_shot) return;
   int bx = 0;
   while (bx < b.nbox - 1 && rw >= g.wg_beg[bx + 1]) bx++;
@@ -410,7 +422,7 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
 }
 
 // one RK mode's k_march for the operator directions sel = 4 dx + 2 dy + dz
-template <typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, int MODE>
+template <typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, int MODE, bool SURF>
 static void launch_march_m(const StageArgs<TS, TC> &a, const MarchSet &b, const MarchGrid &g, dim3 grid, dim3 block,
                            int sel, hipStream_t st) {
   // 16-bit storage, constant metric, PML form, 32x8 tile: S1/S2 compiled for
@@ -420,7 +432,7 @@ static void launch_march_m(const StageArgs<TS, TC> &a, const MarchSet &b, const 
   // slower or no faster there.
   constexpr int MB = (sizeof(TS) == 2 && CART && PML && MODE == MODE_S12 && TX == 32 && TY == 8) ? 3 : MINB;
 #define CGFD_L(X, Y, Z) \
-  hipLaunchKernelGGL((k_march<X, Y, Z, TS, TC, TX, TY, MB, CART, PML, MODE>), grid, block, 0, st, a, b, g)
+  hipLaunchKernelGGL((k_march<X, Y, Z, TS, TC, TX, TY, MB, CART, PML, MODE, SURF>), grid, block, 0, st, a, b, g)
   switch (sel) {
     case 0: CGFD_L(0, 0, 0); break;
     case 1: CGFD_L(0, 0, 1); break;
@@ -434,7 +446,7 @@ static void launch_march_m(const StageArgs<TS, TC> &a, const MarchSet &b, const 
 #undef CGFD_L
 }
 
-template <typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML>
+template <typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, bool SURF>
 static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz,
                                  int nshots, hipStream_t st) {
   MarchGrid g{};
@@ -447,12 +459,16 @@ static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, 
     acc += g.ntx[q] * g.nty[q] * g.nzc[q];
   }
   g.wg_beg[b.nbox] = acc;
-  const long nwg = 8L * ((acc + 7) / 8) * nshots;  // see the remap at the top of the kernel
+  if (SURF) {
+    g.sntx = (a.L.ni + kSurfX - 1) / kSurfX;
+    g.snty = (a.L.nj + kSurfY - 1) / kSurfY;
+  }
+  const long nwg = 8L * ((acc + 7) / 8 + (g.sntx * g.snty * 4 + 7) / 8) * nshots;  // see the remap in the kernel
   if (nwg == 0) return hipSuccess;
   dim3 grid((unsigned)nwg), block(TX * TY);
   const int sel = dx * 4 + dy * 2 + dz;
 #define CGFD_M(M) \
-  if (a.mode == M) launch_march_m<TS, TC, TX, TY, MINB, CART, PML, M>(a, b, g, grid, block, sel, st)
+  if (a.mode == M) launch_march_m<TS, TC, TX, TY, MINB, CART, PML, M, SURF>(a, b, g, grid, block, sel, st)
   if constexpr (St<TS>::scaled) {
     CGFD_M(MODE_S3);
   } else {
@@ -461,7 +477,7 @@ static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, 
   }
   CGFD_M(MODE_S0);
   CGFD_M(MODE_S12);
-  if constexpr (CGFD_SHAPE == kRhsShape) CGFD_M(MODE_RHS);
+  if constexpr (CGFD_SHAPE == kRhsShape && !SURF) CGFD_M(MODE_RHS);
 #undef CGFD_M
   return hipGetLastError();
 }
@@ -472,12 +488,16 @@ template <typename TS, typename TC, int SHAPE>
 hipError_t launch_interior_shape(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz, int nshots,
                                  hipStream_t st) {
   constexpr int TX = kTile[SHAPE][0], TY = kTile[SHAPE][1], MINB = TX * TY > 256 ? 1 : 2;
-  if (a.met_const) {
-    if (b.pml) return launch_march_t<TS, TC, TX, TY, MINB, true, true>(a, b, dx, dy, dz, nshots, st);
-    return launch_march_t<TS, TC, TX, TY, MINB, true, false>(a, b, dx, dy, dz, nshots, st);
-  }
-  if (b.pml) return launch_march_t<TS, TC, TX, TY, MINB, false, true>(a, b, dx, dy, dz, nshots, st);
-  return launch_march_t<TS, TC, TX, TY, MINB, false, false>(a, b, dx, dy, dz, nshots, st);
+  auto go = [&](auto cart, auto pml, auto surf) {
+    return launch_march_t<TS, TC, TX, TY, MINB, decltype(cart)::value, decltype(pml)::value, decltype(surf)::value>(
+        a, b, dx, dy, dz, nshots, st);
+  };
+  using T = std::true_type;
+  using F = std::false_type;
+  if constexpr (SHAPE == kSurfShape && !St<TS>::scaled)
+    if (b.pml && b.surface) return a.met_const ? go(T{}, T{}, T{}) : go(F{}, T{}, T{});
+  if (b.pml) return a.met_const ? go(T{}, T{}, F{}) : go(F{}, T{}, F{});
+  return a.met_const ? go(T{}, F{}, F{}) : go(F{}, F{}, F{});
 }
 
 #if CGFD_TYPE == 0

@@ -7,6 +7,10 @@ namespace cgfd {
 template <typename TS, typename TC>
 hipError_t launch_point(const StageArgs<TS, TC> &a, int dx, int dy, int dz, int nshots, hipStream_t st);
 
+// the 4 free-surface rows of the whole grid
+template <typename TS, typename TC>
+hipError_t launch_surface(const StageArgs<TS, TC> &a, int dx, int dy, int dz, int nshots, hipStream_t st);
+
 template <typename TS, typename TC> hipError_t launch_source(const SrcArgs<TS, TC> &a, hipStream_t st);
 
 // receivers, source rates of the step (s.src_v set) and *clock_next = *clock + 1
@@ -37,12 +41,14 @@ struct MarchSet {
   int zchunk;  // planes per workgroup along z
   int shape;   // tile shape id, index into kTile
   int pml;     // the boxes reach into PML face boxes
+  int surface; // the launch also updates the free-surface rows (see launch_interior)
 };
 
 // per-box tile counts, filled by the launcher for the chosen tile shape
 struct MarchGrid {
   int ntx[6], nty[6], nzc[6];
   int wg_beg[7];
+  int sntx, snty;  // tiles of a free-surface row (0: none)
 };
 
 // tile shapes the autotuner chooses from (TX x TY threads, one per column)
@@ -50,6 +56,9 @@ constexpr int kNumShapes = 4;
 constexpr int kTile[kNumShapes][2] = {{64, 4}, {32, 8}, {64, 8}, {32, 16}};
 // the bare right-hand side (one operator call, never timed) runs this shape only
 constexpr int kRhsShape = 1;
+// the shape whose PML sweep can take the free-surface rows into its launch (its
+// workgroup is that of a surface tile); not with 16-bit storage
+constexpr int kSurfShape = 1;
 
 template <typename TS, typename TC, int SHAPE>
 hipError_t launch_interior_shape(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz, int nshots,

@@ -5,9 +5,9 @@
 // traction-image / vlow forms on the free-surface rows), the CFS-PML ADE
 // corrections of every face box containing the point, then the fused RK
 // update of the wavefield and of the PML memory (stage-value form, see Mode
-// in el_iso_device.h).  It covers any list of boxes,
-// so it serves both as the boundary-shell kernel next to the z-marching
-// interior kernel and as the whole-domain kernel of the plain method.
+// in el_iso_device.h).  It covers any list of boxes: the PML slabs in the shell
+// split and the whole domain in the plain method.  Next to a sweep the
+// free-surface rows go to k_surface, the tile form of the same update.
 //
 // Semantics follow, in order, sv_curv_col_el_iso_rhs_inner_gpu
 // (src/forward/sv_curv_col_el_iso_gpu.cu:291-452),
@@ -16,59 +16,9 @@
 // sv_curv_col_el_iso_rhs_cfspml_gpu (sv_curv_col_el_iso_gpu.cu:680-1147) and the
 // RK axpys wav_update / wav_update_end (src/forward/wav_t.cu:362-378) as driven by
 // drv_rk_curv_col.cu:339-491.
-#include "el_iso_device.h"
-#include "el_iso_launch.h"
-#include "el_iso_pml.h"
+#include "el_iso_point.h"
 
 namespace cgfd {
-
-template <int DIR, typename TC, typename F>
-__device__ __forceinline__ TC drp5(F f, long s) {
-  constexpr int lo = Drp<TC, DIR>::lo;
-  return Drp<TC, DIR>::c(0) * f((lo + 0) * s) + Drp<TC, DIR>::c(1) * f((lo + 1) * s) +
-         Drp<TC, DIR>::c(2) * f((lo + 2) * s) + Drp<TC, DIR>::c(3) * f((lo + 3) * s) +
-         Drp<TC, DIR>::c(4) * f((lo + 4) * s);
-}
-
-// RK update of the wavefield at one point from its right-hand side h (MODE:
-// the RK mode, a compile-time constant, so each mode's loads are
-// unconditional and issue together)
-template <int MODE, typename TS, typename TC>
-__device__ __forceinline__ void rk_store(const StageArgs<TS, TC> &a, long so, int o, const TC *h) {
-  const long cs = a.L.cs;
-  const unsigned qb = (unsigned)o * (unsigned)sizeof(TS);
-#pragma unroll
-  for (int c = 0; c < kNC; c++) {
-    TS *wout = a.w_out + so + c * cs, *wend = a.w_end + so + c * cs;
-    const TS *wpre = a.w_pre + so + c * cs, *wu2 = a.w_u2 + so + c * cs;
-    const TS *win = a.w_in + so + c * cs;
-    const TC sc = St<TS>::scaled ? (TC)a.sc[c] : TC(1);
-    const TC is = St<TS>::scaled ? (TC)a.isc[c] : TC(1);
-    if constexpr (MODE == MODE_RHS) {
-      St<TS>::st(&at_b(wout, qb), h[c] * is);
-    } else if constexpr (MODE == MODE_S0) {
-      const TC v = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
-      St<TS>::st(&at_b(wout, qb), (v + a.ca * h[c]) * is);
-    } else if constexpr (MODE == MODE_S12) {
-      const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc;
-      St<TS>::st(&at_b(wout, qb), (pre + a.ca * h[c]) * is);
-    } else if constexpr (MODE == MODE_S1Q) {
-      const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc, u1 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
-      TC u2, q;
-      rk_sum(a.rk_w, pre, u1, a.ca, h[c], u2, q);
-      St<TS>::st(&at_b(wout, qb), u2 * is);
-      St<TS>::st(&at_b(wend, qb), q * is);
-    } else if constexpr (MODE == MODE_S3Q) {
-      const TC q = (TC)St<TS>::ld(&at_b(wend, qb)) * sc, u3 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
-      St<TS>::st(&at_b(wend, qb), rk_end(a.rk_w, q, u3, a.cb, h[c]) * is);
-    } else {
-      const TC pre = (TC)St<TS>::ld(&at_b(wpre, qb)) * sc;
-      const TC u3 = (TC)St<TS>::ld(&at_b(win, qb)) * sc;
-      const TC part = rk_partial(a.rk_w, pre, (TC)St<TS>::ld(&at_b(wend, qb)) * sc, (TC)St<TS>::ld(&at_b(wu2, qb)) * sc);
-      St<TS>::st(&at_b(wend, qb), rk_final(pre, part, a.rk_w[2], u3, a.cb * h[c]) * is);
-    }
-  }
-}
 
 // the point of a box list that global thread gid maps to; false past the end
 template <typename TS, typename TC>
@@ -85,134 +35,20 @@ __device__ __forceinline__ bool box_point(const StageArgs<TS, TC> &a, long gid, 
   return true;
 }
 
-template <int DX, int DY, int DZ, int MODE, typename TS, typename TC>
-__device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int shot, int i, int j, int k) {
-  const Layout &L = a.L;
-  // element offsets inside one component stay below 2^31: 32-bit offsets from
-  // uniform component bases let the compiler use scalar-base addressing
-  const int o = (int)L.off(i, j, k);
-  const long so = (long)shot * a.shot_stride;
-  const TS *win = a.w_in + so;
-  const long cs = L.cs;
-  auto W = [&](int c, long d) -> TC {
-    return (TC)St<TS>::ld(&at_b(win + c * cs, (unsigned)(o + (int)d) * (unsigned)sizeof(TS)));
-  };
-  auto S = [&](int c) -> TC { return St<TS>::scaled ? (TC)a.sc[c] : TC(1); };
-
-  TC Dx[kNC], Dy[kNC], Dz[kNC];
-#pragma unroll
-  for (int c = 0; c < kNC; c++) {
-    auto f = [&](long d) { return W(c, d); };
-    Dx[c] = drp5<DX, TC>(f, 1);
-    Dy[c] = drp5<DY, TC>(f, L.px);
-    Dz[c] = drp5<DZ, TC>(f, L.pz);
-    if (St<TS>::scaled) { Dx[c] *= S(c); Dy[c] *= S(c); Dz[c] *= S(c); }
+// derivatives straight from the level in memory
+template <int DX, int DY, typename TS, typename TC> struct MemAcc {
+  const StageArgs<TS, TC> &a;
+  const TS *win;
+  int o;
+  template <int AXIS> __device__ __forceinline__ TC d(std::integral_constant<int, AXIS>, int c) const {
+    auto f = [&](long n) -> TC {
+      return (TC)St<TS>::ld(&at_b(win + c * a.L.cs, (unsigned)(o + (int)n) * (unsigned)sizeof(TS)));
+    };
+    TC v = drp5<AXIS == 0 ? DX : DY, TC>(f, AXIS == 0 ? 1 : a.L.px);
+    if (St<TS>::scaled) v *= (TC)a.sc[c];
+    return v;
   }
-  const TC *met = a.met;
-  auto Mt = [&](int m, long d) -> TC {
-    return at_b(met + m * cs, (unsigned)(o + (int)d) * (unsigned)sizeof(TC));
-  };
-  const TC xix = Mt(XIX, 0), xiy = Mt(XIY, 0), xiz = Mt(XIZ, 0);
-  const TC etx = Mt(ETX, 0), ety = Mt(ETY, 0), etz = Mt(ETZ, 0);
-  const TC ztx = Mt(ZTX, 0), zty = Mt(ZTY, 0), ztz = Mt(ZTZ, 0);
-  const unsigned ob = (unsigned)o * (unsigned)sizeof(TC);
-  const TC lam = at_b(a.med, ob), mu = at_b(a.med + cs, ob), slw = at_b(a.med + 2 * cs, ob);
-  // lam + 2.0*mu: the double-promoted sum of the reference rounds to the same
-  // float as the float sum whenever lam and 2mu are within 2^29 of each other.
-  const TC lam2mu = lam + TC(2) * mu;
-
-  TC h[kNC];
-  const bool top = a.free_top != 0;
-  const int ktop = L.nk - 1;
-  constexpr int zlast = (DZ == 0) ? 1 : 3;
-  if (top && k >= ktop - zlast) {
-    // traction image: conservative form with the odd extension of J*zeta.T
-    constexpr int zlo = (DZ == 0) ? -3 : -1;
-    const int n_free = ktop - k - zlo;
-    const TC slwjac = slw / Mt(JAC, 0);
-    constexpr int T1[3] = {TXX, TXY, TXZ}, T2[3] = {TXY, TYY, TYZ}, T3[3] = {TXZ, TYZ, TZZ};
-#pragma unroll
-    for (int cc = 0; cc < 3; cc++) {
-      auto vec = [&](long d, int e1, int e2, int e3) -> TC {
-        return Mt(JAC, d) * (Mt(e1, d) * (W(T1[cc], d) * S(T1[cc])) + Mt(e2, d) * (W(T2[cc], d) * S(T2[cc])) +
-                             Mt(e3, d) * (W(T3[cc], d) * S(T3[cc])));
-      };
-      constexpr int xlo = (DX == 0) ? -3 : -1, ylo = (DY == 0) ? -3 : -1;
-      TC DxTx = TC(0), DyTy = TC(0), DzTz = TC(0);
-#pragma unroll
-      for (int n = 0; n < 5; n++) {
-        DxTx += Drp<TC, DX>::c(n) * vec((long)(xlo + n), XIX, XIY, XIZ);
-        DyTy += Drp<TC, DY>::c(n) * vec((long)(ylo + n) * L.px, ETX, ETY, ETZ);
-      }
-#pragma unroll
-      for (int n = 0; n < 5; n++) {
-        TC v;
-        if (n < n_free) v = vec((long)(zlo + n) * L.pz, ZTX, ZTY, ZTZ);
-        else if (n == n_free) v = TC(0);
-        else v = -vec((long)(zlo + n - 2 * (n - n_free)) * L.pz, ZTX, ZTY, ZTZ);
-        DzTz += Drp<TC, DZ>::c(n) * v;
-      }
-      h[VX + cc] = (DxTx + DyTy + DzTz) * slwjac;
-    }
-  } else {
-    h[VX] = slw * (xix * Dx[TXX] + xiy * Dx[TXY] + xiz * Dx[TXZ] + etx * Dy[TXX] + ety * Dy[TXY] + etz * Dy[TXZ] +
-                   ztx * Dz[TXX] + zty * Dz[TXY] + ztz * Dz[TXZ]);
-    h[VY] = slw * (xix * Dx[TXY] + xiy * Dx[TYY] + xiz * Dx[TYZ] + etx * Dy[TXY] + ety * Dy[TYY] + etz * Dy[TYZ] +
-                   ztx * Dz[TXY] + zty * Dz[TYY] + ztz * Dz[TYZ]);
-    h[VZ] = slw * (xix * Dx[TXZ] + xiy * Dx[TYZ] + xiz * Dx[TZZ] + etx * Dy[TXZ] + ety * Dy[TYZ] + etz * Dy[TZZ] +
-                   ztx * Dz[TXZ] + zty * Dz[TYZ] + ztz * Dz[TZZ]);
-  }
-
-  TC DzVx = Dz[VX], DzVy = Dz[VY], DzVz = Dz[VZ];
-  if (top && k >= ktop - 2) {
-    const int n = ktop - k;
-    if (n == 0) {
-      const long pl = (long)L.ni * L.nj, q = (long)j * L.ni + i;
-      const TC *A = a.mat + q, *B = a.mat + 9 * pl + q;
-      DzVx = A[0] * Dx[VX] + A[pl] * Dx[VY] + A[2 * pl] * Dx[VZ] + B[0] * Dy[VX] + B[pl] * Dy[VY] + B[2 * pl] * Dy[VZ];
-      DzVy = A[3 * pl] * Dx[VX] + A[4 * pl] * Dx[VY] + A[5 * pl] * Dx[VZ] + B[3 * pl] * Dy[VX] + B[4 * pl] * Dy[VY] +
-             B[5 * pl] * Dy[VZ];
-      DzVz = A[6 * pl] * Dx[VX] + A[7 * pl] * Dx[VY] + A[8 * pl] * Dx[VZ] + B[6 * pl] * Dy[VX] + B[7 * pl] * Dy[VY] +
-             B[8 * pl] * Dy[VZ];
-    } else if (n == 1) {
-      // 2nd-order op, layer 1 (fd_t.cu:82-85, 103-106)
-      const long z = L.pz;
-      if (DZ == 0) {
-        DzVx = -W(VX, -z) + W(VX, 0); DzVy = -W(VY, -z) + W(VY, 0); DzVz = -W(VZ, -z) + W(VZ, 0);
-      } else {
-        DzVx = -W(VX, 0) + W(VX, z); DzVy = -W(VY, 0) + W(VY, z); DzVz = -W(VZ, 0) + W(VZ, z);
-      }
-      DzVx *= S(VX); DzVy *= S(VY); DzVz *= S(VZ);
-    } else {
-      // 4th-order op, layer 2 (fd_t.cu:86-89, 107-110)
-      const long z = L.pz;
-      const TC c0 = (DZ == 0) ? TC(1.0 / 6.0) : TC(-7.0 / 6.0);
-      const TC c1 = (DZ == 0) ? TC(-8.0 / 6.0) : TC(8.0 / 6.0);
-      const TC c2 = (DZ == 0) ? TC(7.0 / 6.0) : TC(-1.0 / 6.0);
-      const long s0 = (DZ == 0) ? -2 * z : 0, s1 = (DZ == 0) ? -z : z, s2 = (DZ == 0) ? 0 : 2 * z;
-      DzVx = (c0 * W(VX, s0) + c1 * W(VX, s1) + c2 * W(VX, s2)) * S(VX);
-      DzVy = (c0 * W(VY, s0) + c1 * W(VY, s1) + c2 * W(VY, s2)) * S(VY);
-      DzVz = (c0 * W(VZ, s0) + c1 * W(VZ, s1) + c2 * W(VZ, s2)) * S(VZ);
-    }
-  }
-  h[TXX] = lam2mu * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx) +
-           lam * (xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy + xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz);
-  h[TYY] = lam2mu * (xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy) +
-           lam * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx + xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz);
-  h[TZZ] = lam2mu * (xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz) +
-           lam * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx + xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy);
-  h[TXY] = mu * (xiy * Dx[VX] + xix * Dx[VY] + ety * Dy[VX] + etx * Dy[VY] + zty * DzVx + ztx * DzVy);
-  h[TXZ] = mu * (xiz * Dx[VX] + xix * Dx[VZ] + etz * Dy[VX] + etx * Dy[VZ] + ztz * DzVx + ztx * DzVz);
-  h[TYZ] = mu * (xiz * Dx[VY] + xiy * Dx[VZ] + etz * Dy[VY] + ety * Dy[VZ] + ztz * DzVy + zty * DzVz);
-
-  // ---- CFS-PML faces, in the reference's face order ----
-  pml_apply<MODE, TS, TC>(a, shot, i, j, k, Dx, Dy, Dz, xix, xiy, xiz, etx, ety, etz, ztx, zty, ztz, lam, mu, lam2mu,
-                          slw, h);
-  if constexpr (kBoxedSrc<TS> && MODE != MODE_RHS)
-    if (a.sbox) src_add<TS, TC>(a, shot, i, j, k, h);
-
-  rk_store<MODE, TS, TC>(a, so, o, h);
-}
+};
 
 template <int DX, int DY, int DZ, int MODE, typename TS, typename TC>
 __global__ __launch_bounds__(256) void k_point(StageArgs<TS, TC> a) {
@@ -221,7 +57,20 @@ __global__ __launch_bounds__(256) void k_point(StageArgs<TS, TC> a) {
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
   int i, j, k;
   if (!box_point(a, gid, i, j, k)) return;
-  point_update<DX, DY, DZ, MODE, TS, TC>(a, shot, i, j, k);
+  const MemAcc<DX, DY, TS, TC> acc{a, a.w_in + (long)shot * a.shot_stride, (int)a.L.off(i, j, k)};
+  point_update<DX, DY, DZ, MODE, false>(a, shot, i, j, k, true, acc);
+}
+
+// The 4 free-surface rows (surface_tile); workgroups as in the sweep: each XCD
+// takes a contiguous eighth of a shot's tiles.
+template <int DX, int DY, int DZ, int MODE, typename TS, typename TC>
+__global__ __launch_bounds__(256, 2) void k_surface(StageArgs<TS, TC> a, int ntx, int nty) {
+  __shared__ TC lds[kSurfLds];
+  const int per_shot = ntx * nty * 4, part = (per_shot + 7) / 8;
+  const int xcd = blockIdx.x % 8, m = blockIdx.x / 8;
+  const int shot = m / part, q = xcd * part + (m - shot * part);
+  if (q >= per_shot || (a.shot_active && !a.shot_active[shot])) return;
+  surface_tile<DX, DY, DZ, MODE>(a, shot, q % ntx, q / ntx % nty, a.L.nk - 4 + q / (ntx * nty), lds);
 }
 
 // ---- sources (sv_curv_col_el_iso_rhs_src_gpu, sv_curv_col_el_gpu.cu:227-301) ----
@@ -434,22 +283,44 @@ hipError_t launch_gather(const TS *w, const Layout &L, int i1, int j1, int k1, i
   return hipGetLastError();
 }
 
-// one RK mode's k_point for the operator directions sel = 4 dx + 2 dy + dz
+// one RK mode's kernel for the operator directions sel = 4 dx + 2 dy + dz
+#define CGFD_DIRS(sel)            \
+  switch (sel) {                  \
+    case 0: CGFD_L(0, 0, 0); break; \
+    case 1: CGFD_L(0, 0, 1); break; \
+    case 2: CGFD_L(0, 1, 0); break; \
+    case 3: CGFD_L(0, 1, 1); break; \
+    case 4: CGFD_L(1, 0, 0); break; \
+    case 5: CGFD_L(1, 0, 1); break; \
+    case 6: CGFD_L(1, 1, 0); break; \
+    default: CGFD_L(1, 1, 1); break; \
+  }
 template <int MODE, typename TS, typename TC>
 static void launch_point_m(const StageArgs<TS, TC> &a, dim3 grid, int sel, hipStream_t st) {
   const dim3 block(256);
 #define CGFD_L(X, Y, Z) hipLaunchKernelGGL((k_point<X, Y, Z, MODE, TS, TC>), grid, block, 0, st, a)
-  switch (sel) {
-    case 0: CGFD_L(0, 0, 0); break;
-    case 1: CGFD_L(0, 0, 1); break;
-    case 2: CGFD_L(0, 1, 0); break;
-    case 3: CGFD_L(0, 1, 1); break;
-    case 4: CGFD_L(1, 0, 0); break;
-    case 5: CGFD_L(1, 0, 1); break;
-    case 6: CGFD_L(1, 1, 0); break;
-    default: CGFD_L(1, 1, 1); break;
-  }
+  CGFD_DIRS(sel)
 #undef CGFD_L
+}
+template <int MODE, typename TS, typename TC>
+static void launch_surface_m(const StageArgs<TS, TC> &a, dim3 grid, int ntx, int nty, int sel, hipStream_t st) {
+  const dim3 block(kSurfX * kSurfY);
+#define CGFD_L(X, Y, Z) hipLaunchKernelGGL((k_surface<X, Y, Z, MODE, TS, TC>), grid, block, 0, st, a, ntx, nty)
+  CGFD_DIRS(sel)
+#undef CGFD_L
+}
+
+// calls f with the RK mode as a compile-time constant (the modes this storage uses)
+template <typename TS, typename F> static void with_mode(int mode, F f) {
+  if constexpr (St<TS>::scaled) {
+    if (mode == MODE_S3) f(std::integral_constant<int, MODE_S3>{});
+  } else {
+    if (mode == MODE_S1Q) f(std::integral_constant<int, MODE_S1Q>{});
+    if (mode == MODE_S3Q) f(std::integral_constant<int, MODE_S3Q>{});
+  }
+  if (mode == MODE_S0) f(std::integral_constant<int, MODE_S0>{});
+  if (mode == MODE_S12) f(std::integral_constant<int, MODE_S12>{});
+  if (mode == MODE_RHS) f(std::integral_constant<int, MODE_RHS>{});
 }
 
 template <typename TS, typename TC>
@@ -457,16 +328,18 @@ hipError_t launch_point(const StageArgs<TS, TC> &a, int dx, int dy, int dz, int 
   const long n = a.nbox ? a.box_end[a.nbox - 1] : 0;
   if (n == 0) return hipSuccess;
   const dim3 grid((unsigned)((n + 255) / 256), (unsigned)nshots);
-  const int sel = dx * 4 + dy * 2 + dz;
-  if constexpr (St<TS>::scaled) {
-    if (a.mode == MODE_S3) launch_point_m<MODE_S3>(a, grid, sel, st);
-  } else {
-    if (a.mode == MODE_S1Q) launch_point_m<MODE_S1Q>(a, grid, sel, st);
-    if (a.mode == MODE_S3Q) launch_point_m<MODE_S3Q>(a, grid, sel, st);
-  }
-  if (a.mode == MODE_S0) launch_point_m<MODE_S0>(a, grid, sel, st);
-  if (a.mode == MODE_S12) launch_point_m<MODE_S12>(a, grid, sel, st);
-  if (a.mode == MODE_RHS) launch_point_m<MODE_RHS>(a, grid, sel, st);
+  with_mode<TS>(a.mode, [&](auto m) { launch_point_m<decltype(m)::value>(a, grid, dx * 4 + dy * 2 + dz, st); });
+  return hipGetLastError();
+}
+
+template <typename TS, typename TC>
+hipError_t launch_surface(const StageArgs<TS, TC> &a, int dx, int dy, int dz, int nshots, hipStream_t st) {
+  if constexpr (St<TS>::scaled) return hipErrorInvalidValue;  // its surface rows go to k_point
+  const int ntx = (a.L.ni + kSurfX - 1) / kSurfX, nty = (a.L.nj + kSurfY - 1) / kSurfY;
+  const dim3 grid((unsigned)(8L * ((ntx * nty * 4 + 7) / 8) * nshots));
+  if constexpr (!St<TS>::scaled)
+    with_mode<TS>(a.mode,
+                  [&](auto m) { launch_surface_m<decltype(m)::value>(a, grid, ntx, nty, dx * 4 + dy * 2 + dz, st); });
   return hipGetLastError();
 }
 
@@ -495,6 +368,7 @@ template <typename T> hipError_t launch_fill(T *p, long n, T v, hipStream_t st) 
 
 #define CGFD_INST(TS, TC)                                                                                   \
   template hipError_t launch_point<TS, TC>(const StageArgs<TS, TC> &, int, int, int, int, hipStream_t);    \
+  template hipError_t launch_surface<TS, TC>(const StageArgs<TS, TC> &, int, int, int, int, hipStream_t);  \
   template hipError_t launch_peak<TS, TC>(const TS *, const TS *, long, const Layout &, TC *, TC, const float *, \
                                           const int *, int, hipStream_t);                                      \
   template hipError_t launch_gather<TS, TC>(const TS *, const Layout &, int, int, int, int, int, int, int, int,   \

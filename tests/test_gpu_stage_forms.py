@@ -60,3 +60,22 @@ def test_sources_in_every_split(split, where, storage):
     assert rel_l2(seis, so) <= TOL[storage]
     for c in range(9):
         assert rel_l2(wave[c], wo[c]) <= TOL[storage], c
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+@pytest.mark.parametrize("shape", [0, 1], ids=["own-launch", "with-sweep"])
+@pytest.mark.parametrize("ni,nj", [(32, 24), (33, 25), (31, 40), (65, 23)])
+def test_surface_rows_at_tile_edges(ni, nj, shape, storage):
+    P = Problem(ni=ni, nj=nj, nk=24, curvilinear=True, hetero=0.05, seed=9, nt_total=9, init_random=True,
+                pml=(4, 4, 4, 4, 4, 0))
+    f = np.float64 if storage == "f64" else np.float32
+    s = cgfd.Session(P.ni, P.nj, P.nk, storage=STORE[storage])
+    P.upload(s, dtype=f)
+    s.set_tile(shape, 8)
+    s.run(0, P.nt_total, P.dt)
+    wave = s.fetch_level(0, cgfd.LEVEL_PRE)
+    s.close()
+    _, wo, _ = P.oracle_run(64 if storage == "f64" else 32)
+    for c in range(9):
+        assert rel_l2(wave[c], wo[c]) <= TOL[storage], c
+        assert rel_l2(wave[c][-7:-3], wo[c][-7:-3]) <= TOL[storage], c
