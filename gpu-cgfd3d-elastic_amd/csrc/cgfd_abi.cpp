@@ -152,7 +152,7 @@ struct cgfd_session {
   void *rhs = nullptr;     // nshots x 1 level (lazy)
   void *met = nullptr, *med = nullptr, *mat = nullptr;
   bool have_met = false, have_med = false;
-  bool met_const = false;  // all metric components constant (Cartesian grid)
+  int met_class = MET_ALL;  // MetClass of the uploaded metric
   double cmet[9] = {0};
   int free_top = 0;
   FaceHost face[6];
@@ -695,7 +695,7 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
   a.med = (const TC *)s->med;
   a.mat = (const TC *)s->mat;
   a.free_top = s->free_top;
-  a.met_const = s->met_const ? 1 : 0;
+  a.met_class = s->met_class;
   for (int c = 0; c < 9; c++) a.cmet[c] = (TC)s->cmet[c];
   const long aux_lvl_shot = 5;
   for (int f = 0; f < 6; f++) {
@@ -898,12 +898,12 @@ int launch_stage(cgfd_session *s, const Shell &sh, StageArgs<TS, TC> &a, int dx,
 // Results are cached per (grid, storage, shots, flags, metric form, PML layout,
 // pinned split) for the life of the process.
 struct TileKey {
-  int ni, nj, nk, storage, nshots, flags, met_const, free_top;
+  int ni, nj, nk, storage, nshots, flags, met_class, free_top;
   std::array<int, 6> nlay;  // PML layers per face (0: none)
   int pinned;               // split pinned by cgfd_set_split, -1: automatic
   bool operator<(const TileKey &o) const {
-    return std::tie(ni, nj, nk, storage, nshots, flags, met_const, free_top, nlay, pinned) <
-           std::tie(o.ni, o.nj, o.nk, o.storage, o.nshots, o.flags, o.met_const, o.free_top, o.nlay, o.pinned);
+    return std::tie(ni, nj, nk, storage, nshots, flags, met_class, free_top, nlay, pinned) <
+           std::tie(o.ni, o.nj, o.nk, o.storage, o.nshots, o.flags, o.met_class, o.free_top, o.nlay, o.pinned);
   }
 };
 struct TileChoice {
@@ -926,7 +926,7 @@ long march_workgroups(const MarchSet &m, int zchunk) {
 }
 
 template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
-  TileKey key{s->d.ni, s->d.nj, s->d.nk, s->d.storage, s->d.nshots, s->d.flags, s->met_const ? 1 : 0, s->free_top,
+  TileKey key{s->d.ni, s->d.nj, s->d.nk, s->d.storage, s->d.nshots, s->d.flags, s->met_class, s->free_top,
               {}, s->split_fixed ? s->split : -1};
   for (int f = 0; f < 6; f++) key.nlay[f] = s->face[f].on ? s->face[f].nlay : 0;
   {
@@ -1001,40 +1001,63 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   float best = 1e30f;
   int bs = 0, bz = 24, bsplit = splits[0];
   bool bfuse = false;
-  for (int split : splits) {
-    s->split = split;
-    for (int shape = 0; shape < kNumShapes; shape++) {
-      s->tile_shape = shape;
-      s->fuse = true;
-      const Shell sh = make_shell(s);  // the core's bounds follow the tile shape
-      const int nz = sh.inner.box[0][5] - sh.inner.box[0][4] + 1;
-      // z chunks near 16..48 planes that split the swept planes evenly: every
-      // chunk re-reads 4 planes below it, so a short last chunk costs almost a
-      // full one (196 planes: 17, 20, 25, 28, 33, 49 instead of 16 .. 48,
-      // whose last chunk has 4 planes).  Chunks of 4..12 planes are for sweeps
-      // that 16-plane chunks would leave with fewer than 2048 workgroups (8 per
-      // CU): there the idle CUs cost more than the planes read twice (64^3: 40
-      // workgroups of 17 planes, 38 us a sweep).  With 16-bit storage they would
-      // also move small grids from one split to another, whose roundings differ.
-      constexpr int kNZ = 12;
-      const int ztarget[kNZ] = {4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
-      int last = 0;
-      for (int target : ztarget) {
-        if (target < 16 && (St<TS>::scaled || march_workgroups(sh.inner, 16) * s->d.nshots >= 2048)) continue;
-        const int n = std::max(1, (nz + target / 2) / target), zc = (nz + n - 1) / n;
-        if (zc == last) continue;
-        last = zc;
-        s->tile_zchunk = zc;
-        for (int fuse = 0; fuse <= (sh.inner.surface || sh.rim.surface ? 1 : 0); fuse++) {
-          s->fuse = fuse != 0;
-          float t;
-          int r = timed(t);
-          if (r) return r;
-          if (t < best) { best = t; bs = shape; bz = zc; bsplit = split; bfuse = s->fuse; }
+  // the fastest of the listed splits, z chunks of zmin planes and more
+  auto search = [&](const std::vector<int> &list, int zmin) -> int {
+    best = 1e30f;
+    for (int split : list) {
+      s->split = split;
+      for (int shape = 0; shape < kNumShapes; shape++) {
+        s->tile_shape = shape;
+        s->fuse = true;
+        const Shell sh = make_shell(s);  // the core's bounds follow the tile shape
+        const int nz = sh.inner.box[0][5] - sh.inner.box[0][4] + 1;
+        // z chunks near 16..48 planes that split the swept planes evenly: every
+        // chunk re-reads 4 planes below it, so a short last chunk costs almost a
+        // full one (196 planes: 17, 20, 25, 28, 33, 49 instead of 16 .. 48,
+        // whose last chunk has 4 planes).  Chunks of 4..12 planes are for sweeps
+        // that 16-plane chunks would leave with fewer than 2048 workgroups (8 per
+        // CU): there the idle CUs cost more than the planes read twice (64^3: 40
+        // workgroups of 17 planes, 38 us a sweep).
+        constexpr int kNZ = 12;
+        const int ztarget[kNZ] = {4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
+        int last = 0;
+        for (int target : ztarget) {
+          if (target < zmin || (target < 16 && march_workgroups(sh.inner, 16) * s->d.nshots >= 2048)) continue;
+          const int n = std::max(1, (nz + target / 2) / target), zc = (nz + n - 1) / n;
+          if (zc == last) continue;
+          last = zc;
+          s->tile_zchunk = zc;
+          for (int fuse = 0; fuse <= (sh.inner.surface || sh.rim.surface ? 1 : 0); fuse++) {
+            s->fuse = fuse != 0;
+            float t;
+            int r = timed(t);
+            if (r) return r;
+            if (t < best) { best = t; bs = shape; bz = zc; bsplit = split; bfuse = s->fuse; }
+          }
         }
       }
     }
+    return CGFD_OK;
+  };
+  // 16-bit storage rounds every stage, and the per-point kernel of the shell
+  // split sums in another order than the sweeps, so the choice between them is
+  // part of a session's results.  It is made on the forms that first made it
+  // (chunks of 16 planes and more, the zero terms of a constant metric taken):
+  // a grid keeps its roundings when a sweep gets faster.  The sweeps of the
+  // chosen side, equal bit for bit, then compete in their present forms.
+  if constexpr (St<TS>::scaled) {
+    if (splits.size() > 1) {
+      if (s->met_class == MET_CONST)
+        for (auto &q : sa) q.met_class = MET_REF;
+      int r = search(splits, 16);
+      if (r) return r;
+      for (auto &q : sa) q.met_class = s->met_class;
+      if (bsplit == CGFD_SPLIT_SHELL) splits = {CGFD_SPLIT_SHELL};
+      else splits = {CGFD_SPLIT_CORE, CGFD_SPLIT_PLANES};
+    }
   }
+  int r = search(splits, 0);
+  if (r) return r;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   s->tile_shape = bs;
@@ -1403,23 +1426,37 @@ int cgfd_upload_metric(cgfd_session *s, int dtype, const void *metric) {
   // largest metric magnitude of its first value and the off-diagonal ones
   // within that of zero; the sweep then takes the first point's diagonal
   // values as arguments and the off-diagonal ones as 0 (a change below
-  // 1e-10 relative in any derivative, far under FP32 rounding).  A uniform
-  // but sheared grid keeps the per-point arrays, as does
+  // 1e-10 relative in any derivative, far under FP32 rounding).  A grid of
+  // evenly spaced vertical lines passes the same test on its xi and eta rows
+  // alone (within 1e-12 in FP64 sessions, whose arithmetic would see more).  A
+  // uniform but sheared grid keeps the per-point arrays, as does
   // CGFD_FLAG_FULL_METRIC.
   const size_t n = (size_t)(s->d.ni + 6) * (s->d.nj + 6) * (s->d.nk + 6);
   double scale = 0.0;
   for (int c = 0; c < 9; c++) scale = std::max(scale, std::fabs(rd(dtype, metric, (size_t)(c + 1) * n)));
-  const double tol = 1e-10 * scale;
-  bool cst = !(s->d.flags & CGFD_FLAG_FULL_METRIC) && scale > 0.0;
-  for (int c = 0; c < 9 && cst; c++) {
+  // component c is its first value (diagonal) or zero (off-diagonal) everywhere, within tol
+  auto fixed = [&](int c, double tol) {
+    const bool diag = c % 4 == 0;  // xi_x, eta_y, zeta_z
     const double v0 = rd(dtype, metric, (size_t)(c + 1) * n);
-    const bool diag = c == 0 || c == 4 || c == 8;  // xi_x, eta_y, zeta_z
-    if (!diag && std::fabs(v0) > tol) { cst = false; break; }
+    if (!diag && !(std::fabs(v0) <= tol)) return false;
     for (size_t q = 1; q < n; q++)
-      if (std::fabs(rd(dtype, metric, (size_t)(c + 1) * n + q) - v0) > tol) { cst = false; break; }
+      if (!(std::fabs(rd(dtype, metric, (size_t)(c + 1) * n + q) - v0) <= tol)) return false;
     s->cmet[c] = diag ? v0 : 0.0;
+    return true;
+  };
+  s->met_class = MET_ALL;
+  if (!(s->d.flags & CGFD_FLAG_FULL_METRIC) && scale > 0.0) {
+    int c = 0;
+    while (c < 9 && fixed(c, 1e-10 * scale)) c++;
+    if (c == 9) {
+      s->met_class = MET_CONST;
+    } else {
+      const double tol = (s->ms == 8 ? 1e-12 : 1e-10) * scale;
+      c = 0;
+      while (c < 6 && fixed(c, tol)) c++;
+      if (c == 6) s->met_class = MET_VERT;
+    }
   }
-  s->met_const = cst;
   invalidate(s);
   return CGFD_OK;
 }
@@ -1863,7 +1900,7 @@ int cgfd_set_split(cgfd_session *s, int split) {
 
 int cgfd_get_const_metric(cgfd_session *s, int *const_metric) {
   if (!s || !const_metric) return fail(CGFD_E_ARG, "null argument");
-  *const_metric = s->met_const ? 1 : 0;
+  *const_metric = s->met_class == MET_CONST ? 1 : 0;
   return CGFD_OK;
 }
 

@@ -34,6 +34,18 @@ enum Met { JAC = 0, XIX, XIY, XIZ, ETX, ETY, ETZ, ZTX, ZTY, ZTZ, NMET };
 // MODE_RHS writes the right-hand side alone (the per-stage operator).
 enum Mode { MODE_RHS = 0, MODE_S0 = 1, MODE_S12 = 2, MODE_S3 = 3, MODE_S1Q = 4, MODE_S3Q = 5 };
 
+// What the nine metric components of a grid need per point.
+//   MET_ALL:   nine arrays
+//   MET_CONST: nothing; xi_x, eta_y, zeta_z are constants and the others zero
+//              (Cartesian grid)
+//   MET_VERT:  zeta_x, zeta_y, zeta_z; xi_x and eta_y are constants and the other
+//              xi, eta terms zero (grid lines in x and y evenly spaced and
+//              vertical lines in z: every grid over topography that moves points
+//              up and down only)
+//   MET_REF:   as MET_CONST, with the products of the zero terms still taken
+//              (16-bit storage, see the autotuner)
+enum MetClass { MET_ALL = 0, MET_CONST = 1, MET_VERT = 2, MET_REF = 3 };
+
 // ---- storage traits ---------------------------------------------------------
 template <typename TS> struct St;
 // ld/st: ordinary accesses; ld_nt/st_nt: non-temporal (streamed once, kept
@@ -209,8 +221,8 @@ template <typename TS, typename TM> struct StageArgs {
   const TM *med;   // lam, mu, 1/rho, stride L.cs
   const TM *mat;   // 18 components [c][j][i] on the physical top plane
   int free_top;
-  int met_const;   // 1: one constant per metric component, off-diagonal ones zero (Cartesian grid)
-  TM cmet[9];      // xi_x..zeta_z when met_const (off-diagonal entries exactly 0)
+  int met_class;   // MetClass of the uploaded metric
+  TM cmet[9];      // xi_x..zeta_z where the class makes them constant (the zero ones exactly 0)
   FaceArgs<TS, TM> f[6];
   // shot-0 level bases: stage input, W^n, output, the last stage's level (S1Q
   // writes Q, S3Q reads Q and S3 reads U1 there; both write W^{n+1} over it)

@@ -18,9 +18,11 @@
 // plane instead of one per dependent load.
 //
 // On a Cartesian grid every metric component is one constant and only the
-// diagonal ones (xi_x, eta_y, zeta_z) are non-zero (CART = true): the metric
+// diagonal ones (xi_x, eta_y, zeta_z) are non-zero (MET_CONST): the metric
 // comes in as arguments instead of nine HBM streams, and each derivative
 // maps to one physical direction (6 of the 9 products per component drop).
+// On a grid of evenly spaced vertical lines (MET_VERT) three streams remain,
+// 24 of 156 words per point and step less (256x256x128 FP32: 1.72 -> 1.5x ms).
 //
 // The PML variant (PML = true) sweeps whole x-y planes, PML face slabs
 // included: a point inside a face box recomputes the nine derivatives along
@@ -36,10 +38,11 @@
 
 namespace cgfd {
 
-template <int DX, int DY, int DZ, typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, int MODE,
+template <int DX, int DY, int DZ, typename TS, typename TC, int TX, int TY, int MINB, int MET, bool PML, int MODE,
           bool SURF>
 __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, MarchSet b, MarchGrid g) {
   constexpr int NT = TX * TY;
+  constexpr bool CART = MET == MET_CONST || MET == MET_REF;
   constexpr int HXL = (DX == 0) ? 3 : 1;
   constexpr int HYL = (DY == 0) ? 3 : 1;
   constexpr int LW = TX + 4, LH = TY + 4;
@@ -248,7 +251,8 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
     }
     const unsigned ob = o * (unsigned)sizeof(TC);
 #pragma unroll
-    for (int m = 0; m < 9; m++) n_met[m] = CART ? a.cmet[m] : (at_b(a.met + (XIX + m) * cs, ob));
+    for (int m = 0; m < 9; m++)
+      if (MET == MET_ALL || (MET == MET_VERT && m >= 6)) n_met[m] = at_b(a.met + (XIX + m) * cs, ob);
 #pragma unroll
     for (int m = 0; m < 3; m++) n_met[9 + m] = (at_b(a.med + m * cs, ob));
     const unsigned qb = o * (unsigned)sizeof(TS);
@@ -279,7 +283,11 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
 #pragma unroll
     for (int p = 0; p < NPER; p++) hv[p] = (TC)St<TS>::cvt(n_hv[p]) * hsc[p];
 #pragma unroll
-    for (int m = 0; m < 12; m++) mt[m] = n_met[m];
+    for (int m = 0; m < 12; m++) {
+      // components that the class makes constant: the diagonal ones from the arguments, the others zero
+      const bool cst = CART ? m < 9 : MET == MET_VERT && m < 6;
+      mt[m] = !cst ? n_met[m] : m % 4 == 0 || MET == MET_REF ? a.cmet[m < 9 ? m : 0] : TC(0);
+    }
     // LATE_RK: this plane's RK levels, issued before the next plane's
     // prefetch (memory counters complete in order), converted where used
     RT pre_r[kNC], u1_r[kNC], u2_r[kNC];
@@ -311,9 +319,9 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
         dy += Drp<TC, DY>::c(n) * lds[buf][c][ly + n][lx + HXL];
         dz += Drp<TC, DZ>::c(n) * q[c][n];
       }
-      const TC g0 = CART ? xix * dx : xix * dx + etx * dy + ztx * dz;
-      const TC g1 = CART ? ety * dy : xiy * dx + ety * dy + zty * dz;
-      const TC g2 = CART ? ztz * dz : xiz * dx + etz * dy + ztz * dz;
+      const TC g0 = CART ? xix * dx : MET == MET_VERT ? xix * dx + ztx * dz : xix * dx + etx * dy + ztx * dz;
+      const TC g1 = CART ? ety * dy : MET == MET_VERT ? ety * dy + zty * dz : xiy * dx + ety * dy + zty * dz;
+      const TC g2 = MET != MET_ALL ? ztz * dz : xiz * dx + etz * dy + ztz * dz;
       if (c < 3) {
         Lg[c][0] = g0; Lg[c][1] = g1; Lg[c][2] = g2;
       } else if (c == TXX) {
@@ -375,7 +383,8 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
           const TC e1 = DIM == 0 ? xix : DIM == 1 ? etx : ztx;
           const TC e2 = DIM == 0 ? xiy : DIM == 1 ? ety : zty;
           const TC e3 = DIM == 0 ? xiz : DIM == 1 ? etz : ztz;
-          pml_face_march<DIM, mode, TS, TC>(a, fi, shot, i, j, k, Dd, e1, e2, e3, lam, mu, lam2mu, slw, h);
+          constexpr bool diag = MET == MET_CONST || (MET == MET_VERT && DIM < 2);
+          pml_face_march<DIM, mode, diag, TS, TC>(a, fi, shot, i, j, k, Dd, e1, e2, e3, lam, mu, lam2mu, slw, h);
         };
 #pragma unroll 1
         for (unsigned fm = plane_faces; fm; fm &= fm - 1) {
@@ -422,17 +431,22 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
 }
 
 // one RK mode's k_march for the operator directions sel = 4 dx + 2 dy + dz
-template <typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, int MODE, bool SURF>
+template <typename TS, typename TC, int TX, int TY, int MINB, int MET, bool PML, int MODE, bool SURF>
 static void launch_march_m(const StageArgs<TS, TC> &a, const MarchSet &b, const MarchGrid &g, dim3 grid, dim3 block,
                            int sel, hipStream_t st) {
-  // 16-bit storage, constant metric, PML form, 32x8 tile: S1/S2 compiled for
-  // three waves per SIMD (168 VGPRs instead of 174, 40 bytes of spill) ran
-  // its sweep 15 % faster on 800x800x400.  The same bound spills 84-336
-  // bytes in the other variants (S3, the general metric, 64x4) and was
-  // slower or no faster there.
-  constexpr int MB = (sizeof(TS) == 2 && CART && PML && MODE == MODE_S12 && TX == 32 && TY == 8) ? 3 : MINB;
+  // Waves per SIMD the compiler has to leave room for.  The PML form of a
+  // constant or vertical-line metric fits three (168 VGPRs) without spilling in
+  // FP32, and with 40 bytes of spill in the 16-bit S1/S2 (15 % faster on
+  // 800x800x400); the other forms spill 84-336 bytes there and ran slower.
+  // FP64's PML form needs more than the 256 of two waves: with one, the rest goes
+  // to the accumulation registers instead of 150-350 bytes of scratch.
+  constexpr bool thin = PML && MET != MET_ALL && TX * TY == 256;
+  constexpr int MB = sizeof(TS) == 8 && PML                                ? 1
+                     : sizeof(TS) == 4 && thin                             ? 3
+                     : sizeof(TS) == 2 && thin && TX == 32 && MODE == MODE_S12 ? 3
+                                                                           : MINB;
 #define CGFD_L(X, Y, Z) \
-  hipLaunchKernelGGL((k_march<X, Y, Z, TS, TC, TX, TY, MB, CART, PML, MODE, SURF>), grid, block, 0, st, a, b, g)
+  hipLaunchKernelGGL((k_march<X, Y, Z, TS, TC, TX, TY, MB, MET, PML, MODE, SURF>), grid, block, 0, st, a, b, g)
   switch (sel) {
     case 0: CGFD_L(0, 0, 0); break;
     case 1: CGFD_L(0, 0, 1); break;
@@ -446,7 +460,7 @@ static void launch_march_m(const StageArgs<TS, TC> &a, const MarchSet &b, const 
 #undef CGFD_L
 }
 
-template <typename TS, typename TC, int TX, int TY, int MINB, bool CART, bool PML, bool SURF>
+template <typename TS, typename TC, int TX, int TY, int MINB, int MET, bool PML, bool SURF>
 static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz,
                                  int nshots, hipStream_t st) {
   MarchGrid g{};
@@ -468,7 +482,7 @@ static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, 
   dim3 grid((unsigned)nwg), block(TX * TY);
   const int sel = dx * 4 + dy * 2 + dz;
 #define CGFD_M(M) \
-  if (a.mode == M) launch_march_m<TS, TC, TX, TY, MINB, CART, PML, M, SURF>(a, b, g, grid, block, sel, st)
+  if (a.mode == M) launch_march_m<TS, TC, TX, TY, MINB, MET, PML, M, SURF>(a, b, g, grid, block, sel, st)
   if constexpr (St<TS>::scaled) {
     CGFD_M(MODE_S3);
   } else {
@@ -477,7 +491,7 @@ static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, 
   }
   CGFD_M(MODE_S0);
   CGFD_M(MODE_S12);
-  if constexpr (CGFD_SHAPE == kRhsShape && !SURF) CGFD_M(MODE_RHS);
+  if constexpr (CGFD_SHAPE == kRhsShape && !SURF && MET != MET_REF) CGFD_M(MODE_RHS);
 #undef CGFD_M
   return hipGetLastError();
 }
@@ -488,16 +502,23 @@ template <typename TS, typename TC, int SHAPE>
 hipError_t launch_interior_shape(const StageArgs<TS, TC> &a, const MarchSet &b, int dx, int dy, int dz, int nshots,
                                  hipStream_t st) {
   constexpr int TX = kTile[SHAPE][0], TY = kTile[SHAPE][1], MINB = TX * TY > 256 ? 1 : 2;
-  auto go = [&](auto cart, auto pml, auto surf) {
-    return launch_march_t<TS, TC, TX, TY, MINB, decltype(cart)::value, decltype(pml)::value, decltype(surf)::value>(
+  auto go = [&](auto met, auto pml, auto surf) {
+    return launch_march_t<TS, TC, TX, TY, MINB, decltype(met)::value, decltype(pml)::value, decltype(surf)::value>(
         a, b, dx, dy, dz, nshots, st);
   };
-  using T = std::true_type;
-  using F = std::false_type;
-  if constexpr (SHAPE == kSurfShape && !St<TS>::scaled)
-    if (b.pml && b.surface) return a.met_const ? go(T{}, T{}, T{}) : go(F{}, T{}, T{});
-  if (b.pml) return a.met_const ? go(T{}, T{}, F{}) : go(F{}, T{}, F{});
-  return a.met_const ? go(T{}, F{}, F{}) : go(F{}, F{}, F{});
+  auto form = [&](auto met) {
+    using T = std::true_type;
+    using F = std::false_type;
+    if constexpr (SHAPE == kSurfShape && !St<TS>::scaled)
+      if (b.pml && b.surface) return go(met, T{}, T{});
+    return b.pml ? go(met, T{}, F{}) : go(met, F{}, F{});
+  };
+  if constexpr (kVertShape<TS>(SHAPE))
+    if (a.met_class == MET_VERT) return form(std::integral_constant<int, MET_VERT>{});
+  if constexpr (St<TS>::scaled)
+    if (a.met_class == MET_REF) return form(std::integral_constant<int, MET_REF>{});
+  if (a.met_class == MET_CONST) return form(std::integral_constant<int, MET_CONST>{});
+  return form(std::integral_constant<int, MET_ALL>{});
 }
 
 #if CGFD_TYPE == 0

@@ -131,8 +131,10 @@ __device__ __forceinline__ bool pml_in_face(const StageArgs<TS, TC> &a, int fi, 
 // compile-time constants (straight-line component loops whose loads are
 // unconditional), every face argument is read once, and on z faces the
 // profile index is uniform across the wave, so the three profile values come
-// through scalar loads.
-template <int DIM, int MODE, typename TS, typename TC>
+// through scalar loads.  DIAG: of the face axis's metric row only the term along
+// its own direction is non-zero, so a third of the derivatives and most products
+// drop (the sums keep the value they have with zeros in them).
+template <int DIM, int MODE, bool DIAG, typename TS, typename TC>
 __device__ __forceinline__ void pml_face_march(const StageArgs<TS, TC> &a, int fi, int shot, int i, int j, int k,
                                                const TC *Dd, TC e1, TC e2, TC e3, TC lam, TC mu, TC lam2mu, TC slw,
                                                TC *h) {
@@ -147,15 +149,32 @@ __device__ __forceinline__ void pml_face_march(const StageArgs<TS, TC> &a, int f
   auto S = [&](int c) -> TC { return St<TS>::scaled ? (TC)a.sc[c] : TC(1); };
   auto IS = [&](int c) -> TC { return St<TS>::scaled ? (TC)a.isc[c] : TC(1); };
   TC R[kNC];
-  R[VX] = slw * (e1 * Dd[TXX] + e2 * Dd[TXY] + e3 * Dd[TXZ]);
-  R[VY] = slw * (e1 * Dd[TXY] + e2 * Dd[TYY] + e3 * Dd[TYZ]);
-  R[VZ] = slw * (e1 * Dd[TXZ] + e2 * Dd[TYZ] + e3 * Dd[TZZ]);
-  R[TXX] = lam2mu * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam * e3 * Dd[VZ];
-  R[TYY] = lam * e1 * Dd[VX] + lam2mu * e2 * Dd[VY] + lam * e3 * Dd[VZ];
-  R[TZZ] = lam * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam2mu * e3 * Dd[VZ];
-  R[TXY] = mu * (e2 * Dd[VX] + e1 * Dd[VY]);
-  R[TXZ] = mu * (e3 * Dd[VX] + e1 * Dd[VZ]);
-  R[TYZ] = mu * (e3 * Dd[VY] + e2 * Dd[VZ]);
+  if constexpr (DIAG) {
+    // velocity component along the axis, the stresses it drives and the two
+    // shear stresses that hold the axis
+    constexpr int VN = DIM, V1 = DIM == 0 ? VY : VX, V2 = DIM == 2 ? VY : VZ;
+    constexpr int TN = TXX + DIM, T1 = DIM == 2 ? TXZ : TXY, T2 = DIM == 0 ? TXZ : TYZ;
+    constexpr int S1 = TXX + V1, S2 = TXX + V2, S0 = DIM == 0 ? TYZ : DIM == 1 ? TXZ : TXY;
+    const TC e = DIM == 0 ? e1 : DIM == 1 ? e2 : e3;
+    R[VN] = slw * (e * Dd[TN]);
+    R[V1] = slw * (e * Dd[T1]);
+    R[V2] = slw * (e * Dd[T2]);
+    R[TN] = lam2mu * e * Dd[VN];
+    R[S1] = R[S2] = lam * e * Dd[VN];
+    R[T1] = mu * (e * Dd[V1]);
+    R[T2] = mu * (e * Dd[V2]);
+    R[S0] = TC(0);
+  } else {
+    R[VX] = slw * (e1 * Dd[TXX] + e2 * Dd[TXY] + e3 * Dd[TXZ]);
+    R[VY] = slw * (e1 * Dd[TXY] + e2 * Dd[TYY] + e3 * Dd[TYZ]);
+    R[VZ] = slw * (e1 * Dd[TXZ] + e2 * Dd[TYZ] + e3 * Dd[TZZ]);
+    R[TXX] = lam2mu * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam * e3 * Dd[VZ];
+    R[TYY] = lam * e1 * Dd[VX] + lam2mu * e2 * Dd[VY] + lam * e3 * Dd[VZ];
+    R[TZZ] = lam * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam2mu * e3 * Dd[VZ];
+    R[TXY] = mu * (e2 * Dd[VX] + e1 * Dd[VY]);
+    R[TXZ] = mu * (e3 * Dd[VX] + e1 * Dd[VZ]);
+    R[TYZ] = mu * (e3 * Dd[VY] + e2 * Dd[VZ]);
+  }
   TC P[kNC], pre[kNC], part[kNC];
 #pragma unroll
   for (int c = 0; c < kNC; c++) P[c] = (TC)St<TS>::ld(&at_b(pin, qb(c))) * S(c);
