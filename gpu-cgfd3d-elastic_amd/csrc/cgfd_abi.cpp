@@ -1014,12 +1014,13 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
         // z chunks near 16..48 planes that split the swept planes evenly: every
         // chunk re-reads 4 planes below it, so a short last chunk costs almost a
         // full one (196 planes: 17, 20, 25, 28, 33, 49 instead of 16 .. 48,
-        // whose last chunk has 4 planes).  Chunks of 4..12 planes are for sweeps
+        // whose last chunk has 4 planes).  Chunks of 2..12 planes are for sweeps
         // that 16-plane chunks would leave with fewer than 2048 workgroups (8 per
         // CU): there the idle CUs cost more than the planes read twice (64^3: 40
-        // workgroups of 17 planes, 38 us a sweep).
-        constexpr int kNZ = 12;
-        const int ztarget[kNZ] = {4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
+        // workgroups of 17 planes, 38 us a sweep; 480 of 2 planes with the
+        // surface tiles beside them, 22 us).
+        constexpr int kNZ = 14;
+        const int ztarget[kNZ] = {2, 3, 4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
         int last = 0;
         for (int target : ztarget) {
           if (target < zmin || (target < 16 && march_workgroups(sh.inner, 16) * s->d.nshots >= 2048)) continue;

@@ -22,7 +22,8 @@
 // comes in as arguments instead of nine HBM streams, and each derivative
 // maps to one physical direction (6 of the 9 products per component drop).
 // On a grid of evenly spaced vertical lines (MET_VERT) three streams remain,
-// 24 of 156 words per point and step less (256x256x128 FP32: 1.72 -> 1.5x ms).
+// 24 of 156 words per point and step less (256x256x128 FP32: core sweep of S1/S2
+// 188 -> 166 us).
 //
 // The PML variant (PML = true) sweeps whole x-y planes, PML face slabs
 // included: a point inside a face box recomputes the nine derivatives along
@@ -79,8 +80,8 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
     if (rm >= part) {
       const int q = xcd * spart + rm - part;
       if (q >= nsurf || (a.shot_active && !a.shot_active[shot])) return;
-      surface_tile<DX, DY, DZ, MODE>(a, shot, q % g.sntx, q / g.sntx % g.snty, a.L.nk - 4 + q / (g.sntx * g.snty),
-                                     &lds[0][0][0][0]);
+      surface_tile<DX, DY, DZ, MODE, MET>(a, shot, q % g.sntx, q / g.sntx % g.snty,
+                                          a.L.nk - 4 + q / (g.sntx * g.snty), &lds[0][0][0][0]);
       return;
     }
   }
@@ -368,9 +369,7 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
         // LDS columns or the z queue)
         auto face = [&](auto dimc, int fi) {
           constexpr int DIM = decltype(dimc)::value;
-          TC Dd[kNC];
-#pragma unroll
-          for (int c = 0; c < kNC; c++) {
+          auto dd = [&](int c) -> TC {
             TC d = TC(0);
 #pragma unroll
             for (int n = 0; n < 5; n++) {
@@ -378,13 +377,20 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
               else if constexpr (DIM == 1) d += Drp<TC, DY>::c(n) * lds[buf][c][ly + n][lx + HXL];
               else d += Drp<TC, DZ>::c(n) * q[c][n];
             }
-            Dd[c] = d;
-          }
+            return d;
+          };
           const TC e1 = DIM == 0 ? xix : DIM == 1 ? etx : ztx;
           const TC e2 = DIM == 0 ? xiy : DIM == 1 ? ety : zty;
           const TC e3 = DIM == 0 ? xiz : DIM == 1 ? etz : ztz;
           constexpr bool diag = MET == MET_CONST || (MET == MET_VERT && DIM < 2);
-          pml_face_march<DIM, mode, diag, TS, TC>(a, fi, shot, i, j, k, Dd, e1, e2, e3, lam, mu, lam2mu, slw, h);
+          if constexpr (sizeof(TC) == 8 && MET != MET_ALL) {
+            pml_face_march_halves<DIM, mode, diag>(a, fi, shot, i, j, k, dd, e1, e2, e3, lam, mu, lam2mu, slw, h);
+          } else {
+            TC Dd[kNC];
+#pragma unroll
+            for (int c = 0; c < kNC; c++) Dd[c] = dd(c);
+            pml_face_march<DIM, mode, diag, TS, TC>(a, fi, shot, i, j, k, Dd, e1, e2, e3, lam, mu, lam2mu, slw, h);
+          }
         };
 #pragma unroll 1
         for (unsigned fm = plane_faces; fm; fm &= fm - 1) {
@@ -434,17 +440,20 @@ __global__ __launch_bounds__(TX *TY, MINB) void k_march(StageArgs<TS, TC> a, Mar
 template <typename TS, typename TC, int TX, int TY, int MINB, int MET, bool PML, int MODE, bool SURF>
 static void launch_march_m(const StageArgs<TS, TC> &a, const MarchSet &b, const MarchGrid &g, dim3 grid, dim3 block,
                            int sel, hipStream_t st) {
-  // Waves per SIMD the compiler has to leave room for.  The PML form of a
-  // constant or vertical-line metric fits three (168 VGPRs) without spilling in
-  // FP32, and with 40 bytes of spill in the 16-bit S1/S2 (15 % faster on
-  // 800x800x400); the other forms spill 84-336 bytes there and ran slower.
-  // FP64's PML form needs more than the 256 of two waves: with one, the rest goes
-  // to the accumulation registers instead of 150-350 bytes of scratch.
-  constexpr bool thin = PML && MET != MET_ALL && TX * TY == 256;
-  constexpr int MB = sizeof(TS) == 8 && PML                                ? 1
-                     : sizeof(TS) == 4 && thin                             ? 3
+  // Waves per SIMD the compiler has to leave room for.  In FP32 the PML form of
+  // a constant or vertical-line metric fits three (168 VGPRs) without spilling;
+  // so does the 16-bit S1/S2 of a constant metric (15 % faster on 800x800x400).
+  // The other forms spill 64-336 bytes there and ran slower (200x180x100
+  // curvilinear FP32, all at three: 24.2 -> 26.0 ms).  FP64's PML form of the
+  // general metric spills 250-340 bytes to scratch at two waves; with one they
+  // go to the accumulation registers (67x53x45: 3.73 -> 3.54 ms).  Its other
+  // forms spill 0-140 bytes at two, which is still faster than one
+  // (128x128x96: 20.1 -> 19.4 ms).
+  constexpr bool thin = PML && TX * TY == 256 && MET != MET_ALL;
+  constexpr int MB = sizeof(TS) == 8 && PML && MET == MET_ALL                ? 1
+                     : sizeof(TS) == 4 && thin                               ? 3
                      : sizeof(TS) == 2 && thin && TX == 32 && MODE == MODE_S12 ? 3
-                                                                           : MINB;
+                                                                             : MINB;
 #define CGFD_L(X, Y, Z) \
   hipLaunchKernelGGL((k_march<X, Y, Z, TS, TC, TX, TY, MB, MET, PML, MODE, SURF>), grid, block, 0, st, a, b, g)
   switch (sel) {

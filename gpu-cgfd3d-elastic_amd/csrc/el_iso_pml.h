@@ -126,6 +126,46 @@ __device__ __forceinline__ bool pml_in_face(const StageArgs<TS, TC> &a, int fi, 
   return F.on && i >= F.i1 && i <= F.i2 && j >= F.j1 && j <= F.j2 && k >= F.k1 && k <= F.k2;
 }
 
+// Right-hand side along the axis DIM of a face from the derivatives along it: the
+// velocities' (VEL) and the stresses' (STR) part.
+template <int DIM, bool DIAG, bool VEL, bool STR, typename TC>
+__device__ __forceinline__ void face_rates(const TC *Dd, TC e1, TC e2, TC e3, TC lam, TC mu, TC lam2mu, TC slw, TC *R) {
+  if constexpr (DIAG) {
+    // velocity component along the axis, the stresses it drives and the two
+    // shear stresses that hold the axis
+    constexpr int VN = DIM, V1 = DIM == 0 ? VY : VX, V2 = DIM == 2 ? VY : VZ;
+    constexpr int TN = TXX + DIM, T1 = DIM == 2 ? TXZ : TXY, T2 = DIM == 0 ? TXZ : TYZ;
+    constexpr int S1 = TXX + V1, S2 = TXX + V2, S0 = DIM == 0 ? TYZ : DIM == 1 ? TXZ : TXY;
+    const TC e = DIM == 0 ? e1 : DIM == 1 ? e2 : e3;
+    if constexpr (VEL) {
+      R[VN] = slw * (e * Dd[TN]);
+      R[V1] = slw * (e * Dd[T1]);
+      R[V2] = slw * (e * Dd[T2]);
+    }
+    if constexpr (STR) {
+      R[TN] = lam2mu * e * Dd[VN];
+      R[S1] = R[S2] = lam * e * Dd[VN];
+      R[T1] = mu * (e * Dd[V1]);
+      R[T2] = mu * (e * Dd[V2]);
+      R[S0] = TC(0);
+    }
+  } else {
+    if constexpr (VEL) {
+      R[VX] = slw * (e1 * Dd[TXX] + e2 * Dd[TXY] + e3 * Dd[TXZ]);
+      R[VY] = slw * (e1 * Dd[TXY] + e2 * Dd[TYY] + e3 * Dd[TYZ]);
+      R[VZ] = slw * (e1 * Dd[TXZ] + e2 * Dd[TYZ] + e3 * Dd[TZZ]);
+    }
+    if constexpr (STR) {
+      R[TXX] = lam2mu * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam * e3 * Dd[VZ];
+      R[TYY] = lam * e1 * Dd[VX] + lam2mu * e2 * Dd[VY] + lam * e3 * Dd[VZ];
+      R[TZZ] = lam * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam2mu * e3 * Dd[VZ];
+      R[TXY] = mu * (e2 * Dd[VX] + e1 * Dd[VY]);
+      R[TXZ] = mu * (e3 * Dd[VX] + e1 * Dd[VZ]);
+      R[TYZ] = mu * (e3 * Dd[VY] + e2 * Dd[VZ]);
+    }
+  }
+}
+
 // pml_face for a point off the free-surface row (no surface term), the form
 // the z-marching sweep uses: the face axis DIM and the RK mode MODE are
 // compile-time constants (straight-line component loops whose loads are
@@ -149,32 +189,7 @@ __device__ __forceinline__ void pml_face_march(const StageArgs<TS, TC> &a, int f
   auto S = [&](int c) -> TC { return St<TS>::scaled ? (TC)a.sc[c] : TC(1); };
   auto IS = [&](int c) -> TC { return St<TS>::scaled ? (TC)a.isc[c] : TC(1); };
   TC R[kNC];
-  if constexpr (DIAG) {
-    // velocity component along the axis, the stresses it drives and the two
-    // shear stresses that hold the axis
-    constexpr int VN = DIM, V1 = DIM == 0 ? VY : VX, V2 = DIM == 2 ? VY : VZ;
-    constexpr int TN = TXX + DIM, T1 = DIM == 2 ? TXZ : TXY, T2 = DIM == 0 ? TXZ : TYZ;
-    constexpr int S1 = TXX + V1, S2 = TXX + V2, S0 = DIM == 0 ? TYZ : DIM == 1 ? TXZ : TXY;
-    const TC e = DIM == 0 ? e1 : DIM == 1 ? e2 : e3;
-    R[VN] = slw * (e * Dd[TN]);
-    R[V1] = slw * (e * Dd[T1]);
-    R[V2] = slw * (e * Dd[T2]);
-    R[TN] = lam2mu * e * Dd[VN];
-    R[S1] = R[S2] = lam * e * Dd[VN];
-    R[T1] = mu * (e * Dd[V1]);
-    R[T2] = mu * (e * Dd[V2]);
-    R[S0] = TC(0);
-  } else {
-    R[VX] = slw * (e1 * Dd[TXX] + e2 * Dd[TXY] + e3 * Dd[TXZ]);
-    R[VY] = slw * (e1 * Dd[TXY] + e2 * Dd[TYY] + e3 * Dd[TYZ]);
-    R[VZ] = slw * (e1 * Dd[TXZ] + e2 * Dd[TYZ] + e3 * Dd[TZZ]);
-    R[TXX] = lam2mu * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam * e3 * Dd[VZ];
-    R[TYY] = lam * e1 * Dd[VX] + lam2mu * e2 * Dd[VY] + lam * e3 * Dd[VZ];
-    R[TZZ] = lam * e1 * Dd[VX] + lam * e2 * Dd[VY] + lam2mu * e3 * Dd[VZ];
-    R[TXY] = mu * (e2 * Dd[VX] + e1 * Dd[VY]);
-    R[TXZ] = mu * (e3 * Dd[VX] + e1 * Dd[VZ]);
-    R[TYZ] = mu * (e3 * Dd[VY] + e2 * Dd[VZ]);
-  }
+  face_rates<DIM, DIAG, true, true>(Dd, e1, e2, e3, lam, mu, lam2mu, slw, R);
   TC P[kNC], pre[kNC], part[kNC];
 #pragma unroll
   for (int c = 0; c < kNC; c++) P[c] = (TC)St<TS>::ld(&at_b(pin, qb(c))) * S(c);
@@ -235,6 +250,85 @@ __device__ __forceinline__ void pml_face_march(const StageArgs<TS, TC> &a, int f
 #pragma unroll
     for (int c = 0; c < kNC; c++) St<TS>::st(&at_b(pout, qb(c)), Ph[c] * IS(c));
   }
+}
+
+// pml_face_march in FP64 where two waves per SIMD leave 256 registers: the
+// velocities and then the stresses (the memory clobber keeps the second group's
+// loads behind the first's stores); all nine memory variables at once need 50-90
+// registers more.  dd(c): derivative of component c along the face axis.
+template <int DIM, int MODE, bool DIAG, typename TS, typename TC, typename DD>
+__device__ __forceinline__ void pml_face_march_halves(const StageArgs<TS, TC> &a, int fi, int shot, int i, int j, int k,
+                                                      const DD &dd, TC e1, TC e2, TC e3, TC lam, TC mu, TC lam2mu,
+                                                      TC slw, TC *h) {
+  static_assert(!St<TS>::scaled && MODE != MODE_S3, "FP64 forms only");
+  const FaceArgs<TS, TC> &F = a.f[fi];
+  const int i1 = F.i1, j1 = F.j1, k1 = F.k1, bi = F.bi, bj = F.bj;
+  const long fso = (long)shot * F.shot_stride;
+  const TS *pin = F.a_in + fso, *ppre = F.a_pre + fso;
+  TS *pout = F.a_out + fso, *pend = F.a_end + fso;
+  const unsigned fs = (unsigned)F.fsize;
+  const unsigned ia = (unsigned)(((k - k1) * bj + (j - j1)) * bi + (i - i1));
+  auto qb = [&](int c) { return (c * fs + ia) * (unsigned)sizeof(TS); };
+  TC cD, cA, cB;
+  if constexpr (DIM == 2) {
+    typedef const __attribute__((address_space(4))) TC *cptr;
+    const int ic = k - k1;
+    cD = ((cptr)F.D)[ic];
+    cA = ((cptr)F.A)[ic];
+    cB = ((cptr)F.B)[ic];
+  } else {
+    const int ic = DIM == 0 ? i - i1 : j - j1;
+    cD = F.D[ic];
+    cA = F.A[ic];
+    cB = F.B[ic];
+  }
+  const TC Bm1 = cB - TC(1);
+  // components c0 .. c1-1; their right-hand sides need the derivatives of
+  // components d0 .. d1-1
+  auto group = [&](auto c0_, auto c1_, auto d0_, auto d1_) {
+    constexpr int c0 = decltype(c0_)::value, c1 = decltype(c1_)::value;
+    constexpr int d0 = decltype(d0_)::value, d1 = decltype(d1_)::value;
+    TC Dd[kNC], R[kNC];
+#pragma unroll
+    for (int c = d0; c < d1; c++) Dd[c] = dd(c);
+    face_rates<DIM, DIAG, c0 == 0, c1 == kNC>(Dd, e1, e2, e3, lam, mu, lam2mu, slw, R);
+    TC P[kNC], pre[kNC], Ph[kNC];
+#pragma unroll
+    for (int c = c0; c < c1; c++) P[c] = (TC)St<TS>::ld(&at_b(pin, qb(c)));
+    if constexpr (MODE != MODE_S0 && MODE != MODE_RHS) {  // W^n (S3Q: Q)
+      const TS *p = MODE == MODE_S3Q ? pend : ppre;
+#pragma unroll
+      for (int c = c0; c < c1; c++) pre[c] = (TC)St<TS>::ld(&at_b(p, qb(c)));
+    }
+#pragma unroll
+    for (int c = c0; c < c1; c++) {
+      h[c] += Bm1 * R[c] - cB * P[c];
+      Ph[c] = cD * R[c] - cA * P[c];
+    }
+#pragma unroll
+    for (int c = c0; c < c1; c++) {
+      if constexpr (MODE == MODE_S12) {
+        St<TS>::st(&at_b(pout, qb(c)), (pre[c] + a.ca * Ph[c]));
+      } else if constexpr (MODE == MODE_S1Q) {
+        TC u2, q;
+        rk_sum(a.rk_w, pre[c], P[c], a.ca, Ph[c], u2, q);
+        St<TS>::st(&at_b(pout, qb(c)), u2);
+        St<TS>::st(&at_b(pend, qb(c)), q);
+      } else if constexpr (MODE == MODE_S3Q) {
+        St<TS>::st(&at_b(pend, qb(c)), rk_end(a.rk_w, pre[c], P[c], a.cb, Ph[c]));
+      } else if constexpr (MODE == MODE_S0) {
+        St<TS>::st(&at_b(pout, qb(c)), (P[c] + a.ca * Ph[c]));
+      } else {
+        St<TS>::st(&at_b(pout, qb(c)), Ph[c]);
+      }
+    }
+  };
+  using std::integral_constant;
+  group(integral_constant<int, 0>{}, integral_constant<int, 3>{}, integral_constant<int, 3>{},
+        integral_constant<int, kNC>{});
+  __asm__ volatile("" ::: "memory");
+  group(integral_constant<int, 3>{}, integral_constant<int, kNC>{}, integral_constant<int, 0>{},
+        integral_constant<int, 3>{});
 }
 
 // Every face box containing the point, in the reference's face order.

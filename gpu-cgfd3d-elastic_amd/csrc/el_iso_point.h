@@ -60,8 +60,9 @@ __device__ __forceinline__ void rk_store(const StageArgs<TS, TC> &a, long so, in
 // of component c.  SURF: every point of the call lies on one free-surface row,
 // acc.vx / acc.vy hold the conservative traction vectors at the x / y taps, and
 // tder says whether the stress derivatives are needed (inner momentum form, PML
-// faces).
-template <int DX, int DY, int DZ, int MODE, bool SURF, typename TS, typename TC, typename ACC>
+// faces).  MET: the metric components that are constant or zero (MetClass) are
+// neither loaded nor multiplied.
+template <int DX, int DY, int DZ, int MODE, bool SURF, int MET, typename TS, typename TC, typename ACC>
 __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int shot, int i, int j, int k, bool tder,
                                              const ACC &acc) {
   const Layout &L = a.L;
@@ -98,9 +99,10 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
   auto Mt = [&](int m, long d) -> TC {
     return at_b(met + m * cs, (unsigned)(o + (int)d) * (unsigned)sizeof(TC));
   };
-  const TC xix = Mt(XIX, 0), xiy = Mt(XIY, 0), xiz = Mt(XIZ, 0);
-  const TC etx = Mt(ETX, 0), ety = Mt(ETY, 0), etz = Mt(ETZ, 0);
-  const TC ztx = Mt(ZTX, 0), zty = Mt(ZTY, 0), ztz = Mt(ZTZ, 0);
+  constexpr bool ALL = MET == MET_ALL, CST = MET == MET_CONST;
+  const TC xix = ALL ? Mt(XIX, 0) : a.cmet[0], xiy = ALL ? Mt(XIY, 0) : TC(0), xiz = ALL ? Mt(XIZ, 0) : TC(0);
+  const TC etx = ALL ? Mt(ETX, 0) : TC(0), ety = ALL ? Mt(ETY, 0) : a.cmet[4], etz = ALL ? Mt(ETZ, 0) : TC(0);
+  const TC ztx = CST ? TC(0) : Mt(ZTX, 0), zty = CST ? TC(0) : Mt(ZTY, 0), ztz = CST ? a.cmet[8] : Mt(ZTZ, 0);
   const unsigned ob = (unsigned)o * (unsigned)sizeof(TC);
   const TC lam = at_b(a.med, ob), mu = at_b(a.med + cs, ob), slw = at_b(a.med + 2 * cs, ob);
   // lam + 2.0*mu: the double-promoted sum of the reference rounds to the same
@@ -117,6 +119,7 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
 #pragma unroll
     for (int cc = 0; cc < 3; cc++) {
       auto vec = [&](long d, int e1, int e2, int e3) -> TC {
+        if constexpr (CST) return Mt(JAC, d) * (ztz * (W(T3[cc], d) * S(T3[cc])));  // along z only, see SurfAcc
         return Mt(JAC, d) * (Mt(e1, d) * (W(T1[cc], d) * S(T1[cc])) + Mt(e2, d) * (W(T2[cc], d) * S(T2[cc])) +
                              Mt(e3, d) * (W(T3[cc], d) * S(T3[cc])));
       };
@@ -141,6 +144,14 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
         DzTz += Drp<TC, DZ>::c(n) * v;
       }
       h[VX + cc] = (DxTx + DyTy + DzTz) * slwjac;
+    }
+  } else if constexpr (!ALL) {
+    constexpr int T1[3] = {TXX, TXY, TXZ}, T2[3] = {TXY, TYY, TYZ}, T3[3] = {TXZ, TYZ, TZZ};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      TC s = xix * Dx[T1[c]] + ety * Dy[T2[c]] + ztz * Dz[T3[c]];
+      if constexpr (!CST) s += ztx * Dz[T1[c]] + zty * Dz[T2[c]];
+      h[c] = slw * s;
     }
   } else {
     h[VX] = slw * (xix * Dx[TXX] + xiy * Dx[TXY] + xiz * Dx[TXZ] + etx * Dy[TXX] + ety * Dy[TXY] + etz * Dy[TXZ] +
@@ -183,15 +194,36 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
       DzVz = (c0 * W(VZ, s0) + c1 * W(VZ, s1) + c2 * W(VZ, s2)) * S(VZ);
     }
   }
-  h[TXX] = lam2mu * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx) +
-           lam * (xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy + xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz);
-  h[TYY] = lam2mu * (xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy) +
-           lam * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx + xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz);
-  h[TZZ] = lam2mu * (xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz) +
-           lam * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx + xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy);
-  h[TXY] = mu * (xiy * Dx[VX] + xix * Dx[VY] + ety * Dy[VX] + etx * Dy[VY] + zty * DzVx + ztx * DzVy);
-  h[TXZ] = mu * (xiz * Dx[VX] + xix * Dx[VZ] + etz * Dy[VX] + etx * Dy[VZ] + ztz * DzVx + ztx * DzVz);
-  h[TYZ] = mu * (xiz * Dx[VY] + xiy * Dx[VZ] + etz * Dy[VY] + ety * Dy[VZ] + ztz * DzVy + zty * DzVz);
+  if constexpr (!ALL) {
+    const TC DzV[3] = {DzVx, DzVy, DzVz};
+    TC G[3][3];  // G[c][b] = dV_c / dx_b
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      G[c][0] = xix * Dx[c];
+      G[c][1] = ety * Dy[c];
+      G[c][2] = ztz * DzV[c];
+      if constexpr (!CST) {
+        G[c][0] += ztx * DzV[c];
+        G[c][1] += zty * DzV[c];
+      }
+    }
+    h[TXX] = lam2mu * G[0][0] + lam * (G[1][1] + G[2][2]);
+    h[TYY] = lam2mu * G[1][1] + lam * (G[0][0] + G[2][2]);
+    h[TZZ] = lam2mu * G[2][2] + lam * (G[0][0] + G[1][1]);
+    h[TXY] = mu * (G[0][1] + G[1][0]);
+    h[TXZ] = mu * (G[0][2] + G[2][0]);
+    h[TYZ] = mu * (G[1][2] + G[2][1]);
+  } else {
+    h[TXX] = lam2mu * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx) +
+             lam * (xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy + xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz);
+    h[TYY] = lam2mu * (xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy) +
+             lam * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx + xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz);
+    h[TZZ] = lam2mu * (xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz) +
+             lam * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx + xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy);
+    h[TXY] = mu * (xiy * Dx[VX] + xix * Dx[VY] + ety * Dy[VX] + etx * Dy[VY] + zty * DzVx + ztx * DzVy);
+    h[TXZ] = mu * (xiz * Dx[VX] + xix * Dx[VZ] + etz * Dy[VX] + etx * Dy[VZ] + ztz * DzVx + ztx * DzVz);
+    h[TYZ] = mu * (xiz * Dx[VY] + xiy * Dx[VZ] + etz * Dy[VY] + ety * Dy[VZ] + ztz * DzVy + zty * DzVz);
+  }
 
   // ---- CFS-PML faces, in the reference's face order ----
   pml_apply<MODE, TS, TC>(a, shot, i, j, k, Dx, Dy, Dz, xix, xiy, xiz, etx, ety, etz, ztx, zty, ztz, lam, mu, lam2mu,
@@ -230,7 +262,7 @@ template <int DX, int DY, typename TC> struct SurfAcc {
   __device__ __forceinline__ TC vy(int cc, int n) const { return at(kNC + 3 + cc, ly + n, lx + HXL); }
 };
 
-template <int DX, int DY, int DZ, int MODE, typename TS, typename TC>
+template <int DX, int DY, int DZ, int MODE, int MET, typename TS, typename TC>
 __device__ __forceinline__ void surface_tile(const StageArgs<TS, TC> &a, int shot, int tx, int ty, int k, TC *lds) {
   using Acc = SurfAcc<DX, DY, TC>;
   constexpr int LW = Acc::LW, LH = Acc::LH, HXL = Acc::HXL, HYL = Acc::HYL;
@@ -265,8 +297,10 @@ __device__ __forceinline__ void surface_tile(const StageArgs<TS, TC> &a, int sho
       J = Mt(JAC);
 #pragma unroll
       for (int q = 0; q < 3; q++) {
-        ex[q] = vx ? Mt(XIX + q) : TC(0);
-        ey[q] = vy ? Mt(ETX + q) : TC(0);
+        if constexpr (MET == MET_ALL) {
+          ex[q] = vx ? Mt(XIX + q) : TC(0);
+          ey[q] = vy ? Mt(ETX + q) : TC(0);
+        }
       }
     }
 #pragma unroll
@@ -276,6 +310,11 @@ __device__ __forceinline__ void surface_tile(const StageArgs<TS, TC> &a, int sho
       constexpr int T1[3] = {TXX, TXY, TXZ}, T2[3] = {TXY, TYY, TYZ}, T3[3] = {TXZ, TYZ, TZZ};
 #pragma unroll
       for (int cc = 0; cc < 3; cc++) {
+        if constexpr (MET != MET_ALL) {
+          if (vx) lds[(kNC + cc) * (LH * LW) + cell] = J * (a.cmet[0] * w[T1[cc]]);
+          if (vy) lds[(kNC + 3 + cc) * (LH * LW) + cell] = J * (a.cmet[4] * w[T2[cc]]);
+          continue;
+        }
         if (vx) lds[(kNC + cc) * (LH * LW) + cell] = J * (ex[0] * w[T1[cc]] + ex[1] * w[T2[cc]] + ex[2] * w[T3[cc]]);
         if (vy) lds[(kNC + 3 + cc) * (LH * LW) + cell] = J * (ey[0] * w[T1[cc]] + ey[1] * w[T2[cc]] + ey[2] * w[T3[cc]]);
       }
@@ -290,7 +329,7 @@ __device__ __forceinline__ void surface_tile(const StageArgs<TS, TC> &a, int sho
     stage(i0 - HXL + col, j0 + row, (row + HYL) * LW + col, true, false);
   }
   __syncthreads();
-  if (i < L.ni && j < L.nj) point_update<DX, DY, DZ, MODE, true>(a, shot, i, j, k, tder, Acc{lds, lx, ly});
+  if (i < L.ni && j < L.nj) point_update<DX, DY, DZ, MODE, true, MET>(a, shot, i, j, k, tder, Acc{lds, lx, ly});
 }
 
 }  // namespace cgfd

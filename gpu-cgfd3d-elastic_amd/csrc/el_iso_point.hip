@@ -58,19 +58,19 @@ __global__ __launch_bounds__(256) void k_point(StageArgs<TS, TC> a) {
   int i, j, k;
   if (!box_point(a, gid, i, j, k)) return;
   const MemAcc<DX, DY, TS, TC> acc{a, a.w_in + (long)shot * a.shot_stride, (int)a.L.off(i, j, k)};
-  point_update<DX, DY, DZ, MODE, false>(a, shot, i, j, k, true, acc);
+  point_update<DX, DY, DZ, MODE, false, MET_ALL>(a, shot, i, j, k, true, acc);
 }
 
 // The 4 free-surface rows (surface_tile); workgroups as in the sweep: each XCD
 // takes a contiguous eighth of a shot's tiles.
-template <int DX, int DY, int DZ, int MODE, typename TS, typename TC>
+template <int DX, int DY, int DZ, int MODE, int MET, typename TS, typename TC>
 __global__ __launch_bounds__(256, 2) void k_surface(StageArgs<TS, TC> a, int ntx, int nty) {
   __shared__ TC lds[kSurfLds];
   const int per_shot = ntx * nty * 4, part = (per_shot + 7) / 8;
   const int xcd = blockIdx.x % 8, m = blockIdx.x / 8;
   const int shot = m / part, q = xcd * part + (m - shot * part);
   if (q >= per_shot || (a.shot_active && !a.shot_active[shot])) return;
-  surface_tile<DX, DY, DZ, MODE>(a, shot, q % ntx, q / ntx % nty, a.L.nk - 4 + q / (ntx * nty), lds);
+  surface_tile<DX, DY, DZ, MODE, MET>(a, shot, q % ntx, q / ntx % nty, a.L.nk - 4 + q / (ntx * nty), lds);
 }
 
 // ---- sources (sv_curv_col_el_iso_rhs_src_gpu, sv_curv_col_el_gpu.cu:227-301) ----
@@ -302,10 +302,10 @@ static void launch_point_m(const StageArgs<TS, TC> &a, dim3 grid, int sel, hipSt
   CGFD_DIRS(sel)
 #undef CGFD_L
 }
-template <int MODE, typename TS, typename TC>
+template <int MODE, int MET, typename TS, typename TC>
 static void launch_surface_m(const StageArgs<TS, TC> &a, dim3 grid, int ntx, int nty, int sel, hipStream_t st) {
   const dim3 block(kSurfX * kSurfY);
-#define CGFD_L(X, Y, Z) hipLaunchKernelGGL((k_surface<X, Y, Z, MODE, TS, TC>), grid, block, 0, st, a, ntx, nty)
+#define CGFD_L(X, Y, Z) hipLaunchKernelGGL((k_surface<X, Y, Z, MODE, MET, TS, TC>), grid, block, 0, st, a, ntx, nty)
   CGFD_DIRS(sel)
 #undef CGFD_L
 }
@@ -338,8 +338,13 @@ hipError_t launch_surface(const StageArgs<TS, TC> &a, int dx, int dy, int dz, in
   const int ntx = (a.L.ni + kSurfX - 1) / kSurfX, nty = (a.L.nj + kSurfY - 1) / kSurfY;
   const dim3 grid((unsigned)(8L * ((ntx * nty * 4 + 7) / 8) * nshots));
   if constexpr (!St<TS>::scaled)
-    with_mode<TS>(a.mode,
-                  [&](auto m) { launch_surface_m<decltype(m)::value>(a, grid, ntx, nty, dx * 4 + dy * 2 + dz, st); });
+    with_mode<TS>(a.mode, [&](auto m) {
+      constexpr int M = decltype(m)::value;
+      const int sel = dx * 4 + dy * 2 + dz;
+      if (a.met_class == MET_CONST) launch_surface_m<M, MET_CONST>(a, grid, ntx, nty, sel, st);
+      else if (a.met_class == MET_VERT) launch_surface_m<M, MET_VERT>(a, grid, ntx, nty, sel, st);
+      else launch_surface_m<M, MET_ALL>(a, grid, ntx, nty, sel, st);
+    });
   return hipGetLastError();
 }
 
