@@ -55,21 +55,22 @@ KERNEL_PATH = {cgfd.SPLIT_PLANES: "zmarch planes", cgfd.SPLIT_SHELL: "zmarch + p
 # the reference's dataflow with the RK update fused, mean of 39/57/57/39
 # words (wavefield in, 12 coefficients, RK levels in and out).
 ALGO_BYTES = {"f32": 192.0, "f16": 120.0, "bf16": 120.0, "f64": 384.0}
-# This build's own dataflow (stage values): wavefield words per swept point
-# and stage, S0 9 in + 9 out, S1/S2 9 in + 9 W^n + 9 out, S3 9 in + 27 (W^n,
-# U1, U2) + 9 out, mean 29.25; plus 12 coefficient words (3, the medium,
-# when the metric is constant and passed as kernel arguments).  The nine
-# PML memory variables of a (point, face) pair follow the same pattern.
-WAVE_WORDS = 29.25
+# This build's own dataflow: wavefield words per swept point and stage, S0 9 in
+# + 9 out, S1 9 in + 9 W^n + 9 out + 9 of the stage values' sum, S2 9 in + 9
+# W^n + 9 out, S3 9 in + 9 sum + 9 out, mean 27; 16-bit storage keeps no sum (S1
+# 27, S3 9 in + 27 W^n, U1, U2 + 9 out), mean 29.25; plus 12 coefficient words
+# (3, the medium, when the metric is constant and passed as kernel arguments).
+# The nine PML memory variables of a (point, face) pair follow the same pattern.
+WAVE_WORDS = {"f32": 27.0, "f16": 29.25, "bf16": 29.25, "f64": 27.0}
 ES_WAVE = {"f32": 4, "f16": 2, "bf16": 2, "f64": 8}
 ES_MODEL = {"f32": 4, "f16": 4, "bf16": 4, "f64": 8}
 
 
 def path_bytes(storage, const_metric):
-    return WAVE_WORDS * ES_WAVE[storage] + (3 if const_metric else 12) * ES_MODEL[storage]
+    return WAVE_WORDS[storage] * ES_WAVE[storage] + (3 if const_metric else 12) * ES_MODEL[storage]
 
 
-AUX_BYTES = {k: WAVE_WORDS * v for k, v in ES_WAVE.items()}
+AUX_BYTES = {k: WAVE_WORDS[k] * v for k, v in ES_WAVE.items()}
 STORE = {"f32": cgfd.STORE_F32, "f16": cgfd.STORE_F16, "bf16": cgfd.STORE_BF16, "f64": cgfd.STORE_F64}
 
 

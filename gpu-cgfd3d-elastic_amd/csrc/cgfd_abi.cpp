@@ -742,9 +742,9 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
 // planes in two sweeps, the PML-free form over a core box inside every face
 // box whose x extent starts and ends on tile boundaries (so its rows load
 // whole 128-byte lines), and the PML form over the up to six rim boxes around
-// it; the PML-free form needs far fewer registers (FP32 32x8 tile: 108 / 128
-// / 164 VGPRs against 160 / 168 / 212 in S0 / S1-S2 / S3), so more waves
-// hide its latency.  CGFD_SPLIT_SHELL (or CGFD_FLAG_PML_POINT): the sweep
+// it; the PML-free form needs fewer registers (FP32 32x8 tile, constant
+// metric: 102-124 VGPRs, 4 waves per SIMD, against 137-159, 3 waves), so more
+// waves hide its latency.  CGFD_SPLIT_SHELL (or CGFD_FLAG_PML_POINT): the sweep
 // keeps to the box inside every face box and the per-point launch takes the
 // whole shell (face slabs and surface rows: a launch of their own gained
 // nothing next to the slabs, 183 against 162 + 26 us on 211x187x121 bfloat16).

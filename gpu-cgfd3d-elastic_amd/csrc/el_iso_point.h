@@ -239,8 +239,8 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
 // the rows of the traction image the x and y traction vectors J e.T, are staged
 // in LDS once with their halos; a point then reads 90 LDS values where the
 // per-point form made 135 loads for its derivatives and 315 more for the image
-// (J, three metric terms and three stresses at each of its 45 taps, now 40 along
-// z).  The rows are latency-bound either way: one row per workgroup instead of
+// (J, three metric terms and three stresses at each of its 45 taps; what is left
+// of them are the taps along z).  The rows are latency-bound either way: one row per workgroup instead of
 // a march over the four keeps four times as many in flight, which small grids
 // need (64x64 columns: 64 workgroups), for z taps that hit the L2.
 constexpr int kSurfX = 32, kSurfY = 8, kSurfComp = kNC + 6;

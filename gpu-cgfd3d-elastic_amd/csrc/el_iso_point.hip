@@ -109,8 +109,8 @@ __device__ __forceinline__ bool src_rate(const SrcArgs<TS, TC> &a, int p, int it
 }
 
 // One thread per distinct grid point; the rates, from the step's table where
-// there is one (10.5 -> 6 us: the contributions are a chain of dependent
-// loads), are applied to the RK outputs of this stage.  Serves 16-bit storage,
+// there is one (10.8 -> 8.7 us on a single moment source: the contributions
+// are a chain of dependent loads), are applied to the RK outputs of this stage.  Serves 16-bit storage,
 // the bare right-hand side and sources that spread too far for a box (see
 // k_step_head).
 template <typename TS, typename TC>

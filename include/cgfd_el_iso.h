@@ -78,7 +78,7 @@ typedef struct {
 #define CGFD_FLAG_PLAIN 1
 /* PML face slabs by the per-point kernel, the z-marching kernel only on the
  * box inside them (by default the z-marching kernel sweeps whole planes,
- * PML included, and the per-point kernel takes the 4 free-surface rows) */
+ * PML included, and the 4 free-surface rows are updated apart) */
 #define CGFD_FLAG_PML_POINT 2
 /* keep the per-point metric arrays even when the grid is Cartesian (by
  * default a metric whose components are constant to 1e-10 of their largest
@@ -218,10 +218,9 @@ int cgfd_get_tile(cgfd_session *s, int *shape, int *tx, int *ty, int *zchunk);
 
 /* Work split of a stage between the z-marching and the per-point kernel. */
 #define CGFD_SPLIT_SHELL 0  /* sweep inside the PML face boxes; per-point kernel on the slabs and 4 surface rows */
-#define CGFD_SPLIT_PLANES 1 /* sweep whole planes with the PML terms; per-point kernel on the 4 surface rows */
+#define CGFD_SPLIT_PLANES 1 /* sweep whole planes with the PML terms; the 4 surface rows apart */
 #define CGFD_SPLIT_CORE 2   /* whole planes in two sweeps: the PML-free form on a tile-aligned core inside the
-                               face boxes, the PML form on the boxes around it; per-point kernel on the 4
-                               surface rows */
+                               face boxes, the PML form on the boxes around it; the 4 surface rows apart */
 int cgfd_get_split(cgfd_session *s, int *split);
 /* Pin the work split (split < 0: the autotuner chooses again).  With an
  * automatic tile the autotuner then tunes the tile under that split only.
