@@ -970,9 +970,12 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   // minimum over reps 1..2 of one full step's four stages under the session's
-  // present choice
-  auto timed = [&](float &tmin) -> int {
-    const Shell sh = make_shell(s);
+  // present choice: the sweeps, the other launches, or both
+  enum { SWEEPS = 1, OTHERS = 2 };
+  auto timed = [&](float &tmin, int parts) -> int {
+    Shell sh = make_shell(s);
+    if (!(parts & SWEEPS)) sh.inner.nbox = sh.rim.nbox = 0;
+    if (!(parts & OTHERS)) { sh.point.n = 0; sh.surface = false; }
     tmin = 1e30f;
     for (int rep = 0; rep < 3; rep++) {
       HIPCHK(hipEventRecord(e0, s->st));
@@ -1001,11 +1004,19 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   float best = 1e30f;
   int bs = 0, bz = 24, bsplit = splits[0];
   bool bfuse = false;
-  // the fastest of the listed splits, z chunks of zmin planes and more
-  auto search = [&](const std::vector<int> &list, int zmin) -> int {
+  float pml_cost = 1.0f;  // weight of the sweeps with PML terms
+  // the fastest of the listed splits, z chunks of zmin planes and more; apart:
+  // sweeps and other launches timed by themselves and their minima added
+  auto search = [&](const std::vector<int> &list, int zmin, bool apart) -> int {
     best = 1e30f;
     for (int split : list) {
       s->split = split;
+      float others = 0;
+      if (apart) {
+        s->tile_shape = 0;
+        int r = timed(others, OTHERS);
+        if (r) return r;
+      }
       for (int shape = 0; shape < kNumShapes; shape++) {
         s->tile_shape = shape;
         s->fuse = true;
@@ -1031,8 +1042,9 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
           for (int fuse = 0; fuse <= (sh.inner.surface || sh.rim.surface ? 1 : 0); fuse++) {
             s->fuse = fuse != 0;
             float t;
-            int r = timed(t);
+            int r = timed(t, apart ? SWEEPS : SWEEPS | OTHERS);
             if (r) return r;
+            t = (split == CGFD_SPLIT_SHELL ? t : t * pml_cost) + others;
             if (t < best) { best = t; bs = shape; bz = zc; bsplit = split; bfuse = s->fuse; }
           }
         }
@@ -1043,21 +1055,30 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   // 16-bit storage rounds every stage, and the per-point kernel of the shell
   // split sums in another order than the sweeps, so the choice between them is
   // part of a session's results.  It is made on the forms that first made it
-  // (chunks of 16 planes and more, the zero terms of a constant metric taken):
+  // and in the way it was first made (chunks of 16 planes and more, the zero
+  // terms of a constant metric taken, sweeps and slabs timed apart: on whole
+  // stages 256x256x128 float16, 1.97 against 2.00 ms a step, fell to the other side):
   // a grid keeps its roundings when a sweep gets faster.  The sweeps of the
   // chosen side, equal bit for bit, then compete in their present forms.
   if constexpr (St<TS>::scaled) {
     if (splits.size() > 1) {
-      if (s->met_class == MET_CONST)
+      if (s->met_class == MET_CONST) {
         for (auto &q : sa) q.met_class = MET_REF;
-      int r = search(splits, 16);
+        // in FP16 that form compiles to faster code than it first did (64 shots
+        // of 100x100x60, whole step: 12.1 against 13.0 ms, the shell 12.8): of 12
+        // Cartesian grids the shell was taken wherever the sweeps' share of it is
+        // 0.94 and more, the sweeps up to 0.90; bfloat16 shows no such shift
+        if (std::is_same<TS, __half>::value) pml_cost = 1.08f;
+      }
+      int r = search(splits, 16, true);
       if (r) return r;
+      pml_cost = 1.0f;
       for (auto &q : sa) q.met_class = s->met_class;
       if (bsplit == CGFD_SPLIT_SHELL) splits = {CGFD_SPLIT_SHELL};
       else splits = {CGFD_SPLIT_CORE, CGFD_SPLIT_PLANES};
     }
   }
-  int r = search(splits, 0);
+  int r = search(splits, 0, false);
   if (r) return r;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
