@@ -18,19 +18,24 @@ enum Met { JAC = 0, XIX, XIY, XIZ, ETX, ETY, ETZ, ZTX, ZTY, ZTZ, NMET };
 // stage values U1..U3 (U_{i+1} = W^n + a_i dt K_i):
 //   S0:   U1 = W + a0 dt K0                      (input W^n)
 //   S12:  U2 = W + a1 dt K1, U3 = W + a2 dt K2   (input U1 / U2, W^n read at the point)
-//   S1Q:  S12's U2, and Q = (1 - w3) W + w1 (U1 - W) + w2 (U2 - W)
-//   S3Q:  W^{n+1} = Q + w3 U3 + b3 dt K3         (input U3; written over Q)
+//   S1Q:  S12's U2, and Q = W + (U1 - W) / 2 + (U2 - W)
+//   S3Q:  W^{n+1} = Q + w3 (U3 - Q) + b3 dt K3   (input U3; written over Q)
 //   S3:   W^{n+1} = W + w1 (U1 - W) + w2 (U2 - W) + w3 (U3 - W) + b3 dt K3
 //         (input U3; written over U1)
 // with w_i = b_{i-1} / a_{i-1} = 1/3, 2/3, 1/3, which equals
-// W + dt (b0 K0 + b1 K1 + b2 K2 + b3 K3).  FP32 and FP64 storage run S0, S1Q,
-// S12, S3Q: Q carries W, U1 and U2 into the last stage in one level, 108
-// instead of 117 level words per point and step, and S3Q reads 9 words at the
-// point where S3 reads 27 (per step, before and after: 400x400x200 Cartesian
-// FP32 5.46 -> 4.96 ms, 64 shots of 100x100x60 12.3 -> 10.7 ms, 128x128x96
-// curvilinear FP64 1.51 -> 1.26 ms; error against FP64 arithmetic 1.8-2.5e-7
-// -> 2.1-2.9e-7 after 19-32 FP32 steps).  16-bit storage runs S0, S12, S12, S3, so that the
-// sum is formed in FP32 from the stored levels and never stored in 16 bits.
+// W + dt (b0 K0 + b1 K1 + b2 K2 + b3 K3); Q's weights are w1 / (1 - w3) = 1/2 and
+// w2 / (1 - w3) = 1.  FP32 and FP64 storage run S0, S1Q, S12, S3Q: Q carries W, U1
+// and U2 into the last stage in one level, 108 instead of 117 level words per
+// point and step, and S3Q reads 9 words at the point where S3 reads 27 (per
+// step, before and after: 400x400x200 Cartesian FP32 5.46 -> 4.96 ms, 64 shots
+// of 100x100x60 12.3 -> 10.7 ms, 128x128x96 curvilinear FP64 1.51 -> 1.26 ms).
+// Q is stored near W, not near (1 - w3) W, and everything added to it is an
+// increment: its rounding reaches W^{n+1} with 1 - w3 = 2/3, the weight that
+// U2's has in S3, and a field with no rates keeps its bits (error against 64
+// bits, Q scaled by (1 - w3) -> this: 400x400x200 1.3 -> 1.1e-7 after 24 FP32
+// steps, 100x100x60 2.7 -> 2.3e-7 after 40, 128x128x96 5.7 -> 5.4e-16 after 24 in
+// FP64; S3 1.3e-7, 2.2e-7).  16-bit storage runs S0, S12, S12, S3, so that the sum
+// is formed in FP32 from the stored levels and never stored in 16 bits.
 // MODE_RHS writes the right-hand side alone (the per-stage operator).
 enum Mode { MODE_RHS = 0, MODE_S0 = 1, MODE_S12 = 2, MODE_S3 = 3, MODE_S1Q = 4, MODE_S3Q = 5 };
 
@@ -145,20 +150,25 @@ template <typename TC> __device__ __forceinline__ TC rk_final(TC y0, TC partial,
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 // S1Q: Q from W, U1 and U2's increment d2 = a1 dt K1 (the increment itself:
-// U2's rounding then stays out of Q).  (1 - w3) W is taken as W - w3 W with the
-// w3 that S3Q adds back, so the 1e-8 by which an FP32 w3 misses 1/3 multiplies
-// U3 - W as it does in S3; a complement rounded on its own drifts twice as fast
-// (2.2e-6 against 1.1e-6, S3 1.2e-6, after 500 FP32 steps of an oscillator).
-template <typename TC> __device__ __forceinline__ void rk_sum(const TC *w, TC y0, TC u1, TC ca, TC h, TC &u2, TC &q) {
+// U2's rounding then stays out of Q).  The weights b_i in FP32 lie 3e-8 above
+// their fractions, all four alike, which S3 and the per-stage sums of the
+// reference carry as a clock that much fast; w[1] = w1 / (1 - w3) / (1/2) - 1 = 4.5e-8
+// lends it to K0 and K1 (without it the DRP coefficients' own -6e-8 stands out: 3.0
+// against 2.4e-7 of the 100x100x60 explosion after 40 steps).  s + e is the
+// exact sum of y0 and t, so Q is rounded once.
+template <typename TC>
+__device__ __forceinline__ void rk_sum(const TC *w, TC y0, TC u1, TC ca, TC h, TC &u2, TC &q) {
 #pragma clang fp contract(off)
   const TC d2 = ca * h;
   u2 = y0 + d2;
-  q = y0 + fma_t(-w[2], y0, fma_t(w[0], u1 - y0, w[1] * d2));
+  const TC t = fma_t(TC(0.5), u1 - y0, d2);
+  const TC s = y0 + t, b = s - y0, e = (y0 - (s - b)) + (t - b);
+  q = s + fma_t(w[1], t, e);
 }
-// S3Q
+// S3Q: the 1e-8 by which an FP32 w3 misses 1/3 multiplies U3 - Q, an increment
 template <typename TC> __device__ __forceinline__ TC rk_end(const TC *w, TC q, TC u3, TC cb, TC h) {
 #pragma clang fp contract(off)
-  return q + fma_t(w[2], u3, cb * h);
+  return q + fma_t(w[2], u3 - q, cb * h);
 }
 
 // ---- operator constants (src/forward/fd_t.cu:76-148) ----------------------
@@ -210,9 +220,12 @@ constexpr int kMaxBox = 26;
 // storage types whose stage kernels add sources from the step's table
 template <typename TS> constexpr bool kBoxedSrc = !St<TS>::scaled;
 
-// Bounding box (physical) of one shot's source points; ni = 0: none.
+// Bounding box (physical) of one shot's source points; ni = 0: none.  The shot's
+// rates of a step are [4 stages][9][nk][nj][ni] from element off of the table.
 struct SrcBox {
   int i0, j0, k0, ni, nj, nk;
+  long off;
+  __host__ __device__ __forceinline__ int vol() const { return ni * nj * nk; }
 };
 
 template <typename TS, typename TM> struct StageArgs {
@@ -231,7 +244,7 @@ template <typename TS, typename TM> struct StageArgs {
   long shot_stride;
   int mode;
   TM ca, cb;      // a_i dt and b_i dt of the stage
-  TM rk_w[3];     // w1, w2, w3 of the last stage's combination
+  TM rk_w[3];     // w1, w2, w3 of the last stage's combination (S1Q, S3Q: see rk_sum)
   float sc[kNC], isc[kNC];  // storage scale (value = stored*sc) and its inverse
   int nbox;
   int box[kMaxBox][6];      // i1,i2,j1,j2,k1,k2 inclusive, physical
@@ -241,14 +254,16 @@ template <typename TS, typename TM> struct StageArgs {
   // right-hand side where it is formed (null: sources come from k_source, and
   // always with 16-bit storage, whose outputs are rounded before the source).
   const SrcBox *sbox;       // [nshots]
-  const TM *src_v;          // shot 0's rates of this stage, [9][src_vol]
-  long src_vol;             // points reserved per box; a shot's stages are 4*9*src_vol apart
+  const TM *src_v;          // the table (SrcBox::off)
+  int istage;
 };
 
-// Source contributions grouped by grid point (CSR), all shots of a session.
+// Source contributions grouped by grid point (CSR), all shots of a session: the
+// points of shots with a box first.
 template <typename TS, typename TM> struct SrcArgs {
   Layout L;
-  int npt;
+  int npt, npt_box;         // points; those of shots with a box
+  int p0;                   // first point k_source takes
   const int *pt_shot;       // [npt]
   const long *pt_off;       // [npt] layout offset
   const int *pt_beg;        // [npt+1] into contributions
@@ -266,16 +281,15 @@ template <typename TS, typename TM> struct SrcArgs {
   long shot_stride;
   int mode, istage;
   TM ca, cb;
-  TM w2;               // U2's weight in Q (S1Q)
   const int *clock;         // current global step
   const int *shot_start;    // per-shot start step
   const int *shot_active;
   int only_shot;            // >= 0: inject this shot only, at step fixed_it
   int fixed_it;
   float isc[kNC];
-  const int *pt_cell;       // [npt] cell in the shot's box
-  TM *src_v;                // [nshots][4][9][src_vol] rates of a step tabulated by k_step_head, or null
-  long src_vol;
+  const int *pt_cell;       // [npt_box] cell in the shot's box
+  const SrcBox *sbox;       // [nshots]
+  TM *src_v;                // rates of a step tabulated by k_step_head (SrcBox::off), or null
 };
 
 template <typename TS, typename TC> struct RecvArgs {
