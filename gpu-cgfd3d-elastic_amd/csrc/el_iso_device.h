@@ -220,12 +220,9 @@ constexpr int kMaxBox = 26;
 // storage types whose stage kernels add sources from the step's table
 template <typename TS> constexpr bool kBoxedSrc = !St<TS>::scaled;
 
-// Bounding box (physical) of one shot's source points; ni = 0: none.  The shot's
-// rates of a step are [4 stages][9][nk][nj][ni] from element off of the table.
+// Bounding box (physical) of one shot's source points; ni = 0: none.
 struct SrcBox {
   int i0, j0, k0, ni, nj, nk;
-  long off;
-  __host__ __device__ __forceinline__ int vol() const { return ni * nj * nk; }
 };
 
 template <typename TS, typename TM> struct StageArgs {
@@ -254,16 +251,14 @@ template <typename TS, typename TM> struct StageArgs {
   // right-hand side where it is formed (null: sources come from k_source, and
   // always with 16-bit storage, whose outputs are rounded before the source).
   const SrcBox *sbox;       // [nshots]
-  const TM *src_v;          // the table (SrcBox::off)
-  int istage;
+  const TM *src_v;          // shot 0's rates of this stage, [9][src_vol]
+  long src_vol;             // points reserved per box; a shot's stages are 4*9*src_vol apart
 };
 
-// Source contributions grouped by grid point (CSR), all shots of a session: the
-// points of shots with a box first.
+// Source contributions grouped by grid point (CSR), all shots of a session.
 template <typename TS, typename TM> struct SrcArgs {
   Layout L;
-  int npt, npt_box;         // points; those of shots with a box
-  int p0;                   // first point k_source takes
+  int npt;
   const int *pt_shot;       // [npt]
   const long *pt_off;       // [npt] layout offset
   const int *pt_beg;        // [npt+1] into contributions
@@ -287,9 +282,9 @@ template <typename TS, typename TM> struct SrcArgs {
   int only_shot;            // >= 0: inject this shot only, at step fixed_it
   int fixed_it;
   float isc[kNC];
-  const int *pt_cell;       // [npt_box] cell in the shot's box
-  const SrcBox *sbox;       // [nshots]
-  TM *src_v;                // rates of a step tabulated by k_step_head (SrcBox::off), or null
+  const int *pt_cell;       // [npt] cell in the shot's box
+  TM *src_v;                // [nshots][4][9][src_vol] rates of a step tabulated by k_step_head, or null
+  long src_vol;
 };
 
 template <typename TS, typename TC> struct RecvArgs {
