@@ -168,14 +168,14 @@ struct cgfd_session {
   long *s_pt_off = nullptr, *s_tab = nullptr;
   void *s_ct_coef = nullptr, *s_F = nullptr, *s_M = nullptr;
   long s_ntab = 0;
-  // Source boxes (src_boxed): every shot's points lie in a box of at most
-  // kMaxSrcBox physical points, and the stages add the rates that the step's
-  // head tabulates over it.  Otherwise k_source follows each stage.
-  bool src_boxed = false;
-  long s_vol = 0;               // points reserved per box
+  // Source boxes: where a shot's points lie in a box of at most kMaxSrcBox
+  // physical points, the stages add the rates that the step's head tabulates
+  // over it; k_source follows each stage for the points of the other shots.
+  // Each shot goes by its own points: its roundings do not depend on its batch.
+  int s_npt_box = 0;            // points of shots with a box (the first of s_npt)
   int *s_pt_cell = nullptr;
   SrcBox *s_box = nullptr;
-  void *s_v = nullptr;          // [nshots][4][9][s_vol]
+  void *s_v = nullptr;          // the rates (SrcBox::off)
   bool src_dirty = false;
   // device receivers
   int r_n = 0;
@@ -500,53 +500,60 @@ template <typename TM> int build_sources(cgfd_session *s) {
   }
   const int npt = (int)pts.size();
   s->s_ntab = ntab;
-  s->src_boxed = false;
+  s->s_npt_box = 0;
   invalidate(s);
   if (npt == 0) { s->src_dirty = false; return CGFD_OK; }
-  // boxes over the shots' points; a point in the ghosts (accepted by the
-  // upload, never updated by a stage) rules them out
+  // a box over each shot's points; a point in the ghosts (accepted by the
+  // upload, never updated by a stage) rules its shot out
   const Layout &L = s->L;
   auto ijk = [&](long off, int *q) {
     q[2] = (int)(off / L.pz) - kNG;
     q[1] = (int)(off % L.pz / L.px) - kNG;
     q[0] = (int)(off % L.px) - L.xa;
   };
-  std::vector<SrcBox> box(s->d.nshots, SrcBox{0, 0, 0, 0, 0, 0});
-  bool boxed = true;
-  long vol = 0;
+  std::vector<SrcBox> box(s->d.nshots, SrcBox{0, 0, 0, 0, 0, 0, 0});
+  std::vector<char> wide(s->d.nshots, 0);
   for (auto &kv : pts) {
+    const int shot = kv.first.first;
+    if (wide[shot]) continue;
     int q[3];
     ijk(kv.first.second, q);
-    if (q[0] < 0 || q[1] < 0 || q[2] < 0 || q[0] >= L.ni || q[1] >= L.nj || q[2] >= L.nk) { boxed = false; break; }
-    SrcBox &b = box[kv.first.first];
-    if (b.ni == 0) { b = SrcBox{q[0], q[1], q[2], 1, 1, 1}; }
+    SrcBox &b = box[shot];
+    if (b.ni == 0) b = SrcBox{q[0], q[1], q[2], 1, 1, 1, 0};
     int *lo[3] = {&b.i0, &b.j0, &b.k0}, *n[3] = {&b.ni, &b.nj, &b.nk};
     for (int d = 0; d < 3; d++) {
       const int hi = std::max(*lo[d] + *n[d] - 1, q[d]);
       *lo[d] = std::min(*lo[d], q[d]);
       *n[d] = hi - *lo[d] + 1;
     }
-    const long v = (long)b.ni * b.nj * b.nk;
-    if (v > kMaxSrcBox) { boxed = false; break; }
-    vol = std::max(vol, v);
-  }
-  std::vector<int> pt_cell;
-  if (boxed)
-    for (auto &kv : pts) {
-      int q[3];
-      ijk(kv.first.second, q);
-      const SrcBox &b = box[kv.first.first];
-      pt_cell.push_back(((q[2] - b.k0) * b.nj + (q[1] - b.j0)) * b.ni + (q[0] - b.i0));
+    if (q[0] < 0 || q[1] < 0 || q[2] < 0 || q[0] >= L.ni || q[1] >= L.nj || q[2] >= L.nk ||
+        (long)b.ni * b.nj * b.nk > kMaxSrcBox) {
+      wide[shot] = 1;
+      b = SrcBox{0, 0, 0, 0, 0, 0, 0};
     }
-  std::vector<int> pt_shot, pt_beg, ct_src;
+  }
+  long table = 0;
+  for (SrcBox &b : box) {
+    b.off = table;
+    table += 4L * kNC * b.vol();
+  }
+  std::vector<int> pt_shot, pt_beg, ct_src, pt_cell;
   std::vector<long> pt_off;
   std::vector<TM> ct_coef;
-  for (auto &kv : pts) {
-    pt_shot.push_back(kv.first.first);
-    pt_off.push_back(kv.first.second);
-    pt_beg.push_back((int)ct_src.size());
-    for (auto &c : kv.second) { ct_src.push_back(c.first); ct_coef.push_back((TM)c.second); }
-  }
+  for (int pass = 0; pass < 2; pass++)
+    for (auto &kv : pts) {
+      const int shot = kv.first.first;
+      if (wide[shot] != pass) continue;
+      pt_shot.push_back(shot);
+      pt_off.push_back(kv.first.second);
+      pt_beg.push_back((int)ct_src.size());
+      for (auto &c : kv.second) { ct_src.push_back(c.first); ct_coef.push_back((TM)c.second); }
+      if (wide[shot]) continue;
+      int q[3];
+      ijk(kv.first.second, q);
+      const SrcBox &b = box[shot];
+      pt_cell.push_back(((q[2] - b.k0) * b.nj + (q[1] - b.j0)) * b.ni + (q[0] - b.i0));
+    }
   pt_beg.push_back((int)ct_src.size());
   int slot = 0;
   auto up = [&](void **dst, const void *src, size_t bytes) -> int {
@@ -570,15 +577,13 @@ template <typename TM> int build_sources(cgfd_session *s) {
   for (int c = 0; c < 6; c++) Mall.insert(Mall.end(), M[c].begin(), M[c].end());
   if ((r = up(&s->s_F, Fall.data(), Fall.size() * sizeof(TM)))) return r;
   if ((r = up(&s->s_M, Mall.data(), Mall.size() * sizeof(TM)))) return r;
-  if (boxed) {
+  if (table > 0) {
     if ((r = up((void **)&s->s_pt_cell, pt_cell.data(), pt_cell.size() * 4))) return r;
     if ((r = up((void **)&s->s_box, box.data(), box.size() * sizeof(SrcBox)))) return r;
     // cells of a box that no point fills stay zero
-    const size_t nv = (size_t)s->d.nshots * 4 * kNC * vol;
-    if ((r = ensure(s, &s->s_v, &s->s_cap[slot++], nv * sizeof(TM)))) return r;
-    if ((r = fill_zero(s, s->s_v, nv, sizeof(TM)))) return r;
-    s->s_vol = vol;
-    s->src_boxed = true;
+    if ((r = ensure(s, &s->s_v, &s->s_cap[slot++], (size_t)table * sizeof(TM)))) return r;
+    if ((r = fill_zero(s, s->s_v, (size_t)table, sizeof(TM)))) return r;
+    s->s_npt_box = (int)pt_cell.size();
   }
   s->s_npt = npt;
   s->src_dirty = false;
@@ -1093,16 +1098,16 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
 }
 
 // Arguments of the source kernels; the stage's outputs and weights are set by
-// the caller.  table: rates tabulated over the boxes (needs src_boxed).
+// the caller.  table: with the rates tabulated over the boxes.
 template <typename TS, typename TC> SrcArgs<TS, TC> source_args(cgfd_session *s, bool table) {
   SrcArgs<TS, TC> sa{};
-  sa.L = s->L; sa.npt = s->s_npt; sa.pt_shot = s->s_pt_shot; sa.pt_off = s->s_pt_off; sa.pt_beg = s->s_pt_beg;
+  sa.L = s->L; sa.npt = s->s_npt; sa.npt_box = s->s_npt_box; sa.pt_shot = s->s_pt_shot; sa.pt_off = s->s_pt_off; sa.pt_beg = s->s_pt_beg;
   sa.ct_src = s->s_ct_src; sa.ct_coef = (const TC *)s->s_ct_coef; sa.s_itb = s->s_itb; sa.s_ite = s->s_ite;
   sa.s_tab = s->s_tab; sa.s_kind = s->s_kind; sa.F = (const TC *)s->s_F; sa.M = (const TC *)s->s_M;
   sa.ntab = s->s_ntab; sa.met = (const TC *)s->met; sa.med = (const TC *)s->med;
   sa.shot_start = s->shot_start; sa.shot_active = s->shot_active;
   sa.only_shot = -1;
-  if (table) { sa.pt_cell = s->s_pt_cell; sa.src_v = (TC *)s->s_v; sa.src_vol = s->s_vol; }
+  if (table) { sa.pt_cell = s->s_pt_cell; sa.sbox = s->s_box; sa.src_v = (TC *)s->s_v; }
   for (int c = 0; c < kNC; c++) sa.isc[c] = s->isc[c];
   return sa;
 }
@@ -1113,7 +1118,9 @@ template <typename TS, typename TC> SrcArgs<TS, TC> source_args(cgfd_session *s,
 // W^{n+1} swap.
 template <typename TS, typename TC>
 int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, bool timed) {
-  const bool boxed = s->s_npt > 0 && s->src_boxed;
+  const bool boxed = s->s_npt > 0 && s->s_npt_box > 0;
+  // k_source takes the points that the stages do not
+  const int src_p0 = kBoxedSrc<TS> ? s->s_npt_box : 0;
   for (int n = 0; n < nsteps; n++) {
     const int it = it0 + n;
     const int *clock = s->clock + (it & 1);
@@ -1143,8 +1150,8 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
       a.cb = (TC)kRkB[istage] * dt;
       if (boxed && kBoxedSrc<TS>) {
         a.sbox = s->s_box;
-        a.src_v = (const TC *)s->s_v + (long)istage * kNC * s->s_vol;
-        a.src_vol = s->s_vol;
+        a.src_v = (const TC *)s->s_v;
+        a.istage = istage;
       }
       const bool tim = timed && sh.inner.nbox;
       if (tim && s->ev.size() < s->ev_used + 2) {
@@ -1155,8 +1162,9 @@ int enqueue_steps(cgfd_session *s, const Shell &sh, int it0, int nsteps, TC dt, 
                                    tim ? s->ev[s->ev_used + 1] : nullptr);
       if (r) return r;
       if (tim) s->ev_used += 2;
-      if (s->s_npt > 0 && !(boxed && kBoxedSrc<TS>)) {
+      if (s->s_npt > src_p0) {
         SrcArgs<TS, TC> sa = source_args<TS, TC>(s, boxed);
+        sa.p0 = src_p0;
         sa.w_out = a.w_out; sa.w_end = a.w_end; sa.shot_stride = s->shot_elems;
         sa.mode = p.mode; sa.istage = istage; sa.ca = a.ca; sa.cb = a.cb;
         sa.clock = clock;

@@ -220,9 +220,12 @@ constexpr int kMaxBox = 26;
 // storage types whose stage kernels add sources from the step's table
 template <typename TS> constexpr bool kBoxedSrc = !St<TS>::scaled;
 
-// Bounding box (physical) of one shot's source points; ni = 0: none.
+// Bounding box (physical) of one shot's source points; ni = 0: none.  The shot's
+// rates of a step are [4 stages][9][nk][nj][ni] from element off of the table.
 struct SrcBox {
   int i0, j0, k0, ni, nj, nk;
+  long off;
+  __host__ __device__ __forceinline__ int vol() const { return ni * nj * nk; }
 };
 
 template <typename TS, typename TM> struct StageArgs {
@@ -251,14 +254,16 @@ template <typename TS, typename TM> struct StageArgs {
   // right-hand side where it is formed (null: sources come from k_source, and
   // always with 16-bit storage, whose outputs are rounded before the source).
   const SrcBox *sbox;       // [nshots]
-  const TM *src_v;          // shot 0's rates of this stage, [9][src_vol]
-  long src_vol;             // points reserved per box; a shot's stages are 4*9*src_vol apart
+  const TM *src_v;          // the table (SrcBox::off)
+  int istage;
 };
 
-// Source contributions grouped by grid point (CSR), all shots of a session.
+// Source contributions grouped by grid point (CSR), all shots of a session: the
+// points of shots with a box first.
 template <typename TS, typename TM> struct SrcArgs {
   Layout L;
-  int npt;
+  int npt, npt_box;         // points; those of shots with a box
+  int p0;                   // first point k_source takes
   const int *pt_shot;       // [npt]
   const long *pt_off;       // [npt] layout offset
   const int *pt_beg;        // [npt+1] into contributions
@@ -282,9 +287,9 @@ template <typename TS, typename TM> struct SrcArgs {
   int only_shot;            // >= 0: inject this shot only, at step fixed_it
   int fixed_it;
   float isc[kNC];
-  const int *pt_cell;       // [npt] cell in the shot's box
-  TM *src_v;                // [nshots][4][9][src_vol] rates of a step tabulated by k_step_head, or null
-  long src_vol;
+  const int *pt_cell;       // [npt_box] cell in the shot's box
+  const SrcBox *sbox;       // [nshots]
+  TM *src_v;                // rates of a step tabulated by k_step_head (SrcBox::off), or null
 };
 
 template <typename TS, typename TC> struct RecvArgs {

@@ -23,9 +23,10 @@ __device__ __forceinline__ void src_add(const StageArgs<TS, TC> &a, int shot, in
   const SrcBox b = a.sbox[shot];
   const int di = i - b.i0, dj = j - b.j0, dk = k - b.k0;
   if ((unsigned)di >= (unsigned)b.ni || (unsigned)dj >= (unsigned)b.nj || (unsigned)dk >= (unsigned)b.nk) return;
-  const TC *v = a.src_v + (long)shot * (4 * kNC) * a.src_vol + ((dk * b.nj + dj) * b.ni + di);
+  const int vol = b.vol();
+  const TC *v = a.src_v + b.off + a.istage * kNC * vol + ((dk * b.nj + dj) * b.ni + di);
 #pragma unroll
-  for (int c = 0; c < kNC; c++) h[c] += v[c * a.src_vol];
+  for (int c = 0; c < kNC; c++) h[c] += v[c * vol];
 }
 
 // One face fi (its box must contain the point): Dd are the raw derivatives

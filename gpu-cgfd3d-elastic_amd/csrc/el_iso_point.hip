@@ -111,11 +111,11 @@ __device__ __forceinline__ bool src_rate(const SrcArgs<TS, TC> &a, int p, int it
 // One thread per distinct grid point; the rates, from the step's table where
 // there is one (10.8 -> 8.7 us on a single moment source: the contributions
 // are a chain of dependent loads), are applied to the RK outputs of this stage.  Serves 16-bit storage,
-// the bare right-hand side and sources that spread too far for a box (see
+// the bare right-hand side and shots whose sources spread too far for a box (see
 // k_step_head).
 template <typename TS, typename TC>
 __global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  const int p = a.p0 + blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= a.npt) return;
   const int shot = a.pt_shot[p];
   if (a.only_shot >= 0 && shot != a.only_shot) return;
@@ -124,10 +124,11 @@ __global__ __launch_bounds__(256) void k_source(SrcArgs<TS, TC> a) {
   const long o = a.pt_off[p];
   const long cs = a.L.cs;
   TC v[kNC];
-  if (a.src_v) {
-    const TC *r = a.src_v + ((long)shot * 4 + a.istage) * kNC * a.src_vol + a.pt_cell[p];
+  if (a.src_v && p < a.npt_box) {
+    const int vol = a.sbox[shot].vol();
+    const TC *r = a.src_v + a.sbox[shot].off + a.istage * kNC * vol + a.pt_cell[p];
 #pragma unroll
-    for (int c = 0; c < kNC; c++) v[c] = r[c * a.src_vol];
+    for (int c = 0; c < kNC; c++) v[c] = r[c * vol];
   } else if (!src_rate(a, p, it, a.istage, v)) {
     return;
   }
@@ -196,15 +197,16 @@ __global__ __launch_bounds__(256) void k_step_head(RecvArgs<TS, TC> r, SrcArgs<T
     return;
   }
   const int t = (blockIdx.x - recv_blocks) * blockDim.x + threadIdx.x;
-  if (!s.src_v || t >= 4 * s.npt) return;
+  if (!s.src_v || t >= 4 * s.npt_box) return;
   const int p = t >> 2, istage = t & 3;
   const int shot = s.pt_shot[p];
   if (!s.shot_active[shot]) return;
   TC v[kNC];
   src_rate(s, p, now - s.shot_start[shot], istage, v);
-  TC *out = s.src_v + ((long)shot * 4 + istage) * kNC * s.src_vol + s.pt_cell[p];
+  const int vol = s.sbox[shot].vol();
+  TC *out = s.src_v + s.sbox[shot].off + istage * kNC * vol + s.pt_cell[p];
 #pragma unroll
-  for (int c = 0; c < kNC; c++) out[c * s.src_vol] = v[c];
+  for (int c = 0; c < kNC; c++) out[c * vol] = v[c];
 }
 
 template <typename T> __global__ __launch_bounds__(256) void k_fill(T *p, long n, T v) {
@@ -349,15 +351,15 @@ hipError_t launch_surface(const StageArgs<TS, TC> &a, int dx, int dy, int dz, in
 }
 
 template <typename TS, typename TC> hipError_t launch_source(const SrcArgs<TS, TC> &a, hipStream_t st) {
-  if (a.npt == 0) return hipSuccess;
-  hipLaunchKernelGGL((k_source<TS, TC>), dim3((a.npt + 255) / 256), dim3(256), 0, st, a);
+  if (a.npt <= a.p0) return hipSuccess;
+  hipLaunchKernelGGL((k_source<TS, TC>), dim3((a.npt - a.p0 + 255) / 256), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
 template <typename TS, typename TC>
 hipError_t launch_step_head(const RecvArgs<TS, TC> &r, const SrcArgs<TS, TC> &s, const int *clock, int *clock_next,
                             hipStream_t st) {
-  const int rb = (r.nrec * kNC + 255) / 256, sb = s.src_v ? (4 * s.npt + 255) / 256 : 0;
+  const int rb = (r.nrec * kNC + 255) / 256, sb = s.src_v ? (4 * s.npt_box + 255) / 256 : 0;
   hipLaunchKernelGGL((k_step_head<TS, TC>), dim3(rb + sb > 0 ? rb + sb : 1), dim3(256), 0, st, r, s, clock, clock_next,
                      rb);
   return hipGetLastError();
