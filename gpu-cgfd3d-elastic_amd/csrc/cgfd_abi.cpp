@@ -152,7 +152,8 @@ struct cgfd_session {
   void *rhs = nullptr;     // nshots x 1 level (lazy)
   void *met = nullptr, *med = nullptr, *mat = nullptr;
   bool have_met = false, have_med = false;
-  int met_class = MET_ALL;  // MetClass of the uploaded metric
+  int met_class = MET_ALL;   // MetClass of the uploaded metric as the sweeps take it
+  int surf_class = MET_ALL;  // and as the free-surface rows do
   double cmet[9] = {0};
   int free_top = 0;
   FaceHost face[6];
@@ -388,6 +389,28 @@ int get_storage(cgfd_session *s, const void *src, size_t n, long comp_stride, st
     }
   }
   return CGFD_OK;
+}
+
+// Whether a metric component stays within two tolerances of its first value
+// and, off the diagonal, that within them of zero (NaN: neither).
+struct Spread {
+  bool loose, strict;
+};
+template <typename T> Spread spread(const T *v, size_t n, bool diag, double loose, double strict) {
+  const double v0 = (double)v[0], z = diag ? 0.0 : std::fabs(v0);
+  Spread r{z <= loose, z <= strict};
+  for (size_t q = 0; q < n && r.loose; q += 4096) {
+    const size_t m = std::min<size_t>(4096, n - q);
+    int far = 0, off = 0;
+    for (size_t p = 0; p < m; p++) {
+      const double d = std::fabs((double)v[q + p] - v0);
+      far |= !(d <= loose);
+      off |= !(d <= strict);
+    }
+    if (far) r.loose = false;
+    if (far || off) r.strict = false;
+  }
+  return r;
 }
 
 void *wav_level(cgfd_session *s, int shot, int slot) {
@@ -701,6 +724,7 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
   a.mat = (const TC *)s->mat;
   a.free_top = s->free_top;
   a.met_class = s->met_class;
+  a.surf_class = s->surf_class;
   for (int c = 0; c < 9; c++) a.cmet[c] = (TC)s->cmet[c];
   const long aux_lvl_shot = 5;
   for (int f = 0; f < 6; f++) {
@@ -815,7 +839,8 @@ Shell make_shell(cgfd_session *s, bool rhs = false) {
   sh.rim.pml = 1;
   // who takes the surface rows next to a whole-plane sweep
   const bool tiles = s->es >= 4;
-  const bool fuse = s->free_top && tiles && s->fuse && !rhs && sh.inner.shape == kSurfShape;
+  const bool fuse = s->free_top && tiles && s->fuse && !rhs && sh.inner.shape == kSurfShape &&
+                    s->surf_class == s->met_class;
   auto surface_rows = [&]() {
     sh.surface = s->free_top && tiles;
     if (!tiles) sh.point.add(0, ni - 1, 0, nj - 1, ktopm + 1, nk - 1);
@@ -904,12 +929,13 @@ int launch_stage(cgfd_session *s, const Shell &sh, StageArgs<TS, TC> &a, int dx,
 // Results are cached per (grid, storage, shots, flags, metric form, PML layout,
 // pinned split) for the life of the process.
 struct TileKey {
-  int ni, nj, nk, storage, nshots, flags, met_class, free_top;
+  int ni, nj, nk, storage, nshots, flags, met_class, surf_class, free_top;
   std::array<int, 6> nlay;  // PML layers per face (0: none)
   int pinned;               // split pinned by cgfd_set_split, -1: automatic
   bool operator<(const TileKey &o) const {
-    return std::tie(ni, nj, nk, storage, nshots, flags, met_class, free_top, nlay, pinned) <
-           std::tie(o.ni, o.nj, o.nk, o.storage, o.nshots, o.flags, o.met_class, o.free_top, o.nlay, o.pinned);
+    return std::tie(ni, nj, nk, storage, nshots, flags, met_class, surf_class, free_top, nlay, pinned) <
+           std::tie(o.ni, o.nj, o.nk, o.storage, o.nshots, o.flags, o.met_class, o.surf_class, o.free_top, o.nlay,
+                    o.pinned);
   }
 };
 struct TileChoice {
@@ -932,8 +958,8 @@ long march_workgroups(const MarchSet &m, int zchunk) {
 }
 
 template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
-  TileKey key{s->d.ni, s->d.nj, s->d.nk, s->d.storage, s->d.nshots, s->d.flags, s->met_class, s->free_top,
-              {}, s->split_fixed ? s->split : -1};
+  TileKey key{s->d.ni, s->d.nj, s->d.nk, s->d.storage, s->d.nshots, s->d.flags, s->met_class, s->surf_class,
+              s->free_top, {}, s->split_fixed ? s->split : -1};
   for (int f = 0; f < 6; f++) key.nlay[f] = s->face[f].on ? s->face[f].nlay : 0;
   {
     std::lock_guard<std::mutex> lk(g_tile_mu);
@@ -1457,36 +1483,37 @@ int cgfd_upload_metric(cgfd_session *s, int dtype, const void *metric) {
   // largest metric magnitude of its first value and the off-diagonal ones
   // within that of zero; the sweep then takes the first point's diagonal
   // values as arguments and the off-diagonal ones as 0 (a change below
-  // 1e-10 relative in any derivative, far under FP32 rounding).  A grid of
-  // evenly spaced vertical lines passes the same test on its xi and eta rows
-  // alone (within 1e-12 in FP64 sessions, whose arithmetic would see more).  A
-  // uniform but sheared grid keeps the per-point arrays, as does
-  // CGFD_FLAG_FULL_METRIC.
+  // 1e-10 relative in any derivative, far under FP32 rounding).  Whether the
+  // free-surface rows drop components too, and whether a grid of evenly spaced
+  // vertical lines drops its xi and eta rows, goes by what the session's
+  // arithmetic rounds anyway: 1e-10 of the row's own diagonal term in FP32, four
+  // roundings of it in FP64 (noise of 5e-14, as computed metrics have it, keeps
+  // the arrays there: dropped, it is 100 times FP64's error); a grid that is
+  // Cartesian by the first test alone keeps them in its surface rows.  A uniform
+  // but sheared grid keeps the per-point arrays, as does CGFD_FLAG_FULL_METRIC.
   const size_t n = (size_t)(s->d.ni + 6) * (s->d.nj + 6) * (s->d.nk + 6);
   double scale = 0.0;
   for (int c = 0; c < 9; c++) scale = std::max(scale, std::fabs(rd(dtype, metric, (size_t)(c + 1) * n)));
-  // component c is its first value (diagonal) or zero (off-diagonal) everywhere, within tol
-  auto fixed = [&](int c, double tol) {
-    const bool diag = c % 4 == 0;  // xi_x, eta_y, zeta_z
-    const double v0 = rd(dtype, metric, (size_t)(c + 1) * n);
-    if (!diag && !(std::fabs(v0) <= tol)) return false;
-    for (size_t q = 1; q < n; q++)
-      if (!(std::fabs(rd(dtype, metric, (size_t)(c + 1) * n + q) - v0) <= tol)) return false;
-    s->cmet[c] = diag ? v0 : 0.0;
-    return true;
-  };
-  s->met_class = MET_ALL;
+  s->met_class = s->surf_class = MET_ALL;
   if (!(s->d.flags & CGFD_FLAG_FULL_METRIC) && scale > 0.0) {
-    int c = 0;
-    while (c < 9 && fixed(c, 1e-10 * scale)) c++;
-    if (c == 9) {
-      s->met_class = MET_CONST;
-    } else {
-      const double tol = (s->ms == 8 ? 1e-12 : 1e-10) * scale;
-      c = 0;
-      while (c < 6 && fixed(c, tol)) c++;
-      if (c == 6) s->met_class = MET_VERT;
+    // components (in order) within the loose and the strict tolerance of their
+    // first value (diagonal: xi_x, eta_y, zeta_z) or of zero (off-diagonal)
+    const double tol = 1e-10 * scale, rel = s->ms == 8 ? 4 * 2.220446049250313e-16 : 1e-10;
+    int loose = 0, strict = 0;
+    for (int c = 0; c < 9 && loose == c; c++) {
+      const double v0 = rd(dtype, metric, (size_t)(c + 1) * n);
+      const double diag = rd(dtype, metric, (size_t)(c / 3 * 4 + 1) * n);
+      const double tight = rel * std::fabs(diag);
+      const Spread d = dtype == CGFD_DT_F64 ? spread((const double *)metric + (c + 1) * n, n, c % 4 == 0, tol, tight)
+                                            : spread((const float *)metric + (c + 1) * n, n, c % 4 == 0, tol, tight);
+      if (!d.loose) break;
+      s->cmet[c] = c % 4 == 0 ? v0 : 0.0;
+      loose++;
+      if (strict == c && d.strict) strict++;
     }
+    const int vert = strict >= 6 ? MET_VERT : MET_ALL;
+    s->met_class = loose == 9 ? (int)MET_CONST : vert;
+    s->surf_class = strict == 9 ? (int)MET_CONST : loose == 9 ? (int)MET_ALL : vert;
   }
   invalidate(s);
   return CGFD_OK;

@@ -234,7 +234,8 @@ template <typename TS, typename TM> struct StageArgs {
   const TM *med;   // lam, mu, 1/rho, stride L.cs
   const TM *mat;   // 18 components [c][j][i] on the physical top plane
   int free_top;
-  int met_class;   // MetClass of the uploaded metric
+  int met_class;   // MetClass of the uploaded metric (sweeps)
+  int surf_class;  // the same for the free-surface rows
   TM cmet[9];      // xi_x..zeta_z where the class makes them constant (the zero ones exactly 0)
   FaceArgs<TS, TM> f[6];
   // shot-0 level bases: stage input, W^n, output, the last stage's level (S1Q

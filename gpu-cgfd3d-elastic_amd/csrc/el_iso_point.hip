@@ -343,8 +343,8 @@ hipError_t launch_surface(const StageArgs<TS, TC> &a, int dx, int dy, int dz, in
     with_mode<TS>(a.mode, [&](auto m) {
       constexpr int M = decltype(m)::value;
       const int sel = dx * 4 + dy * 2 + dz;
-      if (a.met_class == MET_CONST) launch_surface_m<M, MET_CONST>(a, grid, ntx, nty, sel, st);
-      else if (a.met_class == MET_VERT) launch_surface_m<M, MET_VERT>(a, grid, ntx, nty, sel, st);
+      if (a.surf_class == MET_CONST) launch_surface_m<M, MET_CONST>(a, grid, ntx, nty, sel, st);
+      else if (a.surf_class == MET_VERT) launch_surface_m<M, MET_VERT>(a, grid, ntx, nty, sel, st);
       else launch_surface_m<M, MET_ALL>(a, grid, ntx, nty, sel, st);
     });
   return hipGetLastError();
