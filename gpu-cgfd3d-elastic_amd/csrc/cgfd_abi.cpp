@@ -1940,6 +1940,7 @@ int cgfd_set_tile(cgfd_session *s, int shape, int zchunk) {
   }
   if (shape >= kNumShapes || zchunk < 1) return fail(CGFD_E_ARG, "tile %d/%d invalid", shape, zchunk);
   s->tile_fixed = true;
+  s->fuse = true;
   s->tile_shape = shape;
   s->tile_zchunk = zchunk;
   if (!s->split_fixed) s->split = CGFD_SPLIT_PLANES;
@@ -1950,6 +1951,7 @@ int cgfd_set_split(cgfd_session *s, int split) {
   if (!s) return fail(CGFD_E_ARG, "null session");
   if (split > CGFD_SPLIT_CORE) return fail(CGFD_E_ARG, "work split %d invalid", split);
   invalidate(s);
+  s->fuse = true;
   s->split_fixed = split >= 0;
   s->split = split >= 0 ? split : CGFD_SPLIT_PLANES;
   if (!s->tile_fixed) s->tile_shape = -1;  // tune the tile again (under the pinned split)

@@ -146,11 +146,15 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
       h[VX + cc] = (DxTx + DyTy + DzTz) * slwjac;
     }
   } else if constexpr (!ALL) {
+    // here and in the stresses below the roundings are spelled out: the rows ride
+    // with the sweep or have a launch of their own, and the compiler fuses other
+    // products of a sum in one kernel than in the other
+#pragma clang fp contract(off)
     constexpr int T1[3] = {TXX, TXY, TXZ}, T2[3] = {TXY, TYY, TYZ}, T3[3] = {TXZ, TYZ, TZZ};
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      TC s = xix * Dx[T1[c]] + ety * Dy[T2[c]] + ztz * Dz[T3[c]];
-      if constexpr (!CST) s += ztx * Dz[T1[c]] + zty * Dz[T2[c]];
+      TC s = fma_t(xix, Dx[T1[c]], fma_t(ety, Dy[T2[c]], ztz * Dz[T3[c]]));
+      if constexpr (!CST) s = fma_t(ztx, Dz[T1[c]], fma_t(zty, Dz[T2[c]], s));
       h[c] = slw * s;
     }
   } else {
@@ -195,24 +199,23 @@ __device__ __forceinline__ void point_update(const StageArgs<TS, TC> &a, int sho
     }
   }
   if constexpr (!ALL) {
+#pragma clang fp contract(off)
     const TC DzV[3] = {DzVx, DzVy, DzVz};
-    TC G[3][3];  // G[c][b] = dV_c / dx_b
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      G[c][0] = xix * Dx[c];
-      G[c][1] = ety * Dy[c];
-      G[c][2] = ztz * DzV[c];
+    // s + dV_c / dx_b
+    auto add = [&](TC s, int c, int b) -> TC {
+      s = b == 0 ? fma_t(xix, Dx[c], s) : b == 1 ? fma_t(ety, Dy[c], s) : fma_t(ztz, DzV[c], s);
       if constexpr (!CST) {
-        G[c][0] += ztx * DzV[c];
-        G[c][1] += zty * DzV[c];
+        if (b < 2) s = fma_t(b == 0 ? ztx : zty, DzV[c], s);
       }
-    }
-    h[TXX] = lam2mu * G[0][0] + lam * (G[1][1] + G[2][2]);
-    h[TYY] = lam2mu * G[1][1] + lam * (G[0][0] + G[2][2]);
-    h[TZZ] = lam2mu * G[2][2] + lam * (G[0][0] + G[1][1]);
-    h[TXY] = mu * (G[0][1] + G[1][0]);
-    h[TXZ] = mu * (G[0][2] + G[2][0]);
-    h[TYZ] = mu * (G[1][2] + G[2][1]);
+      return s;
+    };
+    const TC g0 = add(TC(0), 0, 0), g1 = add(TC(0), 1, 1), g2 = ztz * DzV[2];
+    h[TXX] = fma_t(lam2mu, g0, lam * add(g2, 1, 1));
+    h[TYY] = fma_t(lam2mu, g1, lam * add(g2, 0, 0));
+    h[TZZ] = fma_t(lam2mu, g2, lam * add(g1, 0, 0));
+    h[TXY] = mu * add(add(TC(0), 1, 0), 0, 1);
+    h[TXZ] = mu * add(add(TC(0), 2, 0), 0, 2);
+    h[TYZ] = mu * add(add(TC(0), 2, 1), 1, 2);
   } else {
     h[TXX] = lam2mu * (xix * Dx[VX] + etx * Dy[VX] + ztx * DzVx) +
              lam * (xiy * Dx[VY] + ety * Dy[VY] + zty * DzVy + xiz * Dx[VZ] + etz * Dy[VZ] + ztz * DzVz);

@@ -234,7 +234,9 @@ int cgfd_set_split(cgfd_session *s, int split);
 int cgfd_get_const_metric(cgfd_session *s, int *const_metric);
 
 /* Enable or disable (default) HIP-event timing of every interior kernel
- * launch.  Timed runs are enqueued launch by launch, without graphs. */
+ * launch.  Timed runs are enqueued launch by launch, without graphs, and the
+ * free-surface rows always have a launch of their own in them (untimed, they
+ * may ride with the PML sweep's); results do not depend on it. */
 int cgfd_set_timing(cgfd_session *s, int on);
 
 /* Peak ground motion on a free surface (PG_calcu_gpu,
