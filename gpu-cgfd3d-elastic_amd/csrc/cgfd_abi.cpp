@@ -833,7 +833,7 @@ Shell make_shell(cgfd_session *s, bool rhs = false) {
     return sh;
   }
   sh.inner.zchunk = s->tile_zchunk;
-  sh.inner.shape = rhs ? kRhsShape : s->tile_shape < 0 ? 0 : s->tile_shape;
+  sh.inner.shape = s->tile_shape < 0 ? 0 : s->tile_shape;
   sh.rim.zchunk = rim_zchunk(sh.inner.zchunk);
   sh.rim.shape = sh.inner.shape;
   sh.rim.pml = 1;

@@ -500,7 +500,7 @@ static hipError_t launch_march_t(const StageArgs<TS, TC> &a, const MarchSet &b, 
   }
   CGFD_M(MODE_S0);
   CGFD_M(MODE_S12);
-  if constexpr (CGFD_SHAPE == kRhsShape && !SURF && MET != MET_REF) CGFD_M(MODE_RHS);
+  if constexpr (!SURF && MET != MET_REF) CGFD_M(MODE_RHS);
 #undef CGFD_M
   return hipGetLastError();
 }

@@ -54,8 +54,6 @@ struct MarchGrid {
 // tile shapes the autotuner chooses from (TX x TY threads, one per column)
 constexpr int kNumShapes = 4;
 constexpr int kTile[kNumShapes][2] = {{64, 4}, {32, 8}, {64, 8}, {32, 16}};
-// the bare right-hand side (one operator call, never timed) runs this shape only
-constexpr int kRhsShape = 1;
 // Shapes with a sweep of their own for grids of vertical lines (MET_VERT); the
 // others, which no FP32 or FP64 grid has chosen, stream all nine components.
 // 16-bit storage streams them on every shape: the products that drop would move
