@@ -256,12 +256,13 @@ void dfree(cgfd_session *s, void *&p) {
 
 // Device buffer of at least `need` bytes, reallocated only when it grows, so
 // that rebuilding small tables between runs does not free memory (a free
-// waits for the whole device, including other sessions' work).
-int ensure(cgfd_session *s, void **p, size_t *cap, size_t need) {
+// waits for the whole device, including other sessions' work).  It never needs
+// more than `most`.
+int ensure(cgfd_session *s, void **p, size_t *cap, size_t need, size_t most = SIZE_MAX) {
   if (*p && need <= *cap) return CGFD_OK;
   if (*p) dfree(s, *p);
   *cap = 0;
-  const size_t want = std::max<size_t>(need + need / 2, 256);
+  const size_t want = std::min(std::max<size_t>(need + need / 2, 256), std::max(need, most));
   int r = dalloc(s, p, want);
   if (r) return r;
   *cap = want;
@@ -490,6 +491,11 @@ int copy_window(cgfd_session *s, int a, int b) {
 // shots: 38 MB at 4096 points) outgrow the launches they save.
 constexpr long kMaxSrcBox = 4096;
 
+// elements of the source table that one shot can take
+long src_table_elems(const cgfd_desc &d) {
+  return 4L * kNC * (long)std::min<long long>(kMaxSrcBox, (long long)d.ni * d.nj * d.nk);
+}
+
 // ---- rebuild device source CSR over all shots ----
 template <typename TM> int build_sources(cgfd_session *s) {
   s->s_npt = 0;
@@ -604,7 +610,9 @@ template <typename TM> int build_sources(cgfd_session *s) {
     if ((r = up((void **)&s->s_pt_cell, pt_cell.data(), pt_cell.size() * 4))) return r;
     if ((r = up((void **)&s->s_box, box.data(), box.size() * sizeof(SrcBox)))) return r;
     // cells of a box that no point fills stay zero
-    if ((r = ensure(s, &s->s_v, &s->s_cap[slot++], (size_t)table * sizeof(TM)))) return r;
+    if ((r = ensure(s, &s->s_v, &s->s_cap[slot++], (size_t)table * sizeof(TM),
+                    (size_t)s->d.nshots * src_table_elems(s->d) * sizeof(TM))))
+      return r;
     if ((r = fill_zero(s, s->s_v, (size_t)table, sizeof(TM)))) return r;
     s->s_npt_box = (int)pt_cell.size();
   }
@@ -1376,10 +1384,10 @@ long long cgfd_footprint_bytes(const cgfd_desc *d, int nrecv, int nt_total) {
   long long wav = ns * 4LL * kNC * L.cs * (long long)es;
   long long model = (long long)(NMET + 3) * L.cs * (long long)ms + 18LL * d->ni * d->nj * (long long)ms;
   // peak-motion maps (when enabled), the sub-volume gather buffer (at most
-  // one component) and the source tables (7^3 points with 36 rates each, 9
-  // tables of 4 stage values per step, per shot)
+  // one component) and the source tables (7^3 points, 9 tables of 4 stage values
+  // per step, and the largest table of rates, per shot)
   long long extra = ns * 18LL * d->ni * d->nj * (long long)ms + L.cs * (long long)ms +
-                    ns * (343LL * (28 + 36 * (long long)ms) + 9LL * 4 * (nt_total > 0 ? nt_total : 0) * (long long)ms);
+                    ns * (343LL * 28 + (src_table_elems(*d) + 9LL * 4 * (nt_total > 0 ? nt_total : 0)) * (long long)ms);
   // PML memory: 5 faces of 11 layers at most is bounded by 5 levels over the shell
   long long shell = 2LL * 11 * d->nj * d->nk + 2LL * 11 * d->ni * d->nk + 2LL * 11 * d->ni * d->nj;
   long long aux = ns * 5LL * kNC * shell * (long long)es;
