@@ -58,16 +58,16 @@ ALGO_BYTES = {"f32": 192.0, "f16": 120.0, "bf16": 120.0, "f64": 384.0}
 # This build's own dataflow: wavefield words per swept point and stage, S0 9 in
 # + 9 out, S1 9 in + 9 W^n + 9 out + 9 of the stage values' sum, S2 9 in + 9
 # W^n + 9 out, S3 9 in + 9 sum + 9 out, mean 27; 16-bit storage keeps no sum (S1
-# 27, S3 9 in + 27 W^n, U1, U2 + 9 out), mean 29.25; plus 12 coefficient words
-# (3, the medium, when the metric is constant and passed as kernel arguments).
+# 27, S3 9 in + 27 W^n, U1, U2 + 9 out), mean 29.25; plus the 3 words of the medium
+# and the metric words that the sweep loads (0, 3 or 9, Session.metric_words).
 # The nine PML memory variables of a (point, face) pair follow the same pattern.
 WAVE_WORDS = {"f32": 27.0, "f16": 29.25, "bf16": 29.25, "f64": 27.0}
 ES_WAVE = {"f32": 4, "f16": 2, "bf16": 2, "f64": 8}
 ES_MODEL = {"f32": 4, "f16": 4, "bf16": 4, "f64": 8}
 
 
-def path_bytes(storage, const_metric):
-    return WAVE_WORDS[storage] * ES_WAVE[storage] + (3 if const_metric else 12) * ES_MODEL[storage]
+def path_bytes(storage, metric_words):
+    return WAVE_WORDS[storage] * ES_WAVE[storage] + (3 + metric_words) * ES_MODEL[storage]
 
 
 AUX_BYTES = {k: WAVE_WORDS[k] * v for k, v in ES_WAVE.items()}
@@ -351,6 +351,7 @@ def timed_session(m, storage, warmup, steps, launch_steps, flags=0, tile="", spl
     out["tile"] = sess.get_tile()
     out["split"] = sess.get_split()
     out["const_metric"] = sess.const_metric()
+    out["metric_words"] = sess.metric_words()
     sess.close()
     return out
 
@@ -370,7 +371,7 @@ def roofline(m, storage, r, stream):
     unit = ALGO_BYTES[storage]
     sec = r["int_avg_ms"] * 1e-3
     ach = unit * cells / sec / 1e9
-    path_unit = path_bytes(storage, r["const_metric"])
+    path_unit = path_bytes(storage, r["metric_words"])
     tile = r["tile"]
     roof = dict(bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS, unit="GB/s", frac=round(ach / HBM_PEAK_GBS, 4),
                 traffic=None,
@@ -381,6 +382,7 @@ def roofline(m, storage, r, stream):
                 tile_arg=f"{tile['shape']},{tile['zchunk']}",
                 sweep_share_of_step=round(4 * r["int_avg_ms"] / r["step_ms_timed"], 4) if r["step_ms_timed"] else None,
                 const_metric=r["const_metric"],
+                metric_words=r["metric_words"],
                 path_bytes_per_point_stage=path_unit,
                 path_GBps=round(path_unit * cells / sec / 1e9, 1),
                 pml_face_pairs=pairs,

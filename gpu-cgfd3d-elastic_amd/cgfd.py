@@ -34,7 +34,8 @@ EXPORTS = [
     "cgfd_upload_receivers", "cgfd_set_level", "cgfd_reset_shot", "cgfd_run",
     "cgfd_el_iso_onestage", "cgfd_read_seismo", "cgfd_fetch_level",
     "cgfd_fetch_pml_aux", "cgfd_set_timing", "cgfd_last_run_timing",
-    "cgfd_set_tile", "cgfd_get_tile", "cgfd_get_split", "cgfd_set_split", "cgfd_get_const_metric", "cgfd_set_graph", "cgfd_set_shot",
+    "cgfd_set_tile", "cgfd_get_tile", "cgfd_get_split", "cgfd_set_split", "cgfd_get_const_metric",
+    "cgfd_get_metric_words", "cgfd_set_graph", "cgfd_set_shot",
     "cgfd_run_async", "cgfd_poll", "cgfd_wait", "cgfd_reserve_receivers", "cgfd_set_seismo_ring",
     "cgfd_grid_cartesian", "cgfd_grid_topography", "cgfd_metric_calc", "cgfd_dt_estimate",
     "cgfd_media_layered", "cgfd_media_homogeneous", "cgfd_rho_to_slow", "cgfd_pml_len_dh",
@@ -173,6 +174,7 @@ def load(path=LIB_PATH):
         "cgfd_get_split": ([vp, C.POINTER(i)], i),
         "cgfd_set_split": ([vp, i], i),
         "cgfd_get_const_metric": ([vp, C.POINTER(i)], i),
+        "cgfd_get_metric_words": ([vp, C.POINTER(i)], i),
         "cgfd_last_run_timing": ([vp, C.POINTER(C.c_double), C.POINTER(C.c_double), C.POINTER(C.c_int)], i),
     }
     d = C.c_double
@@ -376,6 +378,12 @@ class Session:
         v = C.c_int()
         _check(_lib.cgfd_get_const_metric(self.h, C.byref(v)))
         return bool(v.value)
+
+    def metric_words(self):
+        """Metric values per point that the sweeps load under the present tile (0, 3 or 9)."""
+        v = C.c_int()
+        _check(_lib.cgfd_get_metric_words(self.h, C.byref(v)))
+        return v.value
 
     def get_tile(self):
         a, b, c, d = C.c_int(), C.c_int(), C.c_int(), C.c_int()

@@ -1972,6 +1972,14 @@ int cgfd_get_const_metric(cgfd_session *s, int *const_metric) {
   return CGFD_OK;
 }
 
+int cgfd_get_metric_words(cgfd_session *s, int *words) {
+  if (!s || !words) return fail(CGFD_E_ARG, "null argument");
+  const int shape = s->tile_shape < 0 ? 0 : s->tile_shape;
+  const bool vert = s->met_class == MET_VERT && s->es >= 4 && kVertShape<float>(shape);
+  *words = s->met_class == MET_CONST ? 0 : vert ? 3 : 9;
+  return CGFD_OK;
+}
+
 int cgfd_get_split(cgfd_session *s, int *split) {
   if (!s) return fail(CGFD_E_ARG, "null session");
   if (split)

@@ -233,6 +233,11 @@ int cgfd_set_split(cgfd_session *s, int split);
  * diagonal values are kernel arguments instead of nine streams). */
 int cgfd_get_const_metric(cgfd_session *s, int *const_metric);
 
+/* Metric values per point that the sweeps load under the session's present
+ * tile: 0 (Cartesian grid), 3 (evenly spaced vertical lines, FP32 and FP64 on
+ * 64x4 and 32x8 tiles) or 9. */
+int cgfd_get_metric_words(cgfd_session *s, int *words);
+
 /* Enable or disable (default) HIP-event timing of every interior kernel
  * launch.  Timed runs are enqueued launch by launch, without graphs, and the
  * free-surface rows always have a launch of their own in them (untimed, they
