@@ -23,6 +23,7 @@ models; and the CPU baseline (the oracle, a C++/OpenMP restatement of the
 reference loop) on a bounded sample of the headline model.
 """
 import argparse
+import hashlib
 import json
 import os
 import platform
@@ -127,9 +128,20 @@ def cpu_baseline(m, steps):
                      f"OMP_PROC_BIND={os.environ.get('OMP_PROC_BIND')} OMP_PLACES={os.environ.get('OMP_PLACES')}")
 
 
+PROFILES = os.path.join(ROOT, "profiles")
+SWEEP_SOURCES = ("el_iso_interior.hip", "el_iso_point.h", "el_iso_pml.h", "el_iso_device.h", "el_iso_launch.h")
+
+
+def sweep_id():
+    """Fingerprint of the sweep's sources, comments and layout apart: counters
+    belong to the kernels they were taken of."""
+    text = "".join(open(os.path.join(PKG, "csrc", f)).read() for f in SWEEP_SOURCES)
+    return hashlib.sha256(" ".join(re.sub(r"//[^\n]*", "", text).split()).encode()).hexdigest()[:12]
+
+
 def measured_traffic(workload, storage, split, tile):
     """(HBM bytes per sweep launch, profiled tile) from the committed counter
-    summary, or (None, None).
+    summary of these kernels ("sweep_id = ..."), or (None, None).
 
     The summary holds FETCH_SIZE + WRITE_SIZE per dispatch of the z-marching
     kernel on this workload and work split, scaled by the same counters on
@@ -139,11 +151,14 @@ def measured_traffic(workload, storage, split, tile):
     nearest z chunk (the chunk changes only the priming planes), and the
     profiled tile is reported beside the figure."""
     name = SPLIT_NAMES[split]
-    path = os.path.join(ROOT, "profiles", f"k_march_{workload}_{storage}_{name}_hbm_counters.txt")
+    path = os.path.join(PROFILES, f"k_march_{workload}_{storage}_{name}_hbm_counters.txt")
     if not os.path.exists(path):
         return None, None
+    lines = open(path).read().splitlines()
+    if f"sweep_id = {sweep_id()}" not in lines:
+        return None, None
     best = None
-    for line in open(path):
+    for line in lines:
         mt = re.match(r"traffic_bytes_per_launch\[(\d+)x(\d+)/(\d+)\]\s*=\s*([0-9.eE+]+)", line)
         if not mt:
             continue
