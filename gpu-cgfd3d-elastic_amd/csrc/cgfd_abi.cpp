@@ -933,7 +933,11 @@ int launch_stage(cgfd_session *s, const Shell &sh, StageArgs<TS, TC> &a, int dx,
 // of pair 0) and keep the fastest; the stages differ in traffic (30 to 57 words
 // per cell), so tuning on one mode alone can pick a tile that loses on the
 // others.  Every level the sweeps write (slots 1..3) is rewritten by the next
-// step before it is read, so tuning between steps leaves the state intact.
+// step before it is read, so tuning between steps leaves the state intact.  A
+// session's first run pays for it: losing choices are timed once and kernels
+// warmed once per shape (with three passes of every choice, the small z chunks,
+// the fused rows and the second search of 16-bit storage had taken the first runs
+// of 17 sessions of 64^3 to 400x400x200 from 8.6 to 14.0 s; now 7.9 s).
 // Results are cached per (grid, storage, shots, flags, metric form, PML layout,
 // pinned split) for the life of the process.
 struct TileKey {
@@ -1009,15 +1013,18 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
-  // minimum over reps 1..2 of one full step's four stages under the session's
-  // present choice: the sweeps, the other launches, or both
+  // minimum over two passes of one full step's four stages under the session's
+  // present choice: the sweeps, the other launches, or both.  A first pass beyond
+  // `limit` ms is the last; kernels not launched before (cold) run once untimed.
+  // apart: another pass goes before the two and counts only where it is 30 %
+  // beyond the limit, and then alone.
   enum { SWEEPS = 1, OTHERS = 2 };
-  auto timed = [&](float &tmin, int parts) -> int {
+  auto timed = [&](float &tmin, int parts, float limit, bool cold, bool apart) -> int {
     Shell sh = make_shell(s);
     if (!(parts & SWEEPS)) sh.inner.nbox = sh.rim.nbox = 0;
     if (!(parts & OTHERS)) { sh.point.n = 0; sh.surface = false; }
     tmin = 1e30f;
-    for (int rep = 0; rep < 3; rep++) {
+    for (int rep = cold || apart ? -1 : 0; rep < 2; rep++) {
       HIPCHK(hipEventRecord(e0, s->st));
       for (int q = 0; q < 4; q++) {
         const int d = (kFlags[0][0] + q) % 2;
@@ -1025,10 +1032,13 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
         if (r) return r;
       }
       HIPCHK(hipEventRecord(e1, s->st));
+      if (rep < 0 && cold) continue;
       HIPCHK(hipEventSynchronize(e1));
       float ms = 0;
       HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-      if (rep > 0) tmin = std::min(tmin, ms);
+      const bool over = ms > (rep < 0 ? 1.3f * limit : limit);
+      if (rep >= 0 || over) tmin = std::min(tmin, ms);
+      if (over) break;
     }
     return CGFD_OK;
   };
@@ -1054,7 +1064,7 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
       float others = 0;
       if (apart) {
         s->tile_shape = 0;
-        int r = timed(others, OTHERS);
+        int r = timed(others, OTHERS, 1e30f, true, true);
         if (r) return r;
       }
       for (int shape = 0; shape < kNumShapes; shape++) {
@@ -1073,6 +1083,7 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
         constexpr int kNZ = 14;
         const int ztarget[kNZ] = {2, 3, 4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96};
         int last = 0;
+        bool cold[2] = {true, true};  // the kernels do not depend on the z chunk
         for (int target : ztarget) {
           if (target < zmin || (target < 16 && march_workgroups(sh.inner, 16) * s->d.nshots >= 2048)) continue;
           const int n = std::max(1, (nz + target / 2) / target), zc = (nz + n - 1) / n;
@@ -1081,10 +1092,14 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
           s->tile_zchunk = zc;
           for (int fuse = 0; fuse <= (sh.inner.surface || sh.rim.surface ? 1 : 0); fuse++) {
             s->fuse = fuse != 0;
+            // a choice 20 % behind the best is timed once; where the timing decides
+            // over 16-bit roundings a first pass is left out of it throughout
+            const float cost = split == CGFD_SPLIT_SHELL ? 1.0f : pml_cost;
             float t;
-            int r = timed(t, apart ? SWEEPS : SWEEPS | OTHERS);
+            int r = timed(t, apart ? SWEEPS : SWEEPS | OTHERS, (1.2f * best - others) / cost, cold[fuse], apart);
             if (r) return r;
-            t = (split == CGFD_SPLIT_SHELL ? t : t * pml_cost) + others;
+            cold[fuse] = false;
+            t = t * cost + others;
             if (t < best) { best = t; bs = shape; bz = zc; bsplit = split; bfuse = s->fuse; }
           }
         }
@@ -1097,9 +1112,18 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   // part of a session's results.  It is made on the forms that first made it
   // and in the way it was first made (chunks of 16 planes and more, the zero
   // terms of a constant metric taken, sweeps and slabs timed apart: on whole
-  // stages 256x256x128 float16, 1.97 against 2.00 ms a step, fell to the other side):
-  // a grid keeps its roundings when a sweep gets faster.  The sweeps of the
-  // chosen side, equal bit for bit, then compete in their present forms.
+  // stages 256x256x128 float16, 1.97 against 2.00 ms a step, fell to the other side),
+  // so that most grids keep the side, and with it the roundings, that they have
+  // had when a sweep gets faster: 416 of 432 sessions of 6e4 to 3e7 points did.
+  // It is a race of timings all the same: near its edge another box, compiler or
+  // number of shots falls to the other side (3 of 246 from one run to the next, 34
+  // of 196 grids between one shot and a batch), and a program that compares
+  // 16-bit runs bit for bit pins the split.  No rule on the grid takes its place:
+  // on storage, metric class, size, layers and lanes filled the best found
+  // keeps 84 % of those sides (89 % with the number of shots), and the
+  // outputs of the other sessions would move by 16-bit roundings.  The
+  // sweeps of the chosen side, equal bit for bit, then compete in their present
+  // forms.
   if constexpr (St<TS>::scaled) {
     if (splits.size() > 1) {
       if (s->met_class == MET_CONST) {

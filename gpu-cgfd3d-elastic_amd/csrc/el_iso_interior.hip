@@ -32,7 +32,9 @@
 // update.  y and z faces are uniform across a wavefront (a wave spans one
 // or two rows of one plane); only the tiles at the two x ends diverge.  The
 // interior variant (PML = false) sweeps a box outside every face box.
-// Points within 4 rows of a free surface go to the per-point kernel.
+// Points within 4 rows of a free surface go to surface tiles (el_iso_point.h),
+// which may ride with a PML-form launch (SURF), and with 16-bit storage to the
+// per-point kernel.
 #include "el_iso_point.h"
 
 #include <type_traits>
