@@ -80,9 +80,12 @@ typedef struct {
  * box inside them (by default the z-marching kernel sweeps whole planes,
  * PML included, and the 4 free-surface rows are updated apart) */
 #define CGFD_FLAG_PML_POINT 2
-/* keep the per-point metric arrays even when the grid is Cartesian (by
- * default a metric whose components are constant to 1e-10 of their largest
- * magnitude runs the constant-metric sweep with the first point's values) */
+/* keep the per-point metric arrays on every grid.  By default a metric whose
+ * components are constant to 1e-10 of their largest magnitude (Cartesian grid)
+ * runs the constant-metric sweep with the first point's values, and one whose xi
+ * and eta rows are constant or zero (vertical lines) drops those rows in FP32 and
+ * FP64 sessions; the latter, and the free-surface rows of either, to 1e-10 of
+ * the row's diagonal term in FP32 and to four roundings of it in FP64 */
 #define CGFD_FLAG_FULL_METRIC 4
 
 /* Point-source tables of one shot: the device mirror of src_t
@@ -170,7 +173,8 @@ int cgfd_run(cgfd_session *s, int it0, int nsteps, double dt);
 
 /* One RK-stage right-hand side into the RHS level (and the PML memory RHS):
  * the operator sv_curv_col_el_iso_onestage
- * (src/forward/sv_curv_col_el_iso_gpu.cu:23-285) reading level in_level. */
+ * (src/forward/sv_curv_col_el_iso_gpu.cu:23-285) reading level in_level, under
+ * the session's tile and split. */
 int cgfd_el_iso_onestage(cgfd_session *s, int shot, int in_level, int ipair, int istage, int it);
 
 /* ---- results ---------------------------------------------------------------- */
@@ -225,7 +229,10 @@ int cgfd_get_split(cgfd_session *s, int *split);
 /* Pin the work split (split < 0: the autotuner chooses again).  With an
  * automatic tile the autotuner then tunes the tile under that split only.
  * A tuning control with no counterpart in the reference, like cgfd_set_tile;
- * every split gives the same results to rounding. */
+ * every split gives the same results to rounding.  With 16-bit storage that is
+ * the rounding of the stored levels, and the automatic choice, a race of timings,
+ * may fall to another side for another batch size or on another box: pin the
+ * split where 16-bit runs are compared bit for bit. */
 int cgfd_set_split(cgfd_session *s, int split);
 
 /* 1 when the uploaded metric runs the constant-metric sweep (a Cartesian
