@@ -17,8 +17,8 @@ z-marching sweep, average launch time from HIP events on its stream, 192
 algorithmic bytes per swept point and stage) beside the streaming read/copy
 ceilings measured in the same run; FP16 / BF16 storage and the FP64 path on
 the same model with their relative L2 errors against FP64; the 400x400x200
-topography model (curvilinear metrics, all 12 coefficient streams); 64
-batched shots on the small medium; a served stream over five resident
+topography model (vertical grid lines: 6 coefficient words a point in FP32,
+12 with 16-bit storage); 64 batched shots on the small medium; a served stream over five resident
 models; and the CPU baseline (the oracle, a C++/OpenMP restatement of the
 reference loop) on a bounded sample of the headline model.
 """
@@ -48,7 +48,7 @@ SWEEP_KERNEL = {
     cgfd.SPLIT_PLANES: "k_march (z-marching sweep, whole planes with the PML slabs)",
     cgfd.SPLIT_SHELL: "k_march (z-marching sweep, inside the PML slabs)",
     cgfd.SPLIT_CORE: "k_march (z-marching sweep, whole planes: PML-free core launch + PML-form rim launch, "
-                     "timed together per stage)",
+                     "timed together per stage, free-surface rows apart)",
 }
 KERNEL_PATH = {cgfd.SPLIT_PLANES: "zmarch planes", cgfd.SPLIT_SHELL: "zmarch + point shell",
                cgfd.SPLIT_CORE: "zmarch core + rim"}
@@ -481,8 +481,7 @@ def precision_leg(m, steps):
 
 
 def topo_leg(steps, warmup, stream):
-    """The 400x400x200 topography model (curvilinear metric, all coefficient
-    streams): FP32 with its sweep roofline, FP16 and BF16 storage."""
+    """The 400x400x200 topography model (vertical grid lines over topography): FP32 with its sweep roofline, FP16 and BF16 storage."""
     m = workloads.topo(nt=warmup + steps + 8)
     cells = workloads.cells(m)
     out = {}

@@ -781,7 +781,7 @@ StageArgs<TS, TC> stage_args(cgfd_session *s, int slot_in, int slot_pre, int slo
 // box whose x extent starts and ends on tile boundaries (so its rows load
 // whole 128-byte lines), and the PML form over the up to six rim boxes around
 // it; the PML-free form needs fewer registers (FP32 32x8 tile, constant
-// metric: 102-124 VGPRs, 4 waves per SIMD, against 137-159, 3 waves), so more
+// metric: 104-128 VGPRs, 4 waves per SIMD, against 135-163, 3 waves), so more
 // waves hide its latency.  CGFD_SPLIT_SHELL (or CGFD_FLAG_PML_POINT): the sweep
 // keeps to the box inside every face box and the per-point launch takes the
 // whole shell (face slabs and surface rows: a launch of their own gained

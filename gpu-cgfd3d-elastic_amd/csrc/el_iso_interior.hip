@@ -443,13 +443,13 @@ template <typename TS, typename TC, int TX, int TY, int MINB, int MET, bool PML,
 static void launch_march_m(const StageArgs<TS, TC> &a, const MarchSet &b, const MarchGrid &g, dim3 grid, dim3 block,
                            int sel, hipStream_t st) {
   // Waves per SIMD the compiler has to leave room for.  In FP32 the PML form of
-  // a constant or vertical-line metric fits three (168 VGPRs) without spilling;
+  // a constant or vertical-line metric fits three (168 VGPRs, at most 20 bytes of spill);
   // so does the 16-bit S1/S2 of a constant metric (15 % faster on 800x800x400).
   // The other forms spill 64-336 bytes there and ran slower (200x180x100
   // curvilinear FP32, all at three: 24.2 -> 26.0 ms).  FP64's PML form of the
   // general metric spills 250-340 bytes to scratch at two waves; with one they
   // go to the accumulation registers (67x53x45: 3.73 -> 3.54 ms).  Its other
-  // forms spill 0-140 bytes at two, which is still faster than one
+  // forms spill 0-156 bytes at two, which is still faster than one
   // (128x128x96: 20.1 -> 19.4 ms).
   constexpr bool thin = PML && TX * TY == 256 && MET != MET_ALL;
   constexpr int MB = sizeof(TS) == 8 && PML && MET == MET_ALL                ? 1
