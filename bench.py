@@ -18,9 +18,10 @@ algorithmic bytes per swept point and stage) beside the streaming read/copy
 ceilings measured in the same run; FP16 / BF16 storage and the FP64 path on
 the same model with their relative L2 errors against FP64; the 400x400x200
 topography model (vertical grid lines: 6 coefficient words a point in FP32,
-12 with 16-bit storage); 64 batched shots on the small medium; a served stream over five resident
-models; and the CPU baseline (the oracle, a C++/OpenMP restatement of the
-reference loop) on a bounded sample of the headline model.
+12 with 16-bit storage); 64 batched shots on the small medium; a served
+stream over five resident models; and the CPU baseline (the oracle, a
+C++/OpenMP restatement of the reference loop) on a bounded sample of the
+headline model.
 """
 import argparse
 import hashlib
@@ -481,7 +482,8 @@ def precision_leg(m, steps):
 
 
 def topo_leg(steps, warmup, stream):
-    """The 400x400x200 topography model (vertical grid lines over topography): FP32 with its sweep roofline, FP16 and BF16 storage."""
+    """The 400x400x200 topography model (vertical grid lines over topography):
+    FP32 with its sweep roofline, FP16 and BF16 storage."""
     m = workloads.topo(nt=warmup + steps + 8)
     cells = workloads.cells(m)
     out = {}

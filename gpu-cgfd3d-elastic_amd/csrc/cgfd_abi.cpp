@@ -1115,7 +1115,7 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
   // stages 256x256x128 float16, 1.97 against 2.00 ms a step, fell to the other side),
   // so that most grids keep the side, and with it the roundings, that they have
   // had when a sweep gets faster: 416 of 432 sessions of 6e4 to 3e7 points did.
-  // It is a race of timings all the same: near its edge another box, compiler or
+  // It is a race of timings all the same: near its edge another machine, compiler or
   // number of shots falls to the other side (3 of 246 from one run to the next, 34
   // of 196 grids between one shot and a batch), and a program that compares
   // 16-bit runs bit for bit pins the split.  No rule on the grid takes its place:
@@ -1159,7 +1159,8 @@ template <typename TS, typename TC> int autotune_t(cgfd_session *s) {
 // the caller.  table: with the rates tabulated over the boxes.
 template <typename TS, typename TC> SrcArgs<TS, TC> source_args(cgfd_session *s, bool table) {
   SrcArgs<TS, TC> sa{};
-  sa.L = s->L; sa.npt = s->s_npt; sa.npt_box = s->s_npt_box; sa.pt_shot = s->s_pt_shot; sa.pt_off = s->s_pt_off; sa.pt_beg = s->s_pt_beg;
+  sa.L = s->L; sa.npt = s->s_npt; sa.npt_box = s->s_npt_box;
+  sa.pt_shot = s->s_pt_shot; sa.pt_off = s->s_pt_off; sa.pt_beg = s->s_pt_beg;
   sa.ct_src = s->s_ct_src; sa.ct_coef = (const TC *)s->s_ct_coef; sa.s_itb = s->s_itb; sa.s_ite = s->s_ite;
   sa.s_tab = s->s_tab; sa.s_kind = s->s_kind; sa.F = (const TC *)s->s_F; sa.M = (const TC *)s->s_M;
   sa.ntab = s->s_ntab; sa.met = (const TC *)s->met; sa.med = (const TC *)s->med;

@@ -231,7 +231,7 @@ int cgfd_get_split(cgfd_session *s, int *split);
  * A tuning control with no counterpart in the reference, like cgfd_set_tile;
  * every split gives the same results to rounding.  With 16-bit storage that is
  * the rounding of the stored levels, and the automatic choice, a race of timings,
- * may fall to another side for another batch size or on another box: pin the
+ * may fall to another side for another batch size or on another machine: pin the
  * split where 16-bit runs are compared bit for bit. */
 int cgfd_set_split(cgfd_session *s, int split);
 
